@@ -158,8 +158,8 @@ static void free_ctx(fm_ctx* c) {
     void* ptrs[] = {c->st[0], c->st[1], c->rdisp, c->ext[0], c->ext[1], c->slot_of, c->moltype[0], c->moltype[1],
                     c->tag[0], c->tag[1], c->teth[0], c->teth[1], c->mono[0], c->mono[1], c->cell_of,
                     c->cell_count, c->cell_start, c->bin_pos, c->scan_part, c->perm, c->nbl, c->nbn, c->bond, c->bondn,
-                    c->pe_lj, c->pe_poly, c->vir, c->rf, c->pxy, c->cvface, c->planes, c->out_flag, c->out_vals,
-                    c->out_slot, c->out_count, c->red, c->d_macros, c->d_ring, c->d_mie, c->d_vmax, c->d_rmax,
+                    c->pe_lj, c->pe_poly, c->vir, c->rf, c->pxy, c->cvface, c->planes, c->out_flag, c->out_mask,
+                    c->out_bits, c->red, c->d_macros, c->d_ring, c->d_mie, c->d_vmax, c->d_rmax,
                     c->d_flags, c->stage, c->brick_order, c->btab, c->hcurve, c->sort_key,
                     c->sort_val, c->sort_key2, c->sort_val2, c->sort_cnt, c->sort_tmp};
     for (void* p : ptrs)
@@ -395,7 +395,7 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
         (rc = dalloc(&c->scan_part, (size_t)c->ncell / 1024 + 2)) ||
         (rc = dalloc(&c->perm, cap)) || (rc = dalloc(&c->nbn, cap)) || (rc = dalloc(&c->pe_lj, cap)) ||
         (rc = dalloc(&c->pe_poly, cap)) || (rc = dalloc(&c->vir, cap)) || (rc = dalloc(&c->out_flag, cap)) ||
-        (rc = dalloc(&c->out_vals, cap)) || (rc = dalloc(&c->out_slot, cap)) || (rc = dalloc(&c->out_count, (cap + FM_BLOCK - 1) / FM_BLOCK + 4)) ||
+        (rc = dalloc(&c->out_mask, cap)) || (rc = dalloc(&c->out_bits, 4 * ((cap + 127) / 128))) ||
         (rc = dalloc(&c->red, (size_t)c->nred_blocks * 8)) || (rc = dalloc(&c->d_macros, 16)) ||
         (rc = dalloc(&c->d_ring, 8 * (size_t)FM_RING_SLOTS)) ||
         (rc = dalloc(&c->d_mie, 7 * (size_t)T2 + FM_MAX_TYPES)) || (rc = dalloc(&c->d_vmax, 1)) ||
@@ -514,6 +514,7 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
     }
     c->timer = new KTimer();
     if ((rc = launch_fill_i32(c, c->d_flags, 0, FLAG_COUNT)) ||
+        (rc = launch_fill_i32(c, (int*)c->out_bits, 0, 4 * ((cap + 127) / 128))) ||
         (rc = launch_fill_i32(c, c->cell_count, 0, (size_t)c->ncell + 1)) || (rc = launch_fill_f64(c, c->d_rmax, 0.0, 1)) ||
         (rc = launch_fill_f64(c, c->st[0], 0.0, 9 * cap)) || (rc = launch_fill_f64(c, c->pe_lj, 0.0, cap)) ||
         (rc = launch_fill_f64(c, c->pe_poly, 0.0, cap)) || (rc = launch_fill_f64(c, c->vir, 0.0, cap))) {
@@ -553,7 +554,7 @@ extern "C" int fm_memory_footprint(const fm_params* p, int32_t np, int64_t* byte
     maxnb = (maxnb + 3) & ~3;
     size_t b = 0;
     b += 2 * 9 * cap * 8 + 3 * cap * 8 + 9 * cap * 8;          // state copies, rdisp, staging
-    b += (2 + 1 + 1 + 1 + 1 + 1 + 3) * cap * 4;                 // ext, slot_of, cell_of, bin_pos, perm, nbn, sendmols scratch
+    b += (2 + 1 + 1 + 1 + 1 + 1 + 2) * cap * 4 + cap / 8;       // ext, slot_of, cell_of, bin_pos, perm, nbn, sendmols scratch
     b += 3 * cap * 8;                                           // pe_lj, pe_poly, vir
     b += (size_t)(maxnb / 4) * cap * 8;                         // neighbour words
     b += 3 * (ncell + 1) * 4;                                   // cell counts, starts, cursors
@@ -1238,11 +1239,16 @@ static int rebuild_lists_queued(fm_ctx* c, bool resets = true, bool keep_acc = f
         return rebuild_lists(c);
     }
     c->cells_valid = c->nlist_valid = false;
-    TRY(launch_sendmols(c, reset, resets ? 5 : 0));
-    TRY(fm_sort_mols(c));
     // every launch queued after this rebuild (the force launch, or nothing until the lists are
     // rebuilt) recomputes all accelerations before reading them
-    TRY(launch_bin(c, keep_acc));
+    if (c->p.sort_flag == 0) {
+        TRY(fm_sort_mols(c));  // (its call counter)
+        TRY(launch_bin(c, keep_acc, true, reset, resets ? 5 : 0));
+    } else {
+        TRY(launch_sendmols(c, reset, resets ? 5 : 0));
+        TRY(fm_sort_mols(c));
+        TRY(launch_bin(c, keep_acc));
+    }
     c->moved_since_bin = false;
     c->cells_valid = true;
     TRY(launch_nlist(c));

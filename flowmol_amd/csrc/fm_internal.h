@@ -80,7 +80,7 @@ struct fm_ctx {
     int* cell_count = nullptr;            // ncell
     int* cell_start = nullptr;            // ncell+1
     int* bin_pos = nullptr;               // cap: each molecule's place among its cell's (binning)
-    int* scan_part = nullptr;             // cell scan: count sums of the 1024-cell chunks
+    int* scan_part = nullptr;             // cell scan: count sums of its chunks
     int* perm = nullptr;                  // cap
 
     // LDS bricks
@@ -134,10 +134,9 @@ struct fm_ctx {
     double mop_shift = 0.0;
 
     // sendmols scratch
-    int* out_flag = nullptr;              // cap
-    int* out_vals = nullptr;              // cap
-    int* out_slot = nullptr;              // cap
-    int* out_count = nullptr;             // per-workgroup leaver counts
+    int* out_flag = nullptr;              // cap: cell index in old slot order (binning)
+    int* out_mask = nullptr;              // cap: per slot, the passes a leaver left in
+    unsigned* out_bits = nullptr;         // one bit per molecule number, in whole 16-byte words
 
     // reductions
     double* red = nullptr;                // partial sums
@@ -200,7 +199,8 @@ int launch_check_vmax(fm_ctx* c);
 int launch_sendmols(fm_ctx* c, const int* reset = nullptr, int nreset = 0);  // also zeroes the listed flags
 // binning (counting sort into cells, x order per cell, permutation of the state); keep_acc false
 // leaves the accelerations out of the permutation (the next force launch overwrites them all)
-int launch_bin(fm_ctx* c, bool keep_acc = true);
+// send: with sendmols before it (not with sort_mols, which comes between them), zeroing `reset`
+int launch_bin(fm_ctx* c, bool keep_acc = true, bool send = false, const int* reset = nullptr, int nreset = 0);
 int launch_reset_flags(fm_ctx* c, const int* which, int n);  // zero the listed flag words
 int launch_nlist(fm_ctx* c);
 // cond: do nothing when a rebuild is pending (FLAG_REBUILD or FLAG_HALT), and raise FLAG_HALT.

@@ -257,7 +257,6 @@ __global__ void k_vmax_finish(unsigned long long* vmax_bits, double* rmax, doubl
 }
 
 // ---- sendmols on one periodic rank, src/messenger.MPI.f90:1383-1904 ---------------------------
-// 1) mark molecules (in molecule-number order) that lie outside the box on any axis
 // zero the listed flag words
 struct FlagList {
     int n;
@@ -272,282 +271,370 @@ __device__ inline void reset_flag(int* flags, int w) {
     if (w == FLAG_HALT) flags[FLAG_HALT_STEP] = 0x7fffffff;
 }
 
-// 1) molecules outside the box, in molecule-number order: workgroup b writes its leavers e
-//    (ascending) to seg[b*FM_BLOCK ..] and their count to bcnt[b].  Workgroup 0 also zeroes the
-//    flag words of `reset` (the resets of a queued rebuild, folded into its first launch).
-__global__ __launch_bounds__(FM_BLOCK) void k_out_select(St s, const int* slot_of, int np, double hx, double hy,
-                                                         double hz, int* seg, int* bcnt, int* flags, FlagList reset) {
-    __shared__ int wc[FM_BLOCK / 64];
-    if (blockIdx.x == 0 && (int)threadIdx.x < reset.n) reset_flag(flags, reset.w[threadIdx.x]);
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    int out = 0;
-    if (e < np) {
-        const int sl = slot_of[e];
-        const double x = s.x[sl], y = s.y[sl], z = s.z[sl];
-        out = (x < -hx) | (x >= hx) | (y < -hy) | (y >= hy) | (z < -hz) | (z >= hz);
-    }
-    const unsigned long long m = __ballot(out);
-    const int rank = __popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) wc[wid] = __popcll(m);
-    __syncthreads();
-    int off = 0, tot = 0;
-    for (int w = 0; w < FM_BLOCK / 64; ++w) {
-        if (w < wid) off += wc[w];
-        tot += wc[w];
-    }
-    if (out) seg[(size_t)blockIdx.x * FM_BLOCK + off + rank] = e;
-    if (threadIdx.x == 0) bcnt[blockIdx.x] = tot;
-}
+// The 3 x (3 axes x 2 directions) exchange passes of sendmols (checksendbuild, sendrecvface,
+// reorderdata): in each pass the molecules beyond that face, in ascending molecule number, are
+// wrapped by -dir*domain and their numbers reversed among them.  Where a molecule leaves depends on
+// its own position alone, so every molecule runs its 18 passes by itself (wrap_molecule) and keeps
+// them as bits; the numbers are then exchanged among the leavers by one workgroup (renumber).
+struct WrapArgs {
+    St s;
+    const int* ext;
+    const int* tag;        // null without tag_move
+    double* teth;
+    int np, cap;
+    double L[3], ws[3];    // domain, wallslidev
+    int* mask;             // per slot: the passes a leaver left in (written for leavers only)
+    unsigned* bits;        // one bit per molecule number: leavers
+    int* flags;
+    FlagList reset;        // flag words zeroed by workgroup 0 (the resets of a queued rebuild)
+};
 
-// 2) one workgroup replays the 3 x (3 axes x 2 directions) passes on the compacted set.
-//    vals[q] ascending molecule numbers of the set (fixed); sl[q] slot currently holding vals[q].
-//    Each pass: leavers in q order (= ascending molecule number) are wrapped by -dir*domain and
-//    their molecule numbers reversed, as checksendbuild + sendrecvface + reorderdata do.
-//    The set is first gathered from the segments of k_out_select in workgroup order.
-__global__ __launch_bounds__(1024) void k_sendmols_passes(St s, double* teth, const int* tag, int* ext,
-                                                          int* slot_of, const int* seg, const int* bcnt, int nblk,
-                                                          int* vals, int* sl, int* lst, int* tmp,
-                                                          int cap, double Lx, double Ly, double Lz,
-                                                          int tag_move, double wsx, double wsy,
-                                                          double wsz) {
-    __shared__ int wsum[16];
-    __shared__ int chunk_base;
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    {  // thread t gathers the segments of a contiguous range of workgroups
-        const int per = (nblk + (int)blockDim.x - 1) / (int)blockDim.x;
-        const int b0 = min(nblk, tid * per), b1 = min(nblk, b0 + per);
-        int mine = 0;
-        for (int b = b0; b < b1; ++b) mine += bcnt[b];
-        int x = mine;
-        for (int d = 1; d < 64; d <<= 1) {
-            const int y = __shfl_up(x, d, 64);
-            if (lane >= d) x += y;
-        }
-        if (lane == 63) wsum[wid] = x;
-        __syncthreads();
-        int pos = x - mine, tot = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-            if (w < wid) pos += wsum[w];
-            tot += wsum[w];
-        }
-        for (int b = b0; b < b1; ++b) {
-            const int cb = bcnt[b];
-            for (int k = 0; k < cb; ++k) vals[pos++] = seg[(size_t)b * FM_BLOCK + k];
-        }
-        if (tid == 0) chunk_base = tot;
-        __syncthreads();
-    }
-    const int n = chunk_base;
-    __syncthreads();
-    const double L[3] = {Lx, Ly, Lz};
-    double* pos[3] = {s.x, s.y, s.z};
-    if (n <= (int)blockDim.x) {
-        // One leaver per thread, held in LDS by list position: its slot and position.  The same
-        // passes as below, without a global read in them; a pass without leavers ends at its
-        // count.  The renumbering moves slots and positions between list positions together.
-        __shared__ int cs[1024], cl[1024], ct[1024];
-        __shared__ double cp[3][1024], cq[3][1024];
-        if (tid < n) {
-            const int slot = slot_of[vals[tid]];
-            cs[tid] = slot;
-            cp[0][tid] = pos[0][slot];
-            cp[1][tid] = pos[1][slot];
-            cp[2][tid] = pos[2][slot];
-        }
-        __syncthreads();
-        for (int it = 0; it < 3; ++it)
-            for (int ax = 0; ax < 3; ++ax)
-                for (int dir = -1; dir <= 1; dir += 2) {
-                    const double h = 0.5 * L[ax];
-                    const bool lv = tid < n && (dir == -1 ? (cp[ax][tid] < -h) : (cp[ax][tid] >= h));
-                    const unsigned long long m = __ballot(lv);
-                    if (lane == 0) wsum[wid] = __popcll(m);
-                    __syncthreads();
-                    int off = 0, k = 0;
-                    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-                        if (w < wid) off += wsum[w];
-                        k += wsum[w];
-                    }
-                    __syncthreads();  // (wsum is written again by the next pass)
-                    if (k == 0) continue;
-                    if (lv) cl[off + __popcll(m & ((1ull << lane) - 1ull))] = tid;
-                    __syncthreads();
-                    // wrap the leavers: r(ixyz) - dir*domain(ixyz)
-                    if (tid < k) {
-                        const int q = cl[tid], slot = cs[q];
-                        cp[ax][q] = cp[ax][q] - (double)dir * L[ax];
-                        pos[ax][slot] = cp[ax][q];
-                        if (tag_move && (tag[slot] == FM_TAG_TETH || tag[slot] == FM_TAG_TETH_SLIDE))
-                            teth[slot + (size_t)ax * cap] = teth[slot + (size_t)ax * cap] - (double)dir * L[ax];
-                    }
-                    __syncthreads();
-                    if (tid < k) {
-                        const int q = cl[k - 1 - tid];
-                        ct[tid] = cs[q];
-                        cq[0][tid] = cp[0][q];
-                        cq[1][tid] = cp[1][q];
-                        cq[2][tid] = cp[2][q];
-                    }
-                    __syncthreads();
-                    if (tid < k) {
-                        const int q = cl[tid], slot = ct[tid];
-                        cs[q] = slot;
-                        cp[0][q] = cq[0][tid];
-                        cp[1][q] = cq[1][tid];
-                        cp[2][q] = cq[2][tid];
-                        if (tag_move) {  // read_tag on the renumbered molecule
-                            const int tg = tag[slot];
-                            const double sg = tg == FM_TAG_TETH_SLIDE   ? copysign(1.0, cq[1][tid])
-                                              : tg == FM_TAG_FIXED_SLIDE ? 1.0
-                                                                         : 0.0;
-                            teth[slot + 3 * (size_t)cap] = sg != 0.0 ? wsx * sg : 0.0;
-                            teth[slot + 4 * (size_t)cap] = sg != 0.0 ? wsy * sg : 0.0;
-                            teth[slot + 5 * (size_t)cap] = sg != 0.0 ? wsz * sg : 0.0;
-                        }
-                    }
-                    __syncthreads();
-                }
-        if (tid < n) {
-            ext[cs[tid]] = vals[tid];
-            slot_of[vals[tid]] = cs[tid];
-        }
-        return;
-    }
-    for (int q = tid; q < n; q += blockDim.x) sl[q] = slot_of[vals[q]];
-    __syncthreads();
+// positions after the passes (r), stored where they changed
+__device__ __forceinline__ void wrap_molecule(const WrapArgs& a, int i, double r[3]) {
+    const double h[3] = {0.5 * a.L[0], 0.5 * a.L[1], 0.5 * a.L[2]};
+    const bool out = (r[0] < -h[0]) | (r[0] >= h[0]) | (r[1] < -h[1]) | (r[1] >= h[1]) | (r[2] < -h[2]) | (r[2] >= h[2]);
+    if (!out) return;
+    const int tg = a.tag ? a.tag[i] : FM_TAG_FREE;
+    const bool held = tg == FM_TAG_TETH || tg == FM_TAG_TETH_SLIDE;
+    int m = 0;
     for (int it = 0; it < 3; ++it)
+#pragma unroll
         for (int ax = 0; ax < 3; ++ax)
-            for (int dir = -1; dir <= 1; dir += 2) {
-                const double h = 0.5 * L[ax];
-                // ordered compaction of leavers into lst[0..k)
-                if (tid == 0) chunk_base = 0;
-                __syncthreads();
-                for (int base = 0; base < n; base += blockDim.x) {
-                    int q = base + tid;
-                    int lv = 0;
-                    if (q < n) {
-                        double r = pos[ax][sl[q]];
-                        lv = dir == -1 ? (r < -h) : (r >= h);
-                    }
-                    unsigned long long m = __ballot(lv);
-                    int rank = __popcll(m & ((1ull << lane) - 1ull));
-                    if (lane == 0) wsum[wid] = __popcll(m);
-                    __syncthreads();
-                    int off = 0, tot = 0;
-                    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-                        if (w < wid) off += wsum[w];
-                        tot += wsum[w];
-                    }
-                    if (lv) lst[chunk_base + off + rank] = q;
-                    __syncthreads();
-                    if (tid == 0) chunk_base += tot;
-                    __syncthreads();
+#pragma unroll
+            for (int dir = -1; dir <= 1; dir += 2)
+                if (dir == -1 ? r[ax] < -h[ax] : r[ax] >= h[ax]) {
+                    r[ax] = r[ax] - (double)dir * a.L[ax];
+                    if (held) a.teth[i + (size_t)ax * a.cap] = a.teth[i + (size_t)ax * a.cap] - (double)dir * a.L[ax];
+                    m |= 1 << (it * 6 + ax * 2 + (dir + 1) / 2);
                 }
-                const int k = chunk_base;
-                if (k == 0) continue;
-                // wrap the leavers: r(ixyz) - dir*domain(ixyz)
-                for (int m = tid; m < k; m += blockDim.x) {
-                    int slot = sl[lst[m]];
-                    pos[ax][slot] = pos[ax][slot] - (double)dir * L[ax];
-                    if (tag_move && (tag[slot] == FM_TAG_TETH || tag[slot] == FM_TAG_TETH_SLIDE))
-                        teth[slot + (size_t)ax * cap] = teth[slot + (size_t)ax * cap] - (double)dir * L[ax];
-                }
-                __syncthreads();
-                for (int m = tid; m < k; m += blockDim.x) tmp[m] = sl[lst[k - 1 - m]];
-                __syncthreads();
-                for (int m = tid; m < k; m += blockDim.x) {
-                    int slot = tmp[m];
-                    sl[lst[m]] = slot;
-                    if (tag_move) {  // read_tag on the renumbered molecule
-                        const int tg = tag[slot];
-                        const double sg = tg == FM_TAG_TETH_SLIDE   ? copysign(1.0, s.y[slot])
-                                          : tg == FM_TAG_FIXED_SLIDE ? 1.0
-                                                                     : 0.0;
-                        teth[slot + 3 * (size_t)cap] = sg != 0.0 ? wsx * sg : 0.0;
-                        teth[slot + 4 * (size_t)cap] = sg != 0.0 ? wsy * sg : 0.0;
-                        teth[slot + 5 * (size_t)cap] = sg != 0.0 ? wsz * sg : 0.0;
-                    }
-                }
-                __syncthreads();
-            }
-    for (int q = tid; q < n; q += blockDim.x) {
-        ext[sl[q]] = vals[q];
-        slot_of[vals[q]] = sl[q];
+    a.s.x[i] = r[0];
+    a.s.y[i] = r[1];
+    a.s.z[i] = r[2];
+    if (a.tag) {
+        // read_tag on the renumbered molecule (the last pass it left in saw its final y)
+        const double sg = tg == FM_TAG_TETH_SLIDE ? copysign(1.0, r[1]) : tg == FM_TAG_FIXED_SLIDE ? 1.0 : 0.0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) a.teth[i + (size_t)(3 + d) * a.cap] = sg != 0.0 ? a.ws[d] * sg : 0.0;
+    }
+    a.mask[i] = m;
+    const int e = a.ext[i];
+    atomicOr(&a.bits[e >> 5], 1u << (e & 31));
+}
+
+__global__ __launch_bounds__(FM_BLOCK) void k_wrap(WrapArgs a) {
+    if (blockIdx.x == 0 && (int)threadIdx.x < a.reset.n) reset_flag(a.flags, a.reset.w[threadIdx.x]);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= a.np) return;
+    double r[3] = {a.s.x[i], a.s.y[i], a.s.z[i]};
+    wrap_molecule(a, i, r);
+}
+
+// Exclusive prefix of v over the workgroup's threads (1024 of them); *total: the sum.  wsum: 16 ints.
+__device__ __forceinline__ int block_prefix(int v, int* wsum, int* total) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    int x = v;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
+    }
+    __syncthreads();  // (wsum may still be read from the call before)
+    if (lane == 63) wsum[wid] = x;
+    __syncthreads();
+    int pre = x - v, tot = 0;
+    for (int w = 0; w < nw; ++w) {
+        const int t = wsum[w];
+        if (w < wid) pre += t;
+        tot += t;
+    }
+    *total = tot;
+    return pre;
+}
+
+// The passes over n leavers by list position q: number V[q] (ascending, fixed), the slot S[q] that
+// carries it and that molecule's passes M[q].  lst, tS, tM: scratch of n each.
+__device__ __forceinline__ void renumber_passes(int n, int passes, int* S, int* M, int* lst, int* tS, int* tM, int* wsum) {
+    const int tid = threadIdx.x, nt = blockDim.x;
+    for (; passes; passes &= passes - 1) {
+        const int bit = passes & -passes;
+        int k = 0;
+        for (int base = 0; base < n; base += nt) {
+            const int q = base + tid;
+            const int lv = q < n && (M[q] & bit) ? 1 : 0;
+            int tot;
+            const int p = block_prefix(lv, wsum, &tot);
+            if (lv) lst[k + p] = q;
+            k += tot;
+        }
+        __syncthreads();
+        for (int m = tid; m < k; m += nt) {
+            const int q = lst[k - 1 - m];
+            tS[m] = S[q];
+            tM[m] = M[q];
+        }
+        __syncthreads();
+        for (int m = tid; m < k; m += nt) {
+            S[lst[m]] = tS[m];
+            M[lst[m]] = tM[m];
+        }
+        __syncthreads();
     }
 }
 
-// Lanes of a wavefront that add to the same counter are served by one atomic: returns each
-// active lane's position among the additions to its counter (consecutive slots mostly share a
-// cell, so a wavefront issues a handful of atomics instead of 64).
+struct RenumArgs {
+    int np;
+    unsigned* bits;
+    const int* mask;
+    int *ext, *slot_of;
+    int* scratch;          // 6 x cap ints, for more than RENUM_LDS leavers
+    int cap;
+    int set_slots;         // write slot_of too (a binning that follows rewrites it)
+    int* flags;
+};
+#define RENUM_LDS 2048
+
+// sendmols' numbers: one workgroup of 1024 threads.  The leavers are read off the bit map in
+// ascending molecule number (each thread a contiguous range of its words, cleared as they are read).
+// When every leaver left in one pass only, no pass moves a number that another one looks at, so all
+// of them are done at once: the position of each leaver among those of its pass, and the slot of the
+// one as far from that pass's end.  A molecule that left in two (an edge of the box: one rebuild in
+// some) makes it the passes in turn, those that some molecule left in.
+// Bound: one workgroup's chain of dependent loads (bits, slots, masks) and barriers.  In a queued
+// rebuild it is one workgroup of the scan's launch.  With the selection it replaced a one-workgroup
+// kernel of 18 passes and a launch that read every position through slot_of (23.6 + 12.1 us a
+// rebuild at 1,048,576 molecules, 17.5 + 3.3 us at 2,048).
+__device__ void renumber(const RenumArgs& a) {
+    constexpr int NW = RENUM_LDS / 64;  // wavefronts' worth of leavers
+    __shared__ int wsum[16], lds[6][RENUM_LDS], cnt[18 * NW + 1], all, multi;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    // 16-byte words, a contiguous run of them per thread
+    const int nv = (a.np + 127) >> 7, per = (nv + (int)blockDim.x - 1) / (int)blockDim.x;
+    const int v0 = min(nv, tid * per), v1 = min(nv, v0 + per);
+    uint4* const B = (uint4*)a.bits;
+    int mine = 0;
+#pragma unroll 8
+    for (int v = v0; v < v1; ++v) {
+        const uint4 w = B[v];
+        mine += __popc(w.x) + __popc(w.y) + __popc(w.z) + __popc(w.w);
+    }
+    if (tid == 0) all = multi = 0;
+    int n;
+    int pos = block_prefix(mine, wsum, &n);
+    const bool small = n <= RENUM_LDS;
+    int* V = small ? lds[0] : a.scratch;
+    int* S = small ? lds[1] : a.scratch + a.cap;
+    int* M = small ? lds[2] : a.scratch + 2 * (size_t)a.cap;
+    for (int u = v0; mine && u < v1; u += 8) {
+        uint4 w[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) w[k] = B[min(u + k, v1 - 1)];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const unsigned c[4] = {w[k].x, w[k].y, w[k].z, w[k].w};
+            if (u + k >= v1 || (c[0] | c[1] | c[2] | c[3]) == 0u) continue;
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+                for (unsigned m = c[d]; m; m &= m - 1) V[pos++] = ((u + k) << 7) + (d << 5) + __ffs((int)m) - 1;
+            B[u + k] = make_uint4(0u, 0u, 0u, 0u);
+        }
+    }
+    __syncthreads();
+    int o = 0;
+    bool two = false;
+    for (int q = tid; q < n; q += blockDim.x) {
+        const int slot = a.slot_of[V[q]], m = a.mask[slot];
+        S[q] = slot;
+        M[q] = m;
+        o |= m;
+        two = two || (m & (m - 1)) != 0;
+    }
+    if (o) atomicOr(&all, o);
+    if (two) multi = 1;
+    __syncthreads();
+    if (!small) {
+        renumber_passes(n, all, S, M, a.scratch + 3 * (size_t)a.cap, a.scratch + 4 * (size_t)a.cap,
+                        a.scratch + 5 * (size_t)a.cap, wsum);
+    } else if (multi) {
+        renumber_passes(n, all, S, M, lds[3], lds[4], lds[5], wsum);
+    } else {
+        // cnt[pass][wavefront]: leavers, then their exclusive prefix in that order
+        int rank[RENUM_LDS / 1024];
+        for (int k = tid; k <= 18 * NW; k += blockDim.x) cnt[k] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < RENUM_LDS / 1024; ++c) {
+            const int q = c * 1024 + tid, m = q < n ? M[q] : 0;
+            rank[c] = 0;
+            for (int ps = all; ps; ps &= ps - 1) {
+                const unsigned long long in = __ballot(m & ps & -ps);
+                if (m & ps & -ps) rank[c] = __popcll(in & ((1ull << lane) - 1ull));
+                if (lane == 0) cnt[(__ffs(ps) - 1) * NW + c * 16 + wid] = __popcll(in);
+            }
+        }
+        __syncthreads();
+        static_assert(18 * NW <= 1024, "a count per thread");
+        int tot;
+        const int pre = block_prefix(tid < 18 * NW ? cnt[tid] : 0, wsum, &tot);
+        if (tid <= 18 * NW) cnt[tid] = pre;
+        __syncthreads();
+        int* lst = lds[3];
+        int* out = lds[4];
+        int p[RENUM_LDS / 1024];
+#pragma unroll
+        for (int c = 0; c < RENUM_LDS / 1024; ++c) {
+            const int q = c * 1024 + tid;
+            p[c] = 0;
+            if (q < n) {
+                const int b = __ffs(M[q]) - 1, at = cnt[b * NW + c * 16 + wid] + rank[c];
+                lst[at] = q;
+                p[c] = cnt[b * NW] + cnt[(b + 1) * NW] - 1 - at;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < RENUM_LDS / 1024; ++c)
+            if (c * 1024 + tid < n) out[c * 1024 + tid] = S[lst[p[c]]];
+        S = out;  // (each thread reads its own below)
+    }
+    for (int q = tid; q < n; q += blockDim.x) {
+        a.ext[S[q]] = V[q];
+        if (a.set_slots) a.slot_of[V[q]] = S[q];
+    }
+    __syncthreads();
+    // an escaped molecule met by k_bin_count before the renumbering: its slot, as ~slot
+    if (tid == 0 && a.flags[FLAG_ERROR] == FM_EESCAPE && a.flags[FLAG_ERROR_MOL] < 0)
+        a.flags[FLAG_ERROR_MOL] = a.ext[~a.flags[FLAG_ERROR_MOL]];
+}
+
+__global__ __launch_bounds__(1024) void k_renumber(RenumArgs a) { renumber(a); }
+
+// Each active lane's position among the additions to its counter.  Lanes of a wavefront with the
+// same counter are served by one atomic (consecutive slots mostly share a cell), and the wavefront's
+// atomics go out together after the lanes are grouped: one round trip, where an atomic inside the
+// grouping loop made it one per distinct cell (16.5 us for the 2,048 molecules of a WCA box with 2.8
+// a cell).
 __device__ inline int wave_aggregated_add(int* counters, int key, bool active) {
     const int lane = threadIdx.x & 63;
-    unsigned long long mask = __ballot(active);
-    int pos = -1;
-    while (mask) {
-        const int leader = __ffsll((long long)mask) - 1;
-        const int lk = __shfl(key, leader, 64);
-        const unsigned long long same = __ballot(active && key == lk) & mask;
-        int base = 0;
-        if (lane == leader) base = atomicAdd(&counters[lk], __popcll(same));
-        base = __shfl(base, leader, 64);
-        if ((same >> lane) & 1ull) pos = base + __popcll(same & ((1ull << lane) - 1ull));
-        mask &= ~same;
+    unsigned long long todo = __ballot(active);
+    int leader = lane, rank = 0, cnt = 0;
+    while (todo) {
+        const int l = __ffsll((long long)todo) - 1;
+        const unsigned long long same = __ballot(active && key == __builtin_amdgcn_readlane(key, l));
+        if ((same >> lane) & 1ull) {
+            leader = l;
+            rank = __popcll(same & ((1ull << lane) - 1ull));
+            cnt = __popcll(same);
+        }
+        todo &= ~same;
     }
-    return pos;
+    int base = 0;
+    if (active && lane == leader) base = atomicAdd(&counters[key], cnt);
+    return __shfl(base, leader, 64) + rank;
 }
 
 // ---- assign_to_cell as a counting sort, src/linklist.f90:2645-2676 -----------------------------
-__global__ __launch_bounds__(FM_BLOCK) void k_bin_count(St s, const int* ext, int np, double hx, double hy,
-                                                        double hz, double csx, double csy, double csz,
-                                                        int nx, int ny, int nz, int* cell_of,
-                                                        int* count, int* pos_out, int* flags) {
+struct BinArgs {
+    double h[3], cs[3];
+    int nc[3];
+    int *cell_of, *count, *pos;
+};
+
+// WRAP: sendmols' wrap first (a queued rebuild: one pass over the positions for both)
+template <bool WRAP>
+__global__ __launch_bounds__(FM_BLOCK) void k_bin_count(WrapArgs a, BinArgs b) {
+    if (WRAP && blockIdx.x == 0 && (int)threadIdx.x < a.reset.n) reset_flag(a.flags, a.reset.w[threadIdx.x]);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     int cell = -1;
-    if (i < np) {
-        double r[3] = {s.x[i], s.y[i], s.z[i]};
-        const double h[3] = {hx, hy, hz}, cs[3] = {csx, csy, csz};
-        const int n[3] = {nx, ny, nz};
-        int c[3];
+    if (i < a.np) {
+        double r[3] = {a.s.x[i], a.s.y[i], a.s.z[i]};
+        if (WRAP) wrap_molecule(a, i, r);
+        int c[3] = {0, 0, 0};
         bool ok = true;
-        for (int d = 0; d < 3 && ok; ++d) {
-            double t = r[d] + h[d];
-            if (!(t > -cs[d] && t < (double)(n[d] + 1) * cs[d])) {  // also rejects NaN
-                ok = false;
-                break;
-            }
-            int ic = (int)ceil(t / cs[d]) + 1;  // 1-based with one halo layer
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            double t = r[d] + b.h[d];
+            ok = ok && t > -b.cs[d] && t < (double)(b.nc[d] + 1) * b.cs[d];  // also rejects NaN
+            int ic = ok ? (int)ceil(t / b.cs[d]) + 1 : 0;  // 1-based with one halo layer
             if (ic == 1 && t == 0.0) {  // exactly on the lower face: the reference's ceiling() gives the halo
-                atomicAdd(&flags[FLAG_EDGE], 1);
+                atomicAdd(&a.flags[FLAG_EDGE], 1);
                 ic = 2;
             }
-            if (ic < 2 || ic > n[d] + 1) {
-                ok = false;
-                break;
-            }
+            ok = ok && ic >= 2 && ic <= b.nc[d] + 1;
             c[d] = ic - 2;
         }
         if (ok) {
-            cell = c[0] + nx * (c[1] + ny * c[2]);
-            cell_of[i] = cell;
+            cell = c[0] + b.nc[0] * (c[1] + b.nc[1] * c[2]);
         } else {
             // counted in cell 0 so that the permutation stays complete; the error stops the run
-            set_err(flags, FM_EESCAPE, ext[i]);
+            // (WRAP: the renumbering that follows turns ~slot into the molecule's number)
+            set_err(a.flags, FM_EESCAPE, WRAP ? ~i : a.ext[i]);
             cell = 0;
-            cell_of[i] = 0;
         }
+        b.cell_of[i] = cell;
     }
     // the molecule's place among its cell's molecules (the order within a cell is arbitrary
     // here: k_bin_order orders each cell by x, ties by molecule number)
-    const int pos = wave_aggregated_add(count, cell, cell >= 0);
-    if (i < np) pos_out[i] = pos;
+    const int pos = wave_aggregated_add(b.count, cell, cell >= 0);
+    if (i < a.np) b.pos[i] = pos;
+}
+
+// start[0..n) = exclusive prefix of the cells' counts, CELL_CH cells a workgroup.  A workgroup adds
+// up the counts before its own: by itself from the counts (part null: up to CELL_DIRECT cells, where
+// the last workgroup's read of them all costs less than the launch that would sum the chunks), or
+// from the chunk sums of k_cell_part.  The counts stay (k_bin_order zeroes them).  One more
+// workgroup, when asked, does sendmols' renumbering, which nothing before k_bin_order reads.
+#define CELL_CH 4096
+#define CELL_DIRECT (1 << 18)
+__global__ __launch_bounds__(1024) void k_cell_part(const int* count, int* part, int n) {
+    __shared__ int wsum[16];
+    int v = 0, tot;
+    for (int k = 0; k < 4; ++k) {
+        const int i = blockIdx.x * CELL_CH + 4 * threadIdx.x + k;
+        v += i < n ? count[i] : 0;
+    }
+    block_prefix(v, wsum, &tot);
+    if (threadIdx.x == 0) part[blockIdx.x] = tot;
+}
+
+__global__ __launch_bounds__(1024) void k_cell_scan(const int* count, int* start, const int* part, int n, int nscan,
+                                                    RenumArgs ra) {
+    __shared__ int wsum[16];
+    if ((int)blockIdx.x == nscan) {
+        renumber(ra);
+        return;
+    }
+    const int tid = threadIdx.x;
+    int before = 0, v[4], s = 0, tot;
+    if (part) {
+        for (int b = tid; b < (int)blockIdx.x; b += blockDim.x) before += part[b];
+    } else {
+        const int4* c4 = (const int4*)count;  // (whole chunks: in range)
+#pragma unroll 4
+        for (int b = 0; b < (int)blockIdx.x; ++b) {
+            const int4 w = c4[b * (CELL_CH / 4) + tid];
+            before += (w.x + w.y) + (w.z + w.w);
+        }
+    }
+    const int i0 = blockIdx.x * CELL_CH + 4 * tid;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        v[k] = i0 + k < n ? count[i0 + k] : 0;
+        s += v[k];
+    }
+    int off;
+    block_prefix(before, wsum, &off);
+    int pre = off + block_prefix(s, wsum, &tot);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (i0 + k < n) {
+            start[i0 + k] = pre;
+            pre += v[k];
+        }
 }
 
 // start[0..n) = exclusive prefix of count[0..n), in chunks of SCAN_CH counts (FM_BLOCK threads,
 // four consecutive counts each): k_scan_part sums each chunk; k_scan_fin adds up the sums of the
 // chunks before its own, scans its chunk (by thread, wavefront and workgroup) and writes the
-// prefixes.  The counts are zeroed as they are read (ready for the next binning) and so is
-// cursor[0..ncur).
+// prefixes (the radix sort's digit counts).
 #define SCAN_CH (4 * FM_BLOCK)
 __device__ inline int block_sum(int v, int* wsum) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -569,8 +656,7 @@ __global__ __launch_bounds__(FM_BLOCK) void k_scan_part(const int* count, int* p
     if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
-__global__ __launch_bounds__(FM_BLOCK) void k_scan_fin(int* count, int* start, const int* part, int n, int* cursor,
-                                                       int ncur) {
+__global__ __launch_bounds__(FM_BLOCK) void k_scan_fin(const int* count, int* start, const int* part, int n) {
     __shared__ int wsum[FM_BLOCK / 64];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     // the sums of the chunks before this one
@@ -598,10 +684,8 @@ __global__ __launch_bounds__(FM_BLOCK) void k_scan_fin(int* count, int* start, c
     for (int k = 0; k < 4; ++k)
         if (i0 + k < n) {
             start[i0 + k] = pre;
-            count[i0 + k] = 0;
             pre += v[k];
         }
-    for (int i = blockIdx.x * FM_BLOCK + tid; i < ncur; i += gridDim.x * FM_BLOCK) cursor[i] = 0;
 }
 
 __global__ __launch_bounds__(FM_BLOCK) void k_bin_scatter(const int* cell_of, const int* start, const int* pos,
@@ -639,6 +723,7 @@ struct PermArgs {
     double* teth_dst;
     int* slot_of;
     const int *start, *perm;
+    int* count;          // zeroed for the next binning
     int ncell, maxcell, cap;
     int* flags;
     int nf;  // state fields moved: 9, or 6 when the accelerations are about to be recomputed
@@ -741,6 +826,7 @@ __global__ __launch_bounds__(FM_BLOCK) void k_bin_order(PermArgs a) {
     if (c0 >= a.ncell) return;  // whole wavefront (each keeps to its own 64 LDS keys)
     const int hl = PER == 2 ? lane & 31 : lane, c = c0 + (PER == 2 ? lane >> 5 : 0);
     const int b = c < a.ncell ? a.start[c] : 0, n = c < a.ncell ? a.start[c + 1] - b : 0;
+    if (hl == 0 && c < a.ncell) a.count[c] = 0;
     if (n > a.maxcell && hl == 0) set_err(a.flags, FM_EOVERFLOW, c);
     if (PER == 2 && __builtin_amdgcn_ballot_w64(n > 32) == 0ull) {
         const bool own = hl < n;
@@ -1139,7 +1225,7 @@ int radix_sort_pairs(fm_ctx* c, int* k0, int* v0, int* k1, int* v1, int n, int e
     for (int shift = 0; shift < end_bit; shift += 8) {
         k_radix_hist<<<nt, FM_BLOCK, 0, c->stream>>>(k0, n, shift, hist, nt);
         k_scan_part<<<nscan, FM_BLOCK, 0, c->stream>>>(hist, part, nh);
-        k_scan_fin<<<nscan, FM_BLOCK, 0, c->stream>>>(hist, start, part, nh, nullptr, 0);
+        k_scan_fin<<<nscan, FM_BLOCK, 0, c->stream>>>(hist, start, part, nh);
         k_radix_scatter<<<nt, FM_BLOCK, 0, c->stream>>>(k0, v0, k1, v1, n, shift, start, nt);
         LAUNCH_CHECK();
         std::swap(k0, k1);
@@ -1212,47 +1298,85 @@ int launch_check_vmax(fm_ctx* c) {
     return 0;
 }
 
-int launch_sendmols(fm_ctx* c, const int* reset, int nreset) {
+static int make_wrap(fm_ctx* c, WrapArgs& a, const int* reset, int nreset) {
     if (nreset > 8) return fm_set_error(FM_EINVAL, "reset of %d flag words", nreset);
-    FlagList l;
-    l.n = nreset;
-    for (int k = 0; k < nreset; ++k) l.w[k] = reset[k];
-    if (c->np == 0) return nreset ? launch_reset_flags(c, reset, nreset) : 0;
-    ktimer_begin(c, KT_SENDMOLS);
-    St s = state_of(c->x(), c->cap);
-    const int nb = nblocks(c->np);
-    // segments in the flag buffer, counts in out_count; lst and tmp of the passes reuse the cell
-    // permutation buffer and the flag buffer (after the gather)
-    k_out_select<<<nb, FM_BLOCK, 0, c->stream>>>(s, c->slot_of, c->np, c->half[0], c->half[1], c->half[2],
-                                                   c->out_flag, c->out_count, c->d_flags, l);
-    LAUNCH_CHECK();
     const bool tm = c->p.ensemble == FM_ENSEMBLE_TAG_MOVE && c->has_tags;
-    k_sendmols_passes<<<1, 1024, 0, c->stream>>>(
-        s, tm ? c->teth[c->cur] : nullptr, tm ? c->tag[c->cur] : nullptr, c->ext[c->cur], c->slot_of,
-        c->out_flag, c->out_count, nb, c->out_vals, c->out_slot, c->perm, c->out_flag, c->cap, c->p.domain[0],
-        c->p.domain[1], c->p.domain[2], tm ? 1 : 0, c->p.wallslidev[0], c->p.wallslidev[1], c->p.wallslidev[2]);
+    a.s = state_of(c->x(), c->cap);
+    a.ext = c->ext[c->cur];
+    a.tag = tm ? c->tag[c->cur] : nullptr;
+    a.teth = tm ? c->teth[c->cur] : nullptr;
+    a.np = c->np;
+    a.cap = c->cap;
+    for (int d = 0; d < 3; ++d) {
+        a.L[d] = c->p.domain[d];
+        a.ws[d] = c->p.wallslidev[d];
+    }
+    a.mask = c->out_mask;
+    a.bits = c->out_bits;
+    a.flags = c->d_flags;
+    a.reset.n = nreset;
+    for (int k = 0; k < nreset; ++k) a.reset.w[k] = reset[k];
+    return 0;
+}
+
+static RenumArgs make_renum(fm_ctx* c, bool set_slots) {
+    RenumArgs r;
+    r.np = c->np;
+    r.bits = c->out_bits;
+    r.mask = c->out_mask;
+    r.ext = c->ext[c->cur];
+    r.slot_of = c->slot_of;
+    r.scratch = (int*)c->stage;  // 9*cap doubles, used by host transfers only
+    r.cap = c->cap;
+    r.set_slots = set_slots ? 1 : 0;
+    r.flags = c->d_flags;
+    return r;
+}
+
+int launch_sendmols(fm_ctx* c, const int* reset, int nreset) {
+    if (c->np == 0) return nreset ? launch_reset_flags(c, reset, nreset) : 0;
+    WrapArgs w;
+    if (int rc = make_wrap(c, w, reset, nreset)) return rc;
+    ktimer_begin(c, KT_SENDMOLS);
+    k_wrap<<<nblocks(c->np), FM_BLOCK, 0, c->stream>>>(w);
+    LAUNCH_CHECK();
+    k_renumber<<<1, 1024, 0, c->stream>>>(make_renum(c, true));
     ktimer_end(c, KT_SENDMOLS);
     LAUNCH_CHECK();
     return 0;
 }
 
-int launch_bin(fm_ctx* c, bool keep_acc) {
+// send: sendmols first, in the binning's own launches (its wrap with the cell counts, its
+// renumbering beside the scan), zeroing the listed flags.  sort_mols, which renumbers between the
+// two, needs them apart.
+int launch_bin(fm_ctx* c, bool keep_acc, bool send, const int* reset, int nreset) {
     c->btab_valid = false;  // new cells: the staging tables wait for the next list build
-    if (c->np == 0) return 0;
+    if (c->np == 0) return nreset ? launch_reset_flags(c, reset, nreset) : 0;
+    WrapArgs w;
+    if (int rc = make_wrap(c, w, reset, nreset)) return rc;
     ktimer_begin(c, KT_BIN);
-    St s = state_of(c->x(), c->cap);
     const int nxt = 1 - c->cur;
     int* cell_tmp = c->out_flag;  // cell index in old slot order
-    k_bin_count<<<nblocks(c->np), FM_BLOCK, 0, c->stream>>>(s, c->ext[c->cur], c->np, c->half[0], c->half[1],
-                                                             c->half[2], c->cs[0], c->cs[1], c->cs[2], c->nc[0],
-                                                             c->nc[1], c->nc[2], cell_tmp, c->cell_count,
-                                                             c->bin_pos, c->d_flags);
+    BinArgs b;
+    for (int d = 0; d < 3; ++d) {
+        b.h[d] = c->half[d];
+        b.cs[d] = c->cs[d];
+        b.nc[d] = c->nc[d];
+    }
+    b.cell_of = cell_tmp;
+    b.count = c->cell_count;
+    b.pos = c->bin_pos;
+    if (send) k_bin_count<true><<<nblocks(c->np), FM_BLOCK, 0, c->stream>>>(w, b);
+    else k_bin_count<false><<<nblocks(c->np), FM_BLOCK, 0, c->stream>>>(w, b);
     LAUNCH_CHECK();
-    const int nscan = (c->ncell + 1 + SCAN_CH - 1) / SCAN_CH;
-    k_scan_part<<<nscan, FM_BLOCK, 0, c->stream>>>(c->cell_count, c->scan_part, c->ncell + 1);
-    LAUNCH_CHECK();
-    k_scan_fin<<<nscan, FM_BLOCK, 0, c->stream>>>(c->cell_count, c->cell_start, c->scan_part, c->ncell + 1,
-                                                  nullptr, 0);
+    const int n = c->ncell + 1, nscan = (n + CELL_CH - 1) / CELL_CH;
+    const bool part = n > CELL_DIRECT;
+    if (part) {
+        k_cell_part<<<nscan, 1024, 0, c->stream>>>(c->cell_count, c->scan_part, n);
+        LAUNCH_CHECK();
+    }
+    k_cell_scan<<<nscan + (send ? 1 : 0), 1024, 0, c->stream>>>(c->cell_count, c->cell_start, part ? c->scan_part : nullptr,
+                                                                n, nscan, make_renum(c, false));
     LAUNCH_CHECK();
     k_bin_scatter<<<nblocks(c->np), FM_BLOCK, 0, c->stream>>>(cell_tmp, c->cell_start, c->bin_pos, c->perm,
                                                                c->np);
@@ -1274,6 +1398,7 @@ int launch_bin(fm_ctx* c, bool keep_acc) {
     a.slot_of = c->slot_of;
     a.start = c->cell_start;
     a.perm = c->perm;
+    a.count = c->cell_count;
     a.ncell = c->ncell;
     a.maxcell = c->p.max_cell_np > 0 ? c->p.max_cell_np : (1 << 26);
     a.cap = c->cap;

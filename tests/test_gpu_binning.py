@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from flowmol_amd import config
+from flowmol_amd._abi import FM_ENSEMBLE_TAG_MOVE, FM_INTEGRATION_LFV, FM_TAG_FIXED_SLIDE
 from flowmol_amd.md import MDContext
 from oracle.oracle import Oracle
 from tests.helpers import canonical_pairs
@@ -53,3 +54,51 @@ def test_cells_of_any_size(counts):
     g.assign_to_neighbourlist()
     assert np.array_equal(canonical_pairs(*o.neighbourlist()), canonical_pairs(*g.neighbourlist()))
     g.close()
+
+
+def near_faces(r, L, count, corners, lo, hi, seed):
+    """r with `count` molecules moved to between lo and hi beyond an upper face of the box (a lower one
+    too when lo is positive), `corners` of them at two or three faces."""
+    rng = np.random.default_rng(seed)
+    r = r.copy()
+    for k, n in enumerate(rng.permutation(r.shape[0])[:count]):
+        for ax in rng.permutation(3)[: (2 + k % 2) if k < corners else 1]:
+            side = rng.choice([-1.0, 1.0]) if lo >= 0.0 else 1.0
+            r[n, ax] = side * (0.5 * L[ax] + rng.uniform(lo, hi))
+    return r
+
+
+@pytest.mark.parametrize("count,corners", [(0, 0), (1, 0), (63, 0), (65, 1), (1024, 0), (1025, 0), (1025, 3),
+                                           (2048, 0), (2049, 0), (2500, 40)])
+def test_renumbering_of_any_leaver_count(count, corners):
+    """sendmols' numbers and positions, alone and inside the binning of a queued rebuild, for leaver
+    counts around the wavefront, the workgroup and its LDS, with and without molecules that leave
+    across an edge."""
+    say(f"case: {count} of 3960 molecules outside the box, {corners} across edges")
+    p, r, v = config.config_fcc((10, 9, 11), 0.8, 2.5, seed=8, tplot=1)
+    out = near_faces(r, p.domain, count, corners, 0.0, 0.3, seed=9)
+    o, g = Oracle(p, out, v), MDContext(p, out, v)
+    for x in (o, g):
+        x.sendmols()
+    for ref, got in zip(o.state()[:2], g.state()[:2]):
+        assert np.array_equal(ref, got)
+    g.close()
+    # the queued rebuild: every molecule slides by 0.2 along x, y and z a step, whatever its force
+    p.ensemble, p.integration_algorithm = FM_ENSEMBLE_TAG_MOVE, FM_INTEGRATION_LFV
+    for d in range(3):
+        p.wallslidev[d] = 0.2 / p.delta_t
+    inside = near_faces(r, p.domain, count, corners, -0.19, -0.01, seed=9)
+    ends = []
+    for queued in (False, True):
+        g = MDContext(p, inside, v)
+        g.set_tags(np.full(r.shape[0], FM_TAG_FIXED_SLIDE, np.int32))
+        g.setup(0)
+        if queued:
+            g.run_lfv(0, 3)
+        else:
+            for it in range(3):
+                g.md_advance_lfv(it)
+        ends.append(g.state() + (g.rtether(),))
+        g.close()
+    for ref, got in zip(*ends):
+        assert np.array_equal(ref, got, equal_nan=True)
