@@ -211,9 +211,45 @@ static int set_brick(fm_ctx* c, const int b[3]) {
     return 0;
 }
 
-// Brick shape: the largest number of cells whose expected molecule count fits one pass of the
-// workgroup (15/16 of its threads), preferring the shape with the least staged halo per cell.
+// Brick shape: the least estimated time of a force launch, among the shapes whose expected molecule
+// count fits one pass of the workgroup (15/16 of its threads).  A workgroup's time goes with the
+// molecules R that it stages (its cells and one halo layer; about 11 ns a molecule and 3 us beside
+// them, the pair loop running under the staging of the CU's other workgroup), and 512 workgroups run
+// at once, two on a CU where the staged regions leave room for two.  So a large domain takes the
+// shape with the least halo per cell (1,048,576 molecules: 3x3x3 cells, 2197 bricks), and one whose
+// bricks would leave workgroup slots empty takes smaller ones, as many as the slots.  Measured, a step
+// of 108,000 molecules (rc 2.5): 3x3x3 (216 bricks) 48.5 us, 3x2x2 (486) 37.1, 2x2x2 (729) 45.5; of
+// 55,296 with rc 4: 2x3x1 78.6 us, 1x1x1 (729, two on a CU) 67.5, 2x1x1 (405, one on a CU) 83; of 5,148:
+// 3x3x2 27.3 us, 1x2x1 (120) 18.5 and with teams of lanes 14.6, 1x1x1 (210) 14.3: single cells of few
+// molecules are left out (each molecule would be staged 27 times over for nothing).
 static void choose_brick(const int nc[3], double occ, int out[3]) {
+    const double target = FB_BLOCK * 15.0 / 16.0;
+    double best = -1.0;
+    out[0] = out[1] = out[2] = 1;
+    for (int bx = 1; bx <= std::min(nc[0], 12); ++bx)
+        for (int by = 1; by <= std::min(nc[1], 12); ++by)
+            for (int bz = 1; bz <= std::min(nc[2], 12); ++bz) {
+                const int P = bx * by * bz;
+                if (P > 1 && P * occ > target) continue;
+                if (P == 1 && occ < 48.0 && 2.0 * occ <= target) continue;
+                const double R = (bx + 2) * (by + 2) * (bz + 2) * occ;
+                const double nb = (double)((nc[0] + bx - 1) / bx) * ((nc[1] + by - 1) / by) * ((nc[2] + bz - 1) / bz);
+                // (27 B a staged molecule with its share of the tables; the largest region 15 % above the mean)
+                const double slots = 256.0 * (R * 1.15 * 27.0 <= 80.0 * 1024.0 ? 2 : 1);
+                const double cost = (nb <= slots ? 1.0 : nb / slots + 0.2) * (R + 300.0);
+                // (of equal ones the longest along x, the order of the slots)
+                if (best < 0.0 || cost <= best * (1.0 + 1e-12)) {
+                    best = cost;
+                    out[0] = bx;
+                    out[1] = by;
+                    out[2] = bz;
+                }
+            }
+}
+
+// The shape with the least halo per cell (mixed precision, whose FP32 sums depend on the shape: the
+// staged offsets are rounded relative to the region's corner)
+static void choose_brick_halo(const int nc[3], double occ, int out[3]) {
     const double target = FB_BLOCK * 15.0 / 16.0;
     double best = -1.0;
     out[0] = out[1] = out[2] = 1;
@@ -230,6 +266,25 @@ static void choose_brick(const int nc[3], double occ, int out[3]) {
                     out[2] = bz;
                 }
             }
+}
+
+static void default_brick(const fm_params* p, const int nc[3], double occ, int out[3]) {
+    if (p->precision == FM_PREC_MIXED) choose_brick_halo(nc, occ, out);
+    else choose_brick(nc, occ, out);
+}
+
+// Lanes per molecule of the force launches: two where a brick's molecules leave over a quarter of the
+// workgroup's threads idle, more while they take at most half of them and a lane keeps two words of the
+// expected list.  Measured at 5,148 molecules (1x1x1 bricks of 25, 73 entries): 1 lane 19.5 us a step,
+// 2 15.6, 4 14.9, 8 14.3, 16 15.4; at 55,296 with rc 4 (bricks of 76, 266 entries): 1 lane 89 us, 2 71.7,
+// 4 71.9, 16 80; 131,072 beads (bricks of 306): 1 lane 71.9 us, 2 68.5, 4 71.4.  One lane in mixed
+// precision (FP32 sums).
+static int team_of(const fm_ctx* c, double occ, double entries) {
+    if (c->p.precision == FM_PREC_MIXED) return 1;
+    const double I = (double)c->brick[0] * c->brick[1] * c->brick[2] * occ;
+    int T = 1;
+    while (T < 16 && 2 * T * I <= (T == 1 ? 1.4 * FB_BLOCK : 0.5 * FB_BLOCK) && 2 * T * 8 <= entries) T *= 2;
+    return T;
 }
 
 // Block curve of sort_mols: SORT_FLAG 1 numbers the blocks x fastest
@@ -357,7 +412,7 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
     if (p->brick[0] > 0 && p->brick[1] > 0 && p->brick[2] > 0) {
         for (int d = 0; d < 3; ++d) c->brick[d] = std::min(p->brick[d], c->nc[d]);
     } else {
-        choose_brick(c->nc, std::max(1.0, (double)np / c->ncell), c->brick);
+        default_brick(p, c->nc, std::max(1.0, (double)np / c->ncell), c->brick);
     }
     {
         hipDeviceProp_t prop;
@@ -371,10 +426,13 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
 
     // neighbour capacity: 1.5x the expected count at the mean density, plus margin
     int maxnb = p->max_neighbours;
+    const double dens = std::max(p->density, np / (p->domain[0] * p->domain[1] * p->domain[2]));
+    const double expect = 4.0 / 3.0 * M_PI * rneighbr * rneighbr * rneighbr * dens;
+    {
+        const double occ = std::max(1.0, (double)np / c->ncell);
+        c->team = team_of(c, occ, expect);
+    }
     if (maxnb <= 0) {
-        double vol = p->domain[0] * p->domain[1] * p->domain[2];
-        double dens = std::max(p->density, np / vol);
-        double expect = 4.0 / 3.0 * M_PI * rneighbr * rneighbr * rneighbr * dens;
         maxnb = (int)(1.5 * expect) + 32;
         maxnb = (maxnb + 3) & ~3;
     }
@@ -568,7 +626,7 @@ extern "C" int fm_memory_footprint(const fm_params* p, int32_t np, int64_t* byte
         if (p->brick[0] > 0 && p->brick[1] > 0 && p->brick[2] > 0) {
             for (int d = 0; d < 3; ++d) br[d] = std::min(p->brick[d], nc[d]);
         } else {
-            choose_brick(nc, std::max(1.0, (double)np / ncell), br);
+            default_brick(p, nc, std::max(1.0, (double)np / ncell), br);
         }
         double halo = 1.0;
         for (int d = 0; d < 3; ++d) halo *= (br[d] + 2.0) / br[d];
@@ -1209,9 +1267,12 @@ static int rebuild_lists_queued(fm_ctx* c, bool resets, bool keep_acc);
 // 1e-12 margin over the force kernels' own test on the same values).  The entries keep the order
 // of the full list (the cell windows and the runs are those of the list radius), and an entry
 // beyond rc adds exactly zero to every force, PE and virial sum, so each sum is the full list's,
-// bit for bit.  Only for pairs that all end at rc: no bonds, no Mie tables.
+// bit for bit.  Only for pairs that all end at rc: no bonds, no Mie tables; and one lane per molecule
+// (teams deal a list's words to their lanes, so leaving entries out changes the partial sums).
+static bool skinless_lists(const fm_ctx* c) { return c->p.potential_flag == 0 && c->p.mie_potential == 0 && c->team == 1; }
+
 static int rebuild_lists_for(fm_ctx* c, bool read_once, bool queued) {
-    const bool skinless = read_once && c->p.potential_flag == 0 && c->p.mie_potential == 0;
+    const bool skinless = read_once && skinless_lists(c);
     c->list_ra2 = skinless ? c->rc2 * (1.0 + 1e-12) : 0.0;
     const int rc = queued ? rebuild_lists_queued(c, true, false) : rebuild_lists(c);
     c->list_ra2 = 0.0;
@@ -1546,8 +1607,7 @@ static int run_lfv_queued(fm_ctx* c, int iter0, int nsteps, fm_macros* macros, i
                 c->rdisp_valid = false;
                 // the loop's last list serves whatever runs next: full radius, accelerations kept
                 const bool last = k + 1 >= end;
-                const bool skinless = !last && lfv_rebuild_known(c, k + 1) && c->p.potential_flag == 0 &&
-                                      c->p.mie_potential == 0;
+                const bool skinless = !last && lfv_rebuild_known(c, k + 1) && skinless_lists(c);
                 c->list_ra2 = skinless ? c->rc2 * (1.0 + 1e-12) : 0.0;
                 const int rc = rebuild_lists_queued(c, false, last);
                 c->list_ra2 = 0.0;

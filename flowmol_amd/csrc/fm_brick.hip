@@ -951,6 +951,7 @@ struct FbArgs {
     const double* planes;
     int* flags;
     int cap, maxreg;
+    int team;              // lanes that share a molecule's list (a power of two up to 16; team_of)
     int rec, ev;
     int kick;              // fused simulation_move_particles_vv(2): v += (0.5*dt)*a
     double hdt;
@@ -1134,49 +1135,70 @@ __device__ __forceinline__ void lj_word_rec(const P4& p, int left, double xi, do
     }
 }
 
+// ---- teams ----------------------------------------------------------------------------------------
+// T lanes (1, 2, 4, 8 or 16, neighbours in a wavefront) share a molecule where a brick has fewer
+// molecules than its workgroup has threads: lane t takes the words t, t + T, ... of its list, the
+// partial sums are added across the lanes by halves, and lane 0 goes on with the molecule.  The split
+// depends on the context alone (team_of), so every launch of a context sums alike; T = 1 is the loop
+// of one lane per molecule.  A lane's list is a serial chain of LDS reads and pair terms: a small
+// domain, whose bricks leave most of the chip's lanes idle, takes as long as its longest chain.
+struct Team {
+    int t, q0, dq, T;  // lane of the team; the workgroup's first molecule of this thread and its stride
+};
+__device__ __forceinline__ Team team_lane(int T) {
+    const int sh = 31 - __clz(T);
+    return Team{(int)threadIdx.x & (T - 1), (int)threadIdx.x >> sh, (int)blockDim.x >> sh, T};
+}
+template <typename V>
+__device__ __forceinline__ V team_sum(V v, int T) {
+    for (int o = 1; o < T; o <<= 1) v = v + __shfl_xor(v, o, 64);
+    return v;
+}
+
 // REC: also the molecule's PE and virial (lj_word_rec).
 template <bool REC = false>
 __device__ __forceinline__ void lj_plain(const double* pos, const uint64_t* row, int n, size_t cap, double xi,
-                                         double yi, double zi, double rc2, double& fx, double& fy, double& fz,
-                                         double potshift = 0.0, double* pe_out = nullptr, double* vir_out = nullptr) {
+                                         double yi, double zi, double rc2, const Team& tm, double& fx, double& fy,
+                                         double& fz, double potshift = 0.0, double* pe_out = nullptr,
+                                         double* vir_out = nullptr) {
     double sx = 0, sy = 0, sz = 0;
     double pe = 0.0, vt = 0.0;
     P4 pa, pb;
-    // At the top of each pass pa holds the positions of word k = kw/4, w1 is word k+1 and w2
-    // word k+2 (in flight).  Word loads past the end re-read the last word (the row always has
+    // At the top of each pass pa holds the positions of word k = kw/4, w1 is the lane's next word and
+    // w2 the one after (in flight).  Word loads past the end re-read the last word (the row always has
     // at least one word), so no load sits behind a branch and each wait is for the oldest load;
     // a pass always evaluates both words (the second one masked off past the end) so that the
     // loop body is one block and the loads stay ahead of their uses.
-    const int lastw = n > 0 ? (n - 1) >> 2 : 0;
-    uint64_t w0 = row[0];
-    lj_stage(pa, pos, n > 0 ? w0 : 0);
-    uint64_t w1 = row[(size_t)min(1, lastw) * cap];
-    uint64_t w2 = row[(size_t)min(2, lastw) * cap];
-    for (int kw = 0; kw < n; kw += 8) {
+    const int lastw = n > 0 ? (n - 1) >> 2 : 0, T = tm.T, T4 = 4 * T;
+    uint64_t w0 = row[(size_t)min(tm.t, lastw) * cap];
+    lj_stage(pa, pos, 4 * tm.t < n ? w0 : 0);
+    uint64_t w1 = row[(size_t)min(tm.t + T, lastw) * cap];
+    uint64_t w2 = row[(size_t)min(tm.t + 2 * T, lastw) * cap];
+    for (int kw = 4 * tm.t; kw < n; kw += 2 * T4) {
         const int k = kw >> 2;
-        lj_stage(pb, pos, kw + 4 < n ? w1 : 0);
+        lj_stage(pb, pos, kw + T4 < n ? w1 : 0);
         // both words two ahead are loaded here, at the top of the pass: the wait the compiler
         // places at the loop head is then for loads a whole pass old
         const uint64_t wk2 = w2;
-        w1 = row[(size_t)min(k + 3, lastw) * cap];
-        w2 = row[(size_t)min(k + 4, lastw) * cap];
+        w1 = row[(size_t)min(k + 3 * T, lastw) * cap];
+        w2 = row[(size_t)min(k + T4, lastw) * cap];
         __builtin_amdgcn_sched_barrier(0);  // keep the reads above the evaluation
         if constexpr (REC) lj_word_rec(pa, n - kw, xi, yi, zi, rc2, potshift, sx, sy, sz, pe, vt);
         else lj_word(pa, n - kw, xi, yi, zi, rc2, sx, sy, sz);
-        lj_stage(pa, pos, kw + 8 < n ? wk2 : 0);
+        lj_stage(pa, pos, kw + 2 * T4 < n ? wk2 : 0);
         __builtin_amdgcn_sched_barrier(0);
         // the second word only when a lane of the wavefront has entries in it
-        if (__builtin_amdgcn_ballot_w64(kw + 4 < n) != 0ull) {
-            if constexpr (REC) lj_word_rec(pb, n - kw - 4, xi, yi, zi, rc2, potshift, sx, sy, sz, pe, vt);
-            else lj_word(pb, n - kw - 4, xi, yi, zi, rc2, sx, sy, sz);
+        if (__builtin_amdgcn_ballot_w64(kw + T4 < n) != 0ull) {
+            if constexpr (REC) lj_word_rec(pb, n - kw - T4, xi, yi, zi, rc2, potshift, sx, sy, sz, pe, vt);
+            else lj_word(pb, n - kw - T4, xi, yi, zi, rc2, sx, sy, sz);
         }
     }
-    fx = 24.0 * sx;
-    fy = 24.0 * sy;
-    fz = 24.0 * sz;
+    fx = 24.0 * team_sum(sx, T);
+    fy = 24.0 * team_sum(sy, T);
+    fz = 24.0 * team_sum(sz, T);
     if constexpr (REC) {
-        *pe_out = pe;
-        *vir_out = 24.0 * vt;
+        *pe_out = team_sum(pe, T);
+        *vir_out = 24.0 * team_sum(vt, T);
     }
 }
 
@@ -1327,7 +1349,8 @@ __device__ __forceinline__ void forces_body(const FbArgs& a, int brick, char* sm
     const size_t cap = a.cap;
     // a record step that tallies PE and virial only (no MOP, CV or rfmol)
     const bool simple_rec = RECORD && (SIMPLE || (!mop && !cvrec && a.rf == nullptr));
-    for (int q = threadIdx.x; q < r.ni; q += blockDim.x) {
+    const Team tm = team_lane(a.team);
+    for (int q = tm.q0; q < r.ni; q += tm.dq) {
         int rci = 0, li, i;
         if (tab) {
             i = tab[2 + a.maxreg + q];
@@ -1354,21 +1377,21 @@ __device__ __forceinline__ void forces_body(const FbArgs& a, int brick, char* sm
         const uint64_t* row = a.nbl + i;
         bool looped = false;  // the pairs went through the branch-free loop
         if constexpr (!MIE && !RECORD && !VIR) {
-            lj_plain(r.pos, row, n, cap, xi, yi, zi, a.rc2, fx, fy, fz);
+            lj_plain(r.pos, row, n, cap, xi, yi, zi, a.rc2, tm, fx, fy, fz);
             looped = true;
         } else if constexpr (!MIE && RECORD && VIR && !EXTRA) {
             if (simple_rec) {  // PE and virial only
-                lj_plain<true>(r.pos, row, n, cap, xi, yi, zi, a.rc2, fx, fy, fz, a.potshift, &pe, &vir);
+                lj_plain<true>(r.pos, row, n, cap, xi, yi, zi, a.rc2, tm, fx, fy, fz, a.potshift, &pe, &vir);
                 looped = true;
             }
         }
         // Four 16-bit entries per word.  The next word is loaded while this one is worked on,
         // and the four entries' positions are read from LDS together (the unused entries of a
         // last, partial word are 0, a valid region index).
-        uint64_t wnext = n > 0 ? row[0] : 0;
-        for (int kw = 0; !looped && kw < n; kw += 4) {
+        uint64_t wnext = 4 * tm.t < n ? row[(size_t)tm.t * cap] : 0;
+        for (int kw = 4 * tm.t; !looped && kw < n; kw += 4 * tm.T) {
             const uint64_t word = wnext;
-            if (kw + 4 < n) wnext = row[(size_t)((kw >> 2) + 1) * cap];
+            if (kw + 4 * tm.T < n) wnext = row[(size_t)((kw >> 2) + tm.T) * cap];
             int jq[4];
             double rxq[4], ryq[4], rzq[4];
 #pragma unroll
@@ -1434,6 +1457,16 @@ __device__ __forceinline__ void forces_body(const FbArgs& a, int brick, char* sm
             }
         }
         }
+        if (!looped && tm.T > 1) {
+            fx = team_sum(fx, tm.T);
+            fy = team_sum(fy, tm.T);
+            fz = team_sum(fz, tm.T);
+            if (VIR) vir = team_sum(vir, tm.T);
+            if (RECORD) pe = team_sum(pe, tm.T);
+            if (do_rf)
+                for (int k = 0; k < 9; ++k) rf[k] = team_sum(rf[k], tm.T);
+        }
+        if (tm.t != 0) continue;
         if constexpr (EXTRA) bond_tether_forces<RECORD, VIR>(a, i, xi, yi, zi, inv_mi, do_rf, rf, fx, fy, fz, vir);
         if constexpr (P1) {  // (k_forces_brick_plain only: its one argument is the FbArgs)
             const FbArgs& b = fargs_again();
@@ -1596,32 +1629,35 @@ __device__ __forceinline__ void mie_word(const P4M& p, int left, double xi, doub
 template <int NT, int NB, bool REC>
 __device__ __forceinline__ void mie_plain(const double* pos, const uint8_t* lt, const uint64_t* row, int n,
                                           size_t cap, double xi, double yi, double zi, const MieRow<NT, REC>& m,
-                                          double& fx, double& fy, double& fz, double& pe, double& vt) {
+                                          const Team& tm, double& fx, double& fy, double& fz, double& pe,
+                                          double& vt) {
     double sx = 0, sy = 0, sz = 0, spe = 0, svt = 0;
     P4M pa, pb;
-    const int lastw = n > 0 ? (n - 1) >> 2 : 0;
-    const uint64_t w0 = row[0];
-    mie_stage(pa, pos, lt, n > 0 ? w0 : 0);
-    uint64_t w1 = row[(size_t)min(1, lastw) * cap];
-    uint64_t w2 = row[(size_t)min(2, lastw) * cap];
-    for (int kw = 0; kw < n; kw += 8) {
+    const int lastw = n > 0 ? (n - 1) >> 2 : 0, T = tm.T, T4 = 4 * T;
+    const uint64_t w0 = row[(size_t)min(tm.t, lastw) * cap];
+    mie_stage(pa, pos, lt, 4 * tm.t < n ? w0 : 0);
+    uint64_t w1 = row[(size_t)min(tm.t + T, lastw) * cap];
+    uint64_t w2 = row[(size_t)min(tm.t + 2 * T, lastw) * cap];
+    for (int kw = 4 * tm.t; kw < n; kw += 2 * T4) {
         const int k = kw >> 2;
-        mie_stage(pb, pos, lt, kw + 4 < n ? w1 : 0);
+        mie_stage(pb, pos, lt, kw + T4 < n ? w1 : 0);
         const uint64_t wk2 = w2;
-        w1 = row[(size_t)min(k + 3, lastw) * cap];
-        w2 = row[(size_t)min(k + 4, lastw) * cap];
+        w1 = row[(size_t)min(k + 3 * T, lastw) * cap];
+        w2 = row[(size_t)min(k + T4, lastw) * cap];
         __builtin_amdgcn_sched_barrier(0);
         mie_word<NT, NB, REC>(pa, n - kw, xi, yi, zi, m, sx, sy, sz, spe, svt);
-        mie_stage(pa, pos, lt, kw + 8 < n ? wk2 : 0);
+        mie_stage(pa, pos, lt, kw + 2 * T4 < n ? wk2 : 0);
         __builtin_amdgcn_sched_barrier(0);
-        if (__builtin_amdgcn_ballot_w64(kw + 4 < n) != 0ull)
-            mie_word<NT, NB, REC>(pb, n - kw - 4, xi, yi, zi, m, sx, sy, sz, spe, svt);
+        if (__builtin_amdgcn_ballot_w64(kw + T4 < n) != 0ull)
+            mie_word<NT, NB, REC>(pb, n - kw - T4, xi, yi, zi, m, sx, sy, sz, spe, svt);
     }
-    fx = sx;
-    fy = sy;
-    fz = sz;
-    pe = spe;
-    vt = svt;
+    fx = team_sum(sx, T);
+    fy = team_sum(sy, T);
+    fz = team_sum(sz, T);
+    if constexpr (REC) {
+        pe = team_sum(spe, T);
+        vt = team_sum(svt, T);
+    }
 }
 
 // LDS of the branch-free Mie launch: positions, region cell and one-byte type of each staged
@@ -1688,8 +1724,10 @@ __device__ __forceinline__ void forces_body_mie(const FbArgs& a, int brick, char
             (P1 ? a.s2.az : a.s.az)[i] = bz;
             if constexpr (REC) a.vir[i] = vir;
         }
+        if (a.team > 1) __syncthreads();  // (the pair loop's team reads it in another thread)
     }
-    for (int q = threadIdx.x; q < r.ni; q += blockDim.x) {
+    const Team tm = team_lane(a.team);
+    for (int q = tm.q0; q < r.ni; q += tm.dq) {
         int li, i;
         imol_tab(r, a.start, tab, a.maxreg, q, li, i);
         const double xi = r.pos[3 * li], yi = r.pos[3 * li + 1], zi = r.pos[3 * li + 2];
@@ -1698,7 +1736,8 @@ __device__ __forceinline__ void forces_body_mie(const FbArgs& a, int brick, char
         mie_row<NT, NB, REC>(a, ti, m);
         const double inv_mi = 1.0 / a.mie[7 * T2 + ti];
         double fx, fy, fz, pe, vir;
-        mie_plain<NT, NB, REC>(r.pos, r.ltype8, a.nbl + i, a.nbn[i], a.cap, xi, yi, zi, m, fx, fy, fz, pe, vir);
+        mie_plain<NT, NB, REC>(r.pos, r.ltype8, a.nbl + i, a.nbn[i], a.cap, xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
+        if (tm.t != 0) continue;
         const FbArgs& b = KA ? fargs_again() : a;  // the arguments below: not held through the pair loop
         fx = fx * inv_mi;
         fy = fy * inv_mi;
@@ -1859,13 +1898,14 @@ __device__ __forceinline__ void lj_word_mop(const FbArgs& a, const P4K& p, int l
 template <bool SLOTS>
 __device__ __forceinline__ void lj_plain_mop(const FbArgs& a, const double* pos, const int* key,
                                              const uint64_t* row, int n, size_t cap, double xi, double yi,
-                                             double zi, MopI& m, double& fx, double& fy, double& fz,
-                                             double& pe_out, double& vir_out) {
+                                             double zi, MopI& m, const Team& tm, double& fx, double& fy,
+                                             double& fz, double& pe_out, double& vir_out) {
     double sx = 0, sy = 0, sz = 0, pe = 0.0, vt = 0.0;
-    uint64_t wn = row[0];
-    for (int kw = 0; kw < n; kw += 4) {
+    const int T = tm.T;
+    uint64_t wn = 4 * tm.t < n ? row[(size_t)tm.t * cap] : 0;
+    for (int kw = 4 * tm.t; kw < n; kw += 4 * T) {
         const uint64_t w = wn;
-        if (kw + 4 < n) wn = row[(size_t)((kw >> 2) + 1) * cap];
+        if (kw + 4 * T < n) wn = row[(size_t)((kw >> 2) + T) * cap];
         if constexpr (SLOTS) {
 #pragma unroll 1
             for (int q = 0; q < 4; ++q) {
@@ -1883,11 +1923,11 @@ __device__ __forceinline__ void lj_plain_mop(const FbArgs& a, const double* pos,
             lj_word_mop<SLOTS>(a, p, n - kw, xi, yi, zi, m, sx, sy, sz, pe, vt);
         }
     }
-    fx = 24.0 * sx;
-    fy = 24.0 * sy;
-    fz = 24.0 * sz;
-    pe_out = pe;
-    vir_out = 24.0 * vt;
+    fx = 24.0 * team_sum(sx, T);
+    fy = 24.0 * team_sum(sy, T);
+    fz = 24.0 * team_sum(sz, T);
+    pe_out = team_sum(pe, T);
+    vir_out = 24.0 * team_sum(vt, T);
 }
 
 template <bool SLOTS>
@@ -1921,7 +1961,8 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
     m.spxy = spxy;
     m.planes = planes;
     const double rct = sqrt(a.rc2) * m.inv_sp;  // rc in plane spacings
-    for (int q = threadIdx.x; q < r.ni; q += blockDim.x) {
+    const Team tm = team_lane(a.team);
+    for (int q = tm.q0; q < r.ni; q += tm.dq) {
         int li, i;
         imol_tab(r, a.start, tab, a.maxreg, q, li, i);
         const double xi = r.pos[3 * li], yi = r.pos[3 * li + 1], zi = r.pos[3 * li + 2];
@@ -1941,7 +1982,7 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
             }
         }
         double fx, fy, fz, pe, vir;
-        lj_plain_mop<SLOTS>(a, r.pos, r.lslot, a.nbl + i, a.nbn[i], cap, xi, yi, zi, m, fx, fy, fz, pe, vir);
+        lj_plain_mop<SLOTS>(a, r.pos, r.lslot, a.nbl + i, a.nbn[i], cap, xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
         if constexpr (SLOTS) {
 #pragma unroll
             for (int s = 0; s < 3; ++s) {
@@ -1952,6 +1993,7 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
                         if (m.c[s][d] != 0.0) atomicAdd(&spxy[3 * k + d], m.c[s][d]);
             }
         }
+        if (tm.t != 0) continue;
         a.s.ax[i] = fx;
         a.s.ay[i] = fy;
         a.s.az[i] = fz;
@@ -2806,6 +2848,7 @@ int make_fargs(fm_ctx* c, int iter, bool kick, void* out, size_t* lds_out, int* 
     a.flags = c->d_flags;
     a.cap = c->cap;
     a.maxreg = c->maxreg;
+    a.team = c->team;
     const int tplot = c->p.tplot, teval = c->p.teval;
     a.step = iter;
     a.rec = (iter % tplot) == 0;

@@ -321,7 +321,8 @@ FB_BLOCK = 512  # threads of one brick workgroup (FB_BLOCK of the brick kernels)
 def brick_candidates(ncells, nmol, max_candidates=4):
     """Brick shapes (cells along x, y, z) whose expected molecule count fits one pass of a
     workgroup (15/16 of FB_BLOCK threads), least staged halo per cell first.  The first one is the
-    library's default shape for the same cells and occupancy."""
+    library's default for a large domain; a domain of fewer bricks than the device runs at once gets a
+    smaller one by default."""
     nc = [int(x) for x in ncells]
     occ = max(1.0, nmol / float(nc[0] * nc[1] * nc[2]))
     target = FB_BLOCK * 15.0 / 16.0
