@@ -431,6 +431,9 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
     {
         const double occ = std::max(1.0, (double)np / c->ncell);
         c->team = team_of(c, occ, expect);
+        // (the rule of k_nlist_tile)
+        c->tile_list = p->precision == FM_PREC_FP64 && occ <= 40.0 &&
+                       c->brick[0] * c->brick[1] * c->brick[2] * occ <= (p->potential_flag == 1 ? 160.0 : 256.0);
     }
     if (maxnb <= 0) {
         maxnb = (int)(1.5 * expect) + 32;

@@ -16,6 +16,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -927,6 +928,421 @@ k_nlist_quant(NlqArgs a) {
             atomicOr(&a.flags[FLAG_NEED], NEED_LIST);
             a.flags[FLAG_HALT] = 1;
         }
+    }
+}
+
+// ---- neighbour list by matrix tiles: cells freshly binned (sorted by x) ---------------------------
+// The same set as k_nlist_brick.  Sixteen x-consecutive interior molecules of one row of cells are a
+// tile, worked on by one wavefront.  Each of the tile's nine runs (rows of region cells around its
+// own, sorted by x and contiguous in the region layout) is cut to the x window of the whole tile, and
+// the squared distances of 32 candidates to the 16 molecules come from two FP32 matrix products:
+//   D = |rj|^2 - 2 ri.rj + (|ri|^2 - rn^2) = rij^2 - rn^2
+// with rows (x, y, z, |r|^2) of the candidates (from the region's centre), columns (-2x, -2y, -2z, 1)
+// of the molecules and |ri|^2 - rn^2 as the accumulator's start.  A lane of the result holds four
+// candidates of one molecule; the candidates' order in the rows is chosen so that the two products
+// give it eight consecutive ones (an octet), whose sign bits are a byte of its hit mask, and so that
+// octet o always falls to the molecule's lane o mod 4.  A value nearer to zero than the error bound
+// below is decided by the reference's FP64 test (rij2 < rneighbr2, src/linklist.f90:717-720,750-754)
+// on the positions in HBM, so the set is the FP64 set exactly.  Each lane then places its hits in LDS
+// behind those of the molecule's lanes before it, and the words of four entries go to HBM for
+// neighbouring slots together.
+//
+// List order: lane by lane (octet mod 4), run by run, by x.  It does not depend on the radius, so a
+// list of a smaller radius is the larger one's with the farther entries left out.
+//
+// The error bound: with u = 2^-24, h the region's largest half extent and rn the list radius, a staged
+// coordinate is within u h, which moves rij^2 near rn^2 by at most 7 u h rn; the roundings of |ri|^2,
+// |rj|^2 and of the sum are seven of u times (|ri| + |rj|)^2 + rn^2, and |rj| <= |ri| + rn there.  The
+// band taken is four times 7 u ((2 |ri| + rn)^2 + rn^2 + h rn).
+// What bounds it: the latency of one tile (windows, products, placing) where a wavefront has one or two,
+// the issue of about 1,700 instructions a tile where it has many; the products themselves are a
+// fiftieth of them.  A list build took, against k_nlist_quant, whose every lane scans its molecule's
+// windows alone: 25 -> 15 us (2,048 WCA molecules), 46 -> 19 us (5,148, bricks of 49), 54 -> 43 us
+// (108,000, bricks of 222); but 73 -> 78 us at 500 molecules a brick, 265 -> 340 us at 1,048,576 (where
+// the scan keeps the vector units 93 % busy with as many instructions) and 131 -> 148 us at rc 4 (windows
+// of five blocks): bricks of at most 256 molecules (160 with bonds, 124 -> 100 us at 153 and 90 -> 95 us at
+// 306) and cells of at most 40 take the tiles.  Mixed precision keeps the scan and its order of entries,
+// on which FP32 sums depend.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+#define NLT_TILE 16
+#define NLT_PAD 64      // candidates read past the region's end (masked off)
+#define NLT_PEND 32     // waiting bond candidates of a molecule
+
+struct NltArgs {
+    St s;
+    BG g;
+    const int* start;
+    uint64_t* nbl;
+    int* nbn;
+    int* flags;
+    int cap, maxnb, maxreg;
+    double ra2;              // pairs kept: r^2 < ra2 (as NlbArgs)
+    float xw, rn, hext;      // window half-width with its margin, list radius, the bound's h
+    int wbytes;              // LDS of one wavefront's buffers
+    double cs[3], hd[3];
+    const int* order;
+    // bond discovery (POLY): monomer fields in slot order, the bond lists, molecule numbers
+    const int* mono;
+    uint32_t* bond;
+    int* bondn;
+    const int* ext;
+    // the bricks' staging tables for the force launches (stage_from_table)
+    int* btab;
+    int btab_stride;
+};
+
+__host__ __device__ inline size_t nlt_wave_bytes(int maxnb, bool poly) {
+    return ((size_t)NLT_TILE * (maxnb + (poly ? NLT_PEND : 0)) * 2 + 15) & ~(size_t)15;
+}
+// LDS before the wavefronts' buffers (which share their space with the staged molecules' region cells)
+__host__ __device__ inline size_t nlt_fixed_bytes(const BG& g, int maxreg, bool poly) {
+    const int nbmax = g.B[0] * g.B[1] * g.B[2];
+    const size_t b = (size_t)(maxreg + NLT_PAD) * (poly ? 20 : 16) +
+                     (size_t)(4 * g.nreg + 1 + 2 * nbmax + 1 + g.B[1] * g.B[2] + 1 + 2) * sizeof(int);
+    return (b + 15) & ~(size_t)15;
+}
+
+// slot and image shift of region index j, by a search over the region cells (rare: undecided pairs)
+__device__ __forceinline__ void region_slot(const Region& r, const BG& g, int j, int& slot, int& sh) {
+    int lo = 0, hi = g.nreg - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (r.off[mid] <= j) lo = mid;
+        else hi = mid - 1;
+    }
+    slot = r.cst[lo] + (j - r.off[lo]);
+    sh = r.sh[lo];
+}
+// the reference's FP64 test of interior molecule li and region entry j
+__device__ __forceinline__ bool nlt_exact(const NltArgs& a, const Region& r, int li, int j) {
+    int si, sj, shi, shj, sx, sy, sz;
+    region_slot(r, a.g, li, si, shi);
+    region_slot(r, a.g, j, sj, shj);
+    decode_shift(shj, sx, sy, sz);
+    const double dx = a.s.x[si] - img(a.s.x[sj], sx, a.g.L[0]), dy = a.s.y[si] - img(a.s.y[sj], sy, a.g.L[1]),
+                 dz = a.s.z[si] - img(a.s.z[sj], sz, a.g.L[2]);
+    return ((dx * dx + dy * dy) + dz * dz) < a.ra2;
+}
+
+// orders a wavefront's LDS writes before the reads of its other lanes (and reads before later writes)
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <bool POLY>
+__global__ __launch_bounds__(FB_BLOCK) __attribute__((amdgpu_waves_per_eu(FB_BLOCK / 128))) void k_nlist_tile(NltArgs a) {
+    extern __shared__ __align__(16) char smem[];
+    const BG& g = a.g;
+    float* pos = (float*)smem;  // x, y, z from the region's centre, |r|^2
+    int* ip = (int*)(pos + 4 * (size_t)(a.maxreg + NLT_PAD));
+    uint32_t* chs = nullptr;    // POLY: chain id << 7 | subchain id (127: no bond flag)
+    if (POLY) {
+        chs = (uint32_t*)ip;
+        ip += a.maxreg + NLT_PAD;
+    }
+    Region r;
+    r.pos = nullptr;
+    r.lslot = nullptr;
+    r.off = ip;
+    ip += g.nreg + 1;
+    r.gc = ip;
+    ip += g.nreg;
+    r.sh = ip;
+    ip += g.nreg;
+    r.cst = ip;
+    ip += g.nreg;
+    r.ic_off = ip;
+    ip += g.B[0] * g.B[1] * g.B[2] + 1;
+    r.ic_rc = ip;
+    ip += g.B[0] * g.B[1] * g.B[2];
+    int* tp = ip;               // tiles before each row of interior cells
+    ip += g.B[1] * g.B[2] + 1;
+    int* ctr = ip;              // next tile
+    char* wbuf = smem + nlt_fixed_bytes(g, a.maxreg, POLY);
+    r.rq = (uint16_t*)wbuf;     // (read while staging only)
+    const int brick = brick_of_block(a.order, blockIdx.x, gridDim.x);
+    if (!stage_tables(r, g, brick, a.start, a.maxreg, a.flags)) return;
+    const int bx = brick % g.nb[0], by = (brick / g.nb[0]) % g.nb[1], bz = brick / (g.nb[0] * g.nb[1]);
+    const int ex = min(g.B[0], g.nc[0] - bx * g.B[0]), ey = min(g.B[1], g.nc[1] - by * g.B[1]),
+              ez = min(g.B[2], g.nc[2] - bz * g.B[2]);
+    const int R0 = g.R[0], R1 = g.R[1], lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    {
+        const double ox = -a.hd[0] + (bx * g.B[0] + 0.5 * g.B[0]) * a.cs[0];
+        const double oy = -a.hd[1] + (by * g.B[1] + 0.5 * g.B[1]) * a.cs[1];
+        const double oz = -a.hd[2] + (bz * g.B[2] + 0.5 * g.B[2]) * a.cs[2];
+        constexpr int SU = 6;  // molecules per thread and pass, loads first (as stage_region)
+        for (int q0 = threadIdx.x; q0 < r.total; q0 += SU * blockDim.x) {
+            int sl[SU], sc[SU];
+            double px[SU], py[SU], pz[SU];
+#pragma unroll
+            for (int k = 0; k < SU; ++k) {
+                const int qc = min(q0 + k * (int)blockDim.x, r.total - 1);
+                const int rc = r.rq[qc];
+                sl[k] = r.cst[rc] + (qc - r.off[rc]);
+                sc[k] = r.sh[rc];
+                px[k] = a.s.x[sl[k]];
+                py[k] = a.s.y[sl[k]];
+                pz[k] = a.s.z[sl[k]];
+            }
+#pragma unroll
+            for (int k = 0; k < SU; ++k) {
+                const int q = q0 + k * (int)blockDim.x;
+                if (q >= r.total) break;
+                int sx, sy, sz;
+                decode_shift(sc[k], sx, sy, sz);
+                const float x = (float)(img(px[k], sx, g.L[0]) - ox), y = (float)(img(py[k], sy, g.L[1]) - oy),
+                            z = (float)(img(pz[k], sz, g.L[2]) - oz);
+                const double w = ((double)x * x + (double)y * y) + (double)z * z;
+                *(f32x4*)(pos + 4 * q) = f32x4{x, y, z, (float)w};
+                if (POLY) {
+                    const int sub = a.mono[sl[k] + (size_t)a.cap];
+                    chs[q] = (uint32_t)a.mono[sl[k]] << 7 | (uint32_t)(sub >= 1 && sub <= 124 ? sub : 127);
+                }
+                a.btab[(size_t)brick * a.btab_stride + 2 + q] = (sl[k] << 5) | sc[k];
+            }
+        }
+        if (threadIdx.x == 0) {
+            a.btab[(size_t)brick * a.btab_stride] = r.total;
+            a.btab[(size_t)brick * a.btab_stride + 1] = r.ni;
+            *ctr = 0;
+        }
+        if (wid == 0) {  // tiles of the rows (x fastest, then y, z), and their prefix
+            for (int k = lane; k < ey * ez; k += 64) {
+                const int c0 = 1 + R0 * ((k % ey + 1) + R1 * (k / ey + 1));
+                tp[k] = (r.off[c0 + ex] - r.off[c0] + NLT_TILE - 1) / NLT_TILE;
+            }
+            wave0_scan(tp, ey * ez);
+        }
+    }
+    // (rows read past the region's end: finite values, masked off by their |r|^2)
+    for (int q = 4 * r.total + threadIdx.x; q < 4 * (r.total + NLT_PAD); q += blockDim.x) pos[q] = 0.0f;
+    __syncthreads();
+    const int nrows = ey * ez, ntiles = tp[nrows];
+    const size_t cap = a.cap;
+    uint16_t* const lb = (uint16_t*)(wbuf + (size_t)wid * a.wbytes);  // this wavefront's list entries
+    uint16_t* const pend = lb + NLT_TILE * a.maxnb;
+    const float ra2f = (float)a.ra2;
+    const int c = lane & 15, gl = lane >> 4;  // molecule of the tile, lane of the molecule
+    int wmax = 0;
+    for (;;) {
+        int t = 0;
+        if (lane == 0) t = atomicAdd(ctr, 1);
+        t = __builtin_amdgcn_readfirstlane(t);
+        if (t >= ntiles) break;
+        int rw = -1;  // the last row whose first tile is not beyond t
+        for (int k0 = 0; k0 < nrows; k0 += 64)
+            rw += __popcll(__builtin_amdgcn_ballot_w64(k0 + lane < nrows && tp[min(k0 + lane, nrows)] <= t));
+        const int ry = rw % ey + 1, rz = rw / ey + 1, rowc = R0 * (ry + R1 * rz);
+        const int li0 = r.off[rowc + 1] + NLT_TILE * (t - tp[rw]), n16 = min(NLT_TILE, r.off[rowc + 1 + ex] - li0);
+        // the runs' windows: lane k < 9 finds run k's first candidate, lane 9 + k its end
+        int jbv, lenv;
+        {
+            const int k = lane < 9 ? lane : (lane < 18 ? lane - 9 : 0);
+            const int rk = R0 * ((ry + k % 3 - 1) + R1 * (rz + k / 3 - 1));
+            const bool end = lane >= 9;
+            const float edge = end ? pos[4 * (li0 + n16 - 1)] + a.xw : pos[4 * li0] - a.xw;
+            int lo = r.off[rk], hi = r.off[rk + R0];
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                const float x = pos[4 * mid];
+                if (end ? x <= edge : x < edge) lo = mid + 1;
+                else hi = mid;
+            }
+            jbv = lo;
+            lenv = __shfl(lo, min(lane + 9, 63), 64) - lo;
+            if (lane >= 9) lenv = 0;
+        }
+        int nb = (lenv + (jbv & 7) + 31) >> 5;  // blocks of four octets of the longest run
+        for (int d = 8; d > 0; d >>= 1) nb = max(nb, __shfl_xor(nb, d, 64));
+        nb = __builtin_amdgcn_readfirstlane(nb);
+        const int li = li0 + min(c, n16 - 1);
+        const bool act = c < n16;
+        const float wi = pos[4 * li + 3], q2 = 2.0f * sqrtf(wi) + a.rn;
+        const float band = (28.0f / 16777216.0f) * (q2 * q2 + ra2f + a.hext * a.rn);
+        const float pv = pos[4 * li + gl], bop = gl < 3 ? -2.0f * pv : 1.0f;
+        const f32x4 cin = {wi - ra2f, wi - ra2f, wi - ra2f, wi - ra2f};
+        // block b of run k (first octet o0): this lane's octet starts at candidate jl + 32 b; row
+        // 4 q + e of the first product is candidate e of lane q's octet, of the second candidate 4 + e
+        auto octet = [&](int o0, int q) { return 8 * (o0 + ((q - o0) & 3)); };
+        auto block_mask = [&](int k, int jb, int len, int b) -> uint32_t {
+            const int o0 = jb >> 3, jr = octet(o0, c >> 2) + (c & 3) + 32 * b, jl = octet(o0, gl) + 32 * b;
+            float a0 = pos[4 * jr + gl], a1 = pos[4 * jr + 16 + gl];
+            // candidates outside the window: a huge |r|^2 (the other components are finite)
+            if (gl == 3) {
+                a0 = (unsigned)(jr - jb) < (unsigned)len ? a0 : 1e30f;
+                a1 = (unsigned)(jr + 4 - jb) < (unsigned)len ? a1 : 1e30f;
+            }
+            const f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, bop, cin, 0, 0, 0);
+            const f32x4 d1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, bop, cin, 0, 0, 0);
+            uint32_t m = 0;
+            float near = 1e30f;
+#pragma unroll
+            for (int e = 3; e >= 0; --e) {
+                m = __builtin_amdgcn_alignbit(m, __float_as_uint(d1[e]), 31);
+                near = fminf(near, fabsf(d1[e]));
+            }
+#pragma unroll
+            for (int e = 3; e >= 0; --e) {
+                m = __builtin_amdgcn_alignbit(m, __float_as_uint(d0[e]), 31);
+                near = fminf(near, fabsf(d0[e]));
+            }
+            if (__builtin_amdgcn_ballot_w64(near < band) != 0ull) {
+                uint32_t u = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    u |= (fabsf(d0[e]) < band ? 1u << e : 0u) | (fabsf(d1[e]) < band ? 16u << e : 0u);
+                for (; u; u &= u - 1) {
+                    const int e = __builtin_ctz(u);
+                    m = (m & ~(1u << e)) | (nlt_exact(a, r, li, jl + e) ? 1u << e : 0u);
+                }
+            }
+            if (k == 4 && (unsigned)(li - jl) < 8u) m &= ~(1u << (li - jl));  // not itself
+            return m;
+        };
+        uint16_t* const row = lb + c * a.maxnb;
+        // hits of mask m (bytes: octets 32 candidates apart, the first at jl) to entries e..
+        auto place = [&](uint32_t m, int jl, int& e) {
+            while (m) {
+                const int b = __builtin_ctz(m);
+                m &= m - 1;
+                row[e++] = (uint16_t)(jl + b + 24 * (b >> 3));
+            }
+        };
+        auto place_checked = [&](uint32_t m, int jl, int& e) {
+            for (; m; m &= m - 1, ++e) {
+                const int b = __builtin_ctz(m);
+                if (e < a.maxnb) row[e] = (uint16_t)(jl + b + 24 * (b >> 3));
+            }
+        };
+        // entries of the molecule's lanes before this one, and of all (cnt)
+        auto lane_prefix = [&](int mine, int& cnt) {
+            int x = mine, y = __shfl_up(x, 16, 64);
+            if (gl >= 1) x += y;
+            y = __shfl_up(x, 32, 64);
+            if (gl >= 2) x += y;
+            cnt = __shfl(x, 48 + c, 64);
+            return x - mine;
+        };
+        int cnt, e;
+        if (nb <= 4) {  // each run's mask in a register
+            uint32_t w[9];
+            int mine = 0;
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {
+                const int jb = __builtin_amdgcn_readlane(jbv, k), len = __builtin_amdgcn_readlane(lenv, k);
+                w[k] = 0;
+                for (int b = 0; 32 * b < len + (jb & 7); ++b) w[k] |= block_mask(k, jb, len, b) << (8 * b);
+                mine += __popc(w[k]);
+            }
+            if (!act) mine = 0;
+            e = lane_prefix(mine, cnt);
+            const bool over = __builtin_amdgcn_ballot_w64(cnt > a.maxnb) != 0ull;
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {
+                const int jl = octet(__builtin_amdgcn_readlane(jbv, k) >> 3, gl);
+                const uint32_t m = act ? w[k] : 0u;
+                if (!over) place(m, jl, e);
+                else place_checked(m, jl, e);
+            }
+        } else {  // wider windows: the masks twice, to count and to place
+            for (int pass = 0; pass < 2; ++pass) {
+                int mine = 0;
+                for (int k = 0; k < 9; ++k) {
+                    const int jb = __builtin_amdgcn_readlane(jbv, k), len = __builtin_amdgcn_readlane(lenv, k);
+                    const int n = (len + (jb & 7) + 31) >> 5;
+                    for (int b0 = 0; b0 < n; b0 += 4) {
+                        uint32_t m = 0;
+                        for (int b = b0; b < min(b0 + 4, n); ++b) m |= block_mask(k, jb, len, b) << (8 * (b - b0));
+                        if (!act) m = 0;
+                        if (pass == 0) mine += __popc(m);
+                        else place_checked(m, octet(jb >> 3, gl) + 32 * b0, e);
+                    }
+                }
+                if (pass == 0) e = lane_prefix(mine, cnt);
+            }
+        }
+        wmax = max(wmax, act ? cnt : 0);
+        wave_sync();
+        const int n = min(cnt, a.maxnb);
+        int rc = rowc + 1;
+        for (int k = 1; k < ex; ++k) rc += li >= r.off[rowc + 1 + k] ? 1 : 0;
+        const int slot = r.cst[rc] + (li - r.off[rc]);
+        if (act) {
+            for (int w = gl; 4 * w < n; w += 4) {
+                uint64_t word = *(const uint64_t*)(row + 4 * w);
+                const int left = n - 4 * w;
+                if (left < 4) word &= (1ull << (16 * left)) - 1ull;
+                a.nbl[(size_t)w * cap + slot] = word;
+            }
+            if (gl == 0) {
+                a.nbn[slot] = n;
+                int* const T = a.btab + (size_t)brick * a.btab_stride + 2 + a.maxreg;
+                const int qi = r.ic_off[ex * rw] + (li - r.off[rowc + 1]);
+                T[qi] = slot;
+                ((uint16_t*)(T + a.maxreg))[qi] = (uint16_t)li;
+            }
+        }
+        if constexpr (POLY) {
+            // the bonds (check_update_adjacentbeadinfo, src/linklist.f90:2542-2584; a bonded partner
+            // lies within R0 <= r_n, so it is an entry): the entries of the molecule's own chain
+            // (25 bits of its id) that carry its bond flag wait in entry order, and those whose full
+            // chain id is the molecule's own are its bonds
+            int bf[4], nbd = 0, np = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) bf[q] = a.mono[slot + (size_t)(3 + q) * cap];
+            const int chain = a.mono[slot], funcy = a.mono[slot + 2 * cap];
+            uint64_t mine = 0;  // the molecule's lanes
+#pragma unroll
+            for (int q = 0; q < 4; ++q) mine |= 1ull << (16 * q + c);
+            const uint64_t below = mine & ((1ull << lane) - 1ull);
+            const uint32_t own = chs[li] >> 7;
+            auto flush = [&]() {
+                wave_sync();
+                for (int p0 = 0; __builtin_amdgcn_ballot_w64(p0 < np) != 0ull; p0 += 4) {
+                    int sj = 0, sh = 0;
+                    bool ok = act && p0 + gl < np;
+                    if (ok) {
+                        region_slot(r, g, pend[c * NLT_PEND + p0 + gl], sj, sh);
+                        ok = a.mono[sj] == chain;
+                    }
+                    const uint64_t on = __builtin_amdgcn_ballot_w64(ok);
+                    const int at = nbd + __popcll(on & below);
+                    if (ok && at < funcy && at < FM_MAX_FUNCY)
+                        a.bond[(size_t)at * cap + slot] = (uint32_t)sj << 5 | (uint32_t)sh;
+                    nbd += __popcll(on & mine);
+                }
+                np = 0;
+                wave_sync();
+            };
+            for (int e0 = 0; __builtin_amdgcn_ballot_w64(act && e0 < n) != 0ull; e0 += 4) {
+                int j = 0;
+                bool ok = act && e0 + gl < n;
+                if (ok) {
+                    j = row[e0 + gl];
+                    const uint32_t w = chs[j];
+                    ok = (w >> 7) == own && (w & 127u) != 127u && bondflag_of(bf, (int)(w & 127u));
+                }
+                const uint64_t on = __builtin_amdgcn_ballot_w64(ok);
+                if (on == 0ull) continue;
+                if (ok) pend[c * NLT_PEND + np + __popcll(on & below)] = (uint16_t)j;
+                np += __popcll(on & mine);
+                if (__builtin_amdgcn_ballot_w64(np > NLT_PEND - 4) != 0ull) flush();
+            }
+            flush();
+            if (act && gl == 0) {
+                a.bondn[slot] = nbd < funcy ? nbd : funcy;
+                if (nbd > funcy) set_err(a.flags, FM_EBOND, a.ext[slot]);
+            }
+        }
+        wave_sync();  // (the buffers are written again)
+    }
+    for (int off = 32; off > 0; off >>= 1) wmax = max(wmax, __shfl_xor(wmax, off, 64));
+    if (lane == 0 && wmax > a.maxnb) {
+        atomicMax(&a.flags[FLAG_MAX_NB], wmax);
+        atomicOr(&a.flags[FLAG_NEED], NEED_LIST);
+        a.flags[FLAG_HALT] = 1;
     }
 }
 
@@ -2702,6 +3118,18 @@ int launch_region_max(fm_ctx* c) {
     return 0;
 }
 
+// Wavefronts per workgroup of the tile list build: the most with which two workgroups share a CU's
+// LDS, or else that fit one; 0 when four do not fit (the FP64 build then runs)
+static int nlt_waves(const fm_ctx* c, const BG& g, bool poly, size_t* lds) {
+    const size_t fixed = nlt_fixed_bytes(g, c->maxreg, poly), wave = nlt_wave_bytes(c->maxnb, poly);
+    for (size_t room : {std::min(c->lds_cu / 2, c->lds_limit), c->lds_limit})
+        for (int nw = FB_BLOCK / 64; nw >= 4; --nw) {
+            *lds = fixed + std::max((size_t)nw * wave, (size_t)c->maxreg * 2 + 16);
+            if (*lds <= room) return nw;
+        }
+    return 0;
+}
+
 int launch_nlist(fm_ctx* c) {
     if (c->np == 0) return 0;
     BG g = make_bg(c);
@@ -2726,6 +3154,48 @@ int launch_nlist(fm_ctx* c) {
     for (int d = 0; d < 3; ++d) {
         a.cs[d] = c->cs[d];
         a.hd[d] = c->half[d];
+    }
+    size_t tile_lds = 0;
+    const int nw = a.xsorted && c->cap < (1 << 26) && c->btab ? nlt_waves(c, g, a.mono != nullptr, &tile_lds) : 0;
+    if (nw > 0 && c->tile_list) {
+        // matrix tiles (slots packed with the shift code in 31 bits)
+        NltArgs q;
+        q.wbytes = (int)nlt_wave_bytes(c->maxnb, a.mono != nullptr);
+        q.mono = a.mono;
+        q.bond = a.bond;
+        q.bondn = a.bondn;
+        q.ext = a.ext;
+        q.s = a.s;
+        q.g = g;
+        q.start = a.start;
+        q.nbl = a.nbl;
+        q.nbn = a.nbn;
+        q.flags = a.flags;
+        q.cap = a.cap;
+        q.maxnb = a.maxnb;
+        q.maxreg = a.maxreg;
+        q.ra2 = a.ra2;
+        q.order = a.order;
+        q.btab = c->btab;
+        q.btab_stride = c->btab_stride;
+        double h = 0.0;
+        for (int d = 0; d < 3; ++d) {
+            q.cs[d] = a.cs[d];
+            q.hd[d] = a.hd[d];
+            h = fmax(h, 0.5 * (g.B[d] + 2) * c->cs[d]);
+        }
+        // the window's margin: the roundings of the staged x and of the edges
+        q.hext = (float)(h * (1.0 + 1e-6));
+        q.rn = (float)(sqrt(a.ra2) * (1.0 + 1e-6));
+        q.xw = (float)(sqrt(a.ra2) * (1.0 + 1e-6) + 1e-6 * h);
+        const dim3 grid(brick_count(c)), blk(64 * nw);
+        ktimer_begin(c, KT_NLIST);
+        if (a.mono) k_nlist_tile<true><<<grid, blk, tile_lds, c->stream>>>(q);
+        else k_nlist_tile<false><<<grid, blk, tile_lds, c->stream>>>(q);
+        LAUNCH_CHECK();
+        ktimer_end(c, KT_NLIST);
+        c->btab_valid = true;
+        return 0;
     }
     if (a.xsorted && c->cap < (1 << 26)) {
         // quantised prefilter (slots packed with the shift code in 31 bits)

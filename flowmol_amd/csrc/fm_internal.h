@@ -86,6 +86,7 @@ struct fm_ctx {
     // LDS bricks
     int brick[3] = {1, 1, 1};
     int team = 1;                         // lanes per molecule of the force launches (team_of)
+    bool tile_list = false;               // the list build by matrix tiles (set with the brick)
     int* brick_order = nullptr;           // bricks in 4x4x4-tile order (XCD-aware workgroup mapping)
     int kt_step = 0;                      // step number attached to kernel timing records
 
