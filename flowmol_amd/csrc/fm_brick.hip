@@ -1671,7 +1671,8 @@ __device__ __forceinline__ void vv_pass2_pass1(const FbArgs& a, int i, double fx
 
 // FENE bonds (simulation_compute_forces_poly) and tethers (tether_force) of molecule i, added to
 // its force (fx, fy, fz already per unit mass); on record steps the bond energy and tallies too.
-template <bool RECORD, bool VIR>
+// (CV: the launch may tally control-volume stresses or rfmol)
+template <bool RECORD, bool VIR, bool CV = true>
 __device__ __forceinline__ void bond_tether_forces(const FbArgs& a, int i, double xi, double yi, double zi,
                                                    double inv_mi, bool do_rf, double* rf, double& fx, double& fy,
                                                    double& fz, double& vir) {
@@ -1698,7 +1699,7 @@ __device__ __forceinline__ void bond_tether_forces(const FbArgs& a, int i, doubl
             fz = fz + acc * rz * inv_mi;
             if (VIR) vir = vir + acc * r2;
             if (RECORD) {
-                if (a.cv) {
+                if (CV && a.cv) {
                     const double ri[3] = {xi, yi, zi}, rj[3] = {xj, yj, zj};
                     cv_entry(a, ri, rj, acc, a.ext[i]);
                 }
@@ -2211,8 +2212,8 @@ __device__ inline void mop_entry_fast(const FbArgs& a, const double ri[3], const
     }
 }
 
-// Record step of an LJ domain with the MOP tally and nothing else (no Mie tables, bonds, tethers
-// in the forces, CV faces or rfmol), in FP64 for both precisions (every pair term the tallies need
+// Record step of an LJ domain with the MOP tally and nothing else (no Mie tables, CV faces or
+// rfmol), in FP64 for both precisions (every pair term the tallies need
 // is an FP64 term, so the FP32 pair law would only add work).  One pass over the list: the forces,
 // PE and virial as the branch-free record loop computes them, and per entry the MOP test; the
 // entries inside rc that cross a plane and that this end tallies add their contribution, in FP64
@@ -2346,7 +2347,9 @@ __device__ __forceinline__ void lj_plain_mop(const FbArgs& a, const double* pos,
     vir_out = 24.0 * team_sum(vt, T);
 }
 
-template <bool SLOTS>
+// EXTRA: tethers (and bonds) in a pass of their own first, their force and virial parked in the launch's
+// output (what they read is then not held through the pair loop: 54 registers spilled otherwise)
+template <bool SLOTS, bool EXTRA>
 __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char* smem) {
     Region r;
     carve(r, smem, a.g, a.maxreg, true);
@@ -2368,6 +2371,20 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
         __syncthreads();
     }
     const size_t cap = a.cap;
+    if constexpr (EXTRA) {
+        for (int q = threadIdx.x; q < r.ni; q += blockDim.x) {
+            int li, i;
+            imol_tab(r, a.start, tab, a.maxreg, q, li, i);
+            double bx = 0.0, by = 0.0, bz = 0.0, vir = 0.0;
+            bond_tether_forces<true, true, false>(a, i, r.pos[3 * li], r.pos[3 * li + 1], r.pos[3 * li + 2], 1.0, false,
+                                                  nullptr, bx, by, bz, vir);
+            a.s.ax[i] = bx;
+            a.s.ay[i] = by;
+            a.s.az[i] = bz;
+            a.vir[i] = vir;
+        }
+        if (a.team > 1) __syncthreads();  // (the pair loop's team reads it in another thread)
+    }
     MopI m;
     m.hps = a.hp - a.shift;
     m.inv_sp = 1.0 / a.spacing;
@@ -2410,6 +2427,12 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
             }
         }
         if (tm.t != 0) continue;
+        if constexpr (EXTRA) {
+            fx = fx + a.s.ax[i];
+            fy = fy + a.s.ay[i];
+            fz = fz + a.s.az[i];
+            vir = vir + a.vir[i];
+        }
         a.s.ax[i] = fx;
         a.s.ay[i] = fy;
         a.s.az[i] = fz;
@@ -2745,12 +2768,19 @@ k_forces_brick_lj(FbArgs a) {
 
 // record steps with the MOP tally only (forces_body_mop): two workgroups per CU, as the LDS of
 // two regions allows
-template <bool SLOTS>
+template <bool SLOTS, bool EXTRA>
 __global__ __launch_bounds__(FB_BLOCK) __attribute__((amdgpu_waves_per_eu(FB_BLOCK / 128))) void
 k_forces_brick_mop(FbArgs a) {
     extern __shared__ __align__(16) char smem[];
     if (halted(a.halt, a.step)) return;
-    forces_body_mop<SLOTS>(a, brick_of_block(a.order, blockIdx.x, gridDim.x), smem);
+    forces_body_mop<SLOTS, EXTRA>(a, brick_of_block(a.order, blockIdx.x, gridDim.x), smem);
+}
+
+// a pair inside rc crosses at most three planes near molecule i when 2 rc < 3 spacings
+__host__ __device__ inline bool mop_slots(const FbArgs& a) { return 2.0 * sqrt(a.rc2) / a.spacing < 3.0 - 1e-6; }
+// a record step of an LJ domain whose only tally beyond PE and virial is MOP
+__host__ __device__ inline bool mop_record(const FbArgs& a) {
+    return a.rec && a.pxy != nullptr && a.cv == nullptr && a.rf == nullptr;
 }
 
 // LJ steps without tallies, bonds or tethers (the common step): registers held to what lets two
@@ -2840,6 +2870,22 @@ k_forces_brick_multi(const FbArgs* descs, const int2* table) {
     if (a.rec) forces_body<MIE, true, EXTRA>(a, t.y, smem);
     else if (a.ev) forces_body<MIE, false, EXTRA, true>(a, t.y, smem);
     else forces_body<MIE, false, EXTRA>(a, t.y, smem);
+}
+
+// FP64 LJ domains, each on a step without tallies or a record step of the one-pass MOP body: those two
+// bodies only, held to two workgroups per CU as the domain's own launches.  A packed record launch of
+// the general kernel above (one workgroup per CU, its per-entry branch loop) took 366 us for four
+// Couette domains of 241,000 molecules together, where a launch without tallies takes 30.
+template <bool EXTRA>
+__global__ __launch_bounds__(FB_BLOCK) __attribute__((amdgpu_waves_per_eu(FB_BLOCK / 128))) void
+k_forces_brick_multi_mop(const FbArgs* descs, const int2* table) {
+    extern __shared__ __align__(16) char smem[];
+    const int2 t = table[blockIdx.x];
+    const FbArgs& a = descs[t.x];
+    if (skip_domain(a)) return;
+    if (!a.rec) forces_body<false, false, EXTRA, false, false, true>(a, t.y, smem);
+    else if (mop_slots(a)) forces_body_mop<true, EXTRA>(a, t.y, smem);
+    else forces_body_mop<false, EXTRA>(a, t.y, smem);
 }
 
 // Mixed precision: image coordinates and differences in FP64, the pair law and the per-molecule
@@ -3277,10 +3323,11 @@ static float band32_of(const fm_ctx* c) {
     return (float)(4.0 * (e * (2.0 * sqrt(3.0) * rc + 3.0 * e) + 6.0 * u * c->rc2));
 }
 
-// a step without record or virial tallies
-bool fargs_plain(const void* fargs) {
+// the packed launch that a domain's step needs
+int fargs_pack(const void* fargs) {
     const FbArgs* a = (const FbArgs*)fargs;
-    return !a->rec && !a->ev;
+    if (!a->rec && !a->ev) return PACK_PLAIN;
+    return mop_record(*a) && !a->mie ? PACK_MOP : PACK_GENERAL;
 }
 
 // a domain's force arguments in a queued packed launch: halted by its own flag words, or idle
@@ -3438,11 +3485,13 @@ int launch_forces(fm_ctx* c, int iter, bool kick, bool cond, int next, bool* fus
     ktimer_begin(c, KT_FORCES);
     dim3 grid(brick_count(c)), blk(FB_BLOCK);
     // a record step whose only tally beyond PE and virial is MOP: the one-pass FP64 kernel (for
-    // both precisions)
-    if ((kind == 0 || kind == 1) && a.rec && a.pxy != nullptr && a.cv == nullptr && a.rf == nullptr) {
-        // a pair inside rc crosses at most three planes near molecule i when 2 rc < 3 spacings
-        if (2.0 * sqrt(a.rc2) / a.spacing < 3.0 - 1e-6) k_forces_brick_mop<true><<<grid, blk, lds, c->stream>>>(a);
-        else k_forces_brick_mop<false><<<grid, blk, lds, c->stream>>>(a);
+    // both precisions; with tethers or bonds in the forces for FP64 only)
+    if ((kind == 0 || kind == 1 || kind == 4) && mop_record(a)) {
+        if (extra) {
+            if (mop_slots(a)) k_forces_brick_mop<true, true><<<grid, blk, lds, c->stream>>>(a);
+            else k_forces_brick_mop<false, true><<<grid, blk, lds, c->stream>>>(a);
+        } else if (mop_slots(a)) k_forces_brick_mop<true, false><<<grid, blk, lds, c->stream>>>(a);
+        else k_forces_brick_mop<false, false><<<grid, blk, lds, c->stream>>>(a);
         ktimer_end(c, KT_FORCES);
         LAUNCH_CHECK();
         return 0;
@@ -3480,10 +3529,16 @@ int launch_forces(fm_ctx* c, int iter, bool kick, bool cond, int next, bool* fus
 }
 
 int launch_forces_multi(hipStream_t st, int kind, const void* d_descs, const int2* d_table, int nblk, size_t lds,
-                        bool plain) {
+                        int pack) {
     if (nblk == 0) return 0;
     const FbArgs* d = (const FbArgs*)d_descs;
-    const bool mixed = kind & 1, mie = kind & 2, extra = kind & 4;
+    const bool mixed = kind & 1, mie = kind & 2, extra = kind & 4, plain = pack == PACK_PLAIN;
+    if (pack == PACK_MOP && !mixed && !mie) {
+        if (extra) k_forces_brick_multi_mop<true><<<nblk, FB_BLOCK, lds, st>>>(d, d_table);
+        else k_forces_brick_multi_mop<false><<<nblk, FB_BLOCK, lds, st>>>(d, d_table);
+        LAUNCH_CHECK();
+        return 0;
+    }
 #define MULTI(K, ...) \
     (plain ? K<__VA_ARGS__, true><<<nblk, FB_BLOCK, lds, st>>>(d, d_table) \
            : K<__VA_ARGS__, false><<<nblk, FB_BLOCK, lds, st>>>(d, d_table))
