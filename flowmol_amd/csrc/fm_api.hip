@@ -1036,9 +1036,12 @@ static int size_regions(fm_ctx* c, int measured) {
         c->maxreg = m0;
         return size_brick_tables(c);
     }
-    const size_t wgs = std::max<size_t>(c->lds_cu / need, 1);
+    // (registers hold the brick kernels to three workgroups per CU: small regions take a third of the
+    // LDS, up to half as much again as measured, and seldom meet a larger region)
+    const size_t wgs = std::min<size_t>(std::max<size_t>(c->lds_cu / need, 1), 3);
     const size_t budget = std::min(c->lds_limit, (c->lds_cu / wgs) & ~(size_t)1023);
-    int lo = m0, hi = 65536;  // largest m in [m0, 65536] with region_bytes(m) <= budget
+    // largest m in [m0, 65536] with region_bytes(m) <= budget
+    int lo = m0, hi = wgs < 3 ? 65536 : std::min(65536, m0 + m0 / 2);
     while (lo < hi) {
         const int mid = lo + (hi - lo + 1) / 2;
         if (region_bytes(c, mid) <= budget) lo = mid;

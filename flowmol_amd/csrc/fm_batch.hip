@@ -423,6 +423,7 @@ extern "C" int fm_batch_run(fm_batch* b, int32_t nsteps, int32_t* n_rebuilds) {
                 // the window's list build met a region or list beyond the capacities: every launch
                 // of the member after it did nothing; build again, then the step's force
                 if (!rb0[k]) return fm_set_error(FM_ESTATE, "capacity request without a queued list build");
+                c->moved_since_bin = false;  // (no pass 1 after the binning ran)
                 TRY(redo_lists_internal(c));
                 TRY(launch_forces(c, it0[k], true));
                 done = 1;
