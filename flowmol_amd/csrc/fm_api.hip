@@ -171,6 +171,7 @@ static void free_ctx(fm_ctx* c) {
         delete c->timer;
     }
     if (c->stream) hipStreamDestroy(c->stream);
+    copy_pool_release();
     delete c;
 }
 
@@ -373,10 +374,12 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
         return fm_set_error(FM_EINVAL, "ntypes must be 1..%d", FM_MAX_TYPES);
 
     fm_ctx* c = new fm_ctx();
+    copy_pool_retain();
     c->p = *p;
     c->dev = -1;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
+        copy_pool_release();
         delete c;
         return fm_set_error(FM_EHIP, "no HIP device");
     }
@@ -700,10 +703,10 @@ extern "C" int fm_upload_state(fm_ctx* c, int32_t np, const double* r, const dou
     if (!r || !v) return fm_set_error(FM_EINVAL, "r and v are required");
     c->np = np;
     const size_t n3 = 3 * (size_t)np;
-    FM_HIP(hipMemcpyAsync(c->stage, r, n3 * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    FM_HIP(hipMemcpyAsync(c->stage + n3, v, n3 * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if (a) FM_HIP(hipMemcpyAsync(c->stage + 2 * n3, a, n3 * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    else TRY(launch_fill_f64(c, c->stage + 2 * n3, 0.0, n3));
+    const size_t b3 = n3 * sizeof(double);
+    const CopySeg seg[3] = {{(void*)r, c->stage, b3}, {(void*)v, c->stage + n3, b3}, {(void*)a, c->stage + 2 * n3, b3}};
+    TRY(copy_segments(c, seg, 3, false));
+    if (!a) TRY(launch_fill_f64(c, c->stage + 2 * n3, 0.0, n3));
     TRY(launch_from_host(c, c->stage));
     FM_HIP(hipStreamSynchronize(c->stream));
     c->cells_valid = c->nlist_valid = c->rdisp_valid = false;
@@ -785,9 +788,9 @@ extern "C" int fm_download_state(fm_ctx* c, double* r, double* v, double* a) {
     CHECK_CTX(c);
     const size_t n3 = 3 * (size_t)c->np;
     TRY(launch_scatter_state_to_host_order(c, c->stage, nullptr));
-    if (r) FM_HIP(hipMemcpyAsync(r, c->stage, n3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    if (v) FM_HIP(hipMemcpyAsync(v, c->stage + n3, n3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    if (a) FM_HIP(hipMemcpyAsync(a, c->stage + 2 * n3, n3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    const size_t b3 = n3 * sizeof(double);
+    const CopySeg seg[3] = {{r, c->stage, b3}, {v, c->stage + n3, b3}, {a, c->stage + 2 * n3, b3}};
+    TRY(copy_segments(c, seg, 3, true));
     FM_HIP(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -796,7 +799,8 @@ extern "C" int fm_download_tags(fm_ctx* c, double* rtether) {
     CHECK_CTX(c);
     if (!c->has_tags) return fm_set_error(FM_EINVAL, "no tags uploaded");
     TRY(launch_slot_to_ext_f64(c, c->stage, c->teth[c->cur], 3));
-    FM_HIP(hipMemcpyAsync(rtether, c->stage, 3 * (size_t)c->np * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    const CopySeg seg = {rtether, c->stage, 3 * (size_t)c->np * sizeof(double)};
+    TRY(copy_segments(c, &seg, 1, true));
     FM_HIP(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -893,7 +897,8 @@ extern "C" int fm_download_rfmol(fm_ctx* c, double* rfmol) {
     CHECK_CTX(c);
     if (!c->rf) return fm_set_error(FM_EINVAL, "rfmol needs pressure_outflag = 1");
     TRY(launch_slot_to_ext_f64(c, c->stage, c->rf, 9));
-    FM_HIP(hipMemcpyAsync(rfmol, c->stage, 9 * (size_t)c->np * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    const CopySeg seg = {rfmol, c->stage, 9 * (size_t)c->np * sizeof(double)};
+    TRY(copy_segments(c, &seg, 1, true));
     FM_HIP(hipStreamSynchronize(c->stream));
     return 0;
 }

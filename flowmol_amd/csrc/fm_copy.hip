@@ -1,0 +1,232 @@
+// fm_copy.hip -- large transfers between device staging and the caller's (pageable) host arrays.
+//
+// A copy to pageable memory runs at the speed of one host thread that also takes the page faults of
+// the caller's fresh arrays (72 MB, the state of 1,048,576 molecules: 8 ms).  Here the data passes
+// through pinned slots: the calling thread queues the device copies in order, and a few threads move
+// each slot to or from the caller's memory as it is ready (the same 72 MB: 3.7 ms, of which the link takes most).
+//
+// The pinned slots belong to a pool of the process: a transfer borrows a set and gives it back before it
+// returns, at most POOL_SETS exist, and the pool is freed with the last context.  A transfer that finds
+// no set, or no thread, is done by the plain copy.
+#include "fm_internal.h"
+
+#include <string.h>
+
+#include <algorithm>
+#include <atomic>
+#include <mutex>
+#include <exception>
+#include <new>
+#include <thread>
+#include <vector>
+
+#define SLOT_BYTES (2u << 20)
+#define NSLOTS 12
+#define POOL_SETS 4
+#define COPY_THREADS 6
+#define COPY_MIN (4u << 20)  // below this the threads cost more than they save
+
+namespace {
+
+struct SlotSet {
+    char* p = nullptr;           // NSLOTS x SLOT_BYTES, pinned
+    hipEvent_t ev[NSLOTS] = {};  // the device copy of each slot
+    int dev = -1;
+    bool busy = false;
+};
+
+std::mutex g_mu;
+SlotSet* g_sets[POOL_SETS] = {};
+int g_contexts = 0;
+
+void free_set(SlotSet* s) {
+    for (hipEvent_t e : s->ev)
+        if (e) hipEventDestroy(e);
+    if (s->p) hipHostFree(s->p);
+    delete s;
+}
+
+SlotSet* borrow(int dev) {
+    std::lock_guard<std::mutex> lock(g_mu);
+    SlotSet** room = nullptr;
+    for (SlotSet*& s : g_sets) {
+        if (!s) room = &s;
+        else if (!s->busy && s->dev == dev) {
+            s->busy = true;
+            return s;
+        }
+    }
+    if (!room) return nullptr;
+    SlotSet* s = new (std::nothrow) SlotSet();
+    if (!s) return nullptr;
+    s->dev = dev;
+    bool ok = hipHostMalloc((void**)&s->p, (size_t)NSLOTS * SLOT_BYTES, hipHostMallocDefault) == hipSuccess;
+    for (int k = 0; ok && k < NSLOTS; ++k) ok = hipEventCreateWithFlags(&s->ev[k], hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        free_set(s);
+        return nullptr;
+    }
+    s->busy = true;
+    *room = s;
+    return s;
+}
+
+void give_back(SlotSet* s) {
+    std::lock_guard<std::mutex> lock(g_mu);
+    s->busy = false;
+}
+
+struct Chunk {
+    char *host, *dev;
+    size_t n;
+};
+
+int plain_copy(fm_ctx* c, const CopySeg* seg, int nseg, bool to_host) {
+    for (int k = 0; k < nseg; ++k)
+        if (seg[k].host && seg[k].bytes) {
+            if (to_host) FM_HIP(hipMemcpyAsync(seg[k].host, seg[k].dev, seg[k].bytes, hipMemcpyDeviceToHost, c->stream));
+            else FM_HIP(hipMemcpyAsync(seg[k].dev, seg[k].host, seg[k].bytes, hipMemcpyHostToDevice, c->stream));
+        }
+    return 0;
+}
+
+// One transfer.  issued: chunks whose device copy is queued (their slot's event recorded); moved[i]:
+// chunk i's host side is done; failed: a HIP call failed, everyone stops.
+struct Transfer {
+    fm_ctx* c;
+    SlotSet* s;
+    std::vector<Chunk> ch;
+    bool to_host;
+    std::atomic<size_t> next{0}, issued{0};
+    std::vector<std::atomic<char>> moved;
+    std::atomic<int> failed{0};
+    explicit Transfer(size_t n) : moved(n) {
+        for (auto& m : moved) m.store(0, std::memory_order_relaxed);
+    }
+
+    bool until_issued(size_t n) {
+        while (issued.load(std::memory_order_acquire) < n) {
+            if (failed.load(std::memory_order_relaxed)) return false;
+            std::this_thread::yield();
+        }
+        return true;
+    }
+    bool until_moved(size_t i) {
+        while (!moved[i].load(std::memory_order_acquire)) {
+            if (failed.load(std::memory_order_relaxed)) return false;
+            std::this_thread::yield();
+        }
+        return true;
+    }
+    bool device_done(size_t slot) {
+        if (hipEventSynchronize(s->ev[slot]) == hipSuccess) return true;
+        failed.store(1);
+        return false;
+    }
+
+    // a worker: the host side of one chunk after another
+    void work() {
+        if (hipSetDevice(c->dev) != hipSuccess) {
+            failed.store(1);
+            return;
+        }
+        for (;;) {
+            const size_t i = next.fetch_add(1);
+            if (i >= ch.size()) return;
+            const size_t slot = i % NSLOTS;
+            char* pin = s->p + slot * SLOT_BYTES;
+            if (to_host) {
+                if (!until_issued(i + 1) || !device_done(slot)) return;
+                memcpy(ch[i].host, pin, ch[i].n);
+            } else {
+                // (the slot's copy of NSLOTS chunks ago has left it)
+                if (i >= NSLOTS && (!until_issued(i - NSLOTS + 1) || !device_done(slot))) return;
+                memcpy(pin, ch[i].host, ch[i].n);
+            }
+            moved[i].store(1, std::memory_order_release);
+        }
+    }
+
+    // the calling thread: the device side in order
+    bool issue() {
+        for (size_t i = 0; i < ch.size(); ++i) {
+            const size_t slot = i % NSLOTS;
+            char* pin = s->p + slot * SLOT_BYTES;
+            if (to_host ? (i >= NSLOTS && !until_moved(i - NSLOTS)) : !until_moved(i)) return false;
+            const hipError_t e = to_host
+                                     ? hipMemcpyAsync(pin, ch[i].dev, ch[i].n, hipMemcpyDeviceToHost, c->stream)
+                                     : hipMemcpyAsync(ch[i].dev, pin, ch[i].n, hipMemcpyHostToDevice, c->stream);
+            if (e != hipSuccess || hipEventRecord(s->ev[slot], c->stream) != hipSuccess) {
+                failed.store(1);
+                return false;
+            }
+            issued.store(i + 1, std::memory_order_release);
+        }
+        return true;
+    }
+};
+
+}  // namespace
+
+void copy_pool_retain() {
+    std::lock_guard<std::mutex> lock(g_mu);
+    ++g_contexts;
+}
+
+void copy_pool_release() {
+    std::lock_guard<std::mutex> lock(g_mu);
+    if (--g_contexts > 0) return;
+    for (SlotSet*& s : g_sets) {
+        if (s) free_set(s);
+        s = nullptr;
+    }
+}
+
+// Copies the segments between the device and the host, in stream order.  Host data is in place (to the
+// device: no longer needed) when it returns, unless the transfer is small: then after the stream's
+// next synchronisation, which every caller does.
+int copy_segments(fm_ctx* c, const CopySeg* seg, int nseg, bool to_host) {
+    size_t total = 0;
+    for (int k = 0; k < nseg; ++k) total += seg[k].host ? seg[k].bytes : 0;
+    if (total < COPY_MIN) return plain_copy(c, seg, nseg, to_host);
+    SlotSet* s = borrow(c->dev);
+    if (!s) return plain_copy(c, seg, nseg, to_host);
+    int rc = 0;
+    std::vector<std::thread> th;
+    try {
+        std::vector<Chunk> ch;
+        for (int k = 0; k < nseg; ++k)
+            for (size_t o = 0; seg[k].host && o < seg[k].bytes;) {
+                // (chunks end where the host's 2 MB pages do: no two threads take the fault of one page)
+                char* h = (char*)seg[k].host + o;
+                const size_t n = std::min<size_t>(SLOT_BYTES - ((uintptr_t)h & (SLOT_BYTES - 1)), seg[k].bytes - o);
+                ch.push_back({h, (char*)seg[k].dev + o, n});
+                o += n;
+            }
+        Transfer t(ch.size());
+        t.c = c;
+        t.s = s;
+        t.ch.swap(ch);
+        t.to_host = to_host;
+        const size_t want = std::min<size_t>(COPY_THREADS, t.ch.size() / 2);
+        th.reserve(want);
+        try {
+            while (th.size() < want) th.emplace_back([&t] { t.work(); });
+        } catch (const std::exception&) {  // fewer threads, or none
+        }
+        if (th.empty()) {
+            rc = plain_copy(c, seg, nseg, to_host);
+        } else {
+            const bool ok = t.issue();
+            for (auto& x : th) x.join();
+            // (a slot is lent again only after its last device copy)
+            const hipError_t e = hipStreamSynchronize(c->stream);
+            if (!ok || t.failed.load() || e != hipSuccess) rc = fm_set_error(FM_EHIP, "staged host copy failed: %s", hipGetErrorString(e));
+        }
+    } catch (const std::bad_alloc&) {  // (before any thread started)
+        rc = plain_copy(c, seg, nseg, to_host);
+    }
+    give_back(s);
+    return rc;
+}

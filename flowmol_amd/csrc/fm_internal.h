@@ -254,6 +254,16 @@ size_t brick_lds_bytes(const fm_ctx* c, int maxreg, int kind);  // kind 0 list b
 int launch_region_max(fm_ctx* c);
 int launch_decode_nlist(fm_ctx* c, uint32_t* out);
 
+// transfers between device staging and the caller's host arrays (fm_copy.hip)
+struct CopySeg {
+    void* host;   // null: skipped
+    void* dev;
+    size_t bytes;
+};
+int copy_segments(fm_ctx* c, const CopySeg* seg, int nseg, bool to_host);
+void copy_pool_retain();   // a context lives
+void copy_pool_release();  // one less: the last frees the pinned slots
+
 // stable radix sort of (key, value) pairs (fm_kernels.hip)
 size_t radix_sort_bytes(int n_items);
 int radix_sort_pairs(fm_ctx* c, int* k0, int* v0, int* k1, int* v1, int n, int end_bit, int** vals);

@@ -1,0 +1,55 @@
+"""Host transfers of any size: states below and above the size that passes through the pinned slots, with
+remainders of a slot, from several threads at once, come back as they went."""
+import sys
+import threading
+
+import numpy as np
+import pytest
+
+from flowmol_amd import config
+from flowmol_amd.md import MDContext
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def round_trip(n, seed, times, failed):
+    try:
+        rng = np.random.default_rng(seed)
+        p = config.make_params((60.0, 60.0, 60.0), n / 60.0 ** 3, 2.5)
+        g = None
+        for _ in range(times):
+            r, v, a = (rng.uniform(-29.0, 29.0, (n, 3)) for _ in range(3))
+            if g is None:
+                g = MDContext(p, r, v, a)
+            else:
+                g.upload_state(r, v, a)
+            for sent, got in zip((r, v, a), g.state()):
+                assert np.array_equal(sent, got)
+        g.close()
+    except Exception as e:  # noqa: BLE001 (reported by the caller)
+        failed.append(e)
+
+
+# 72 bytes a molecule: 4 MiB is 58,254 of them, a 2 MiB slot 87,381 vectors
+@pytest.mark.parametrize("n", [1, 58254, 58255, 87381, 87382, 300001])
+def test_round_trip(n):
+    say(f"case: {n} molecules up and down")
+    failed = []
+    round_trip(n, n, 2, failed)
+    assert not failed, failed
+
+
+def test_round_trips_from_seven_threads():
+    say("case: seven threads, a context each, 70,000 molecules")
+    failed = []
+    th = [threading.Thread(target=round_trip, args=(70000 + k, k, 3, failed)) for k in range(7)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not failed, failed
