@@ -622,6 +622,17 @@ __global__ __launch_bounds__(FB_BLOCK) void k_nlist_brick(NlbArgs a) {
 // and a candidate between the two is decided by the reference's FP64 test
 // (rij2 < rneighbr2, src/linklist.f90:717-720,750-754) on its positions in HBM.  The margins (1e-9 t^2)
 // cover the rounding of the FP64 test itself, so the set is the FP64 set exactly.
+//
+// A molecule's candidates are an x window of each of its nine runs, as whole x bins: the first
+// molecule of each bin of the rows of region cells (sixteen bins a cell) stands in an LDS table, built
+// once a brick, so a window costs one square root and two LDS reads.  The windows only leave out
+// molecules that cannot be pairs; the bins widen them by about a twentieth.
+// What bounds it: instruction issue (VALU busy nine tenths of the time).  Of a wavefront's 5,900
+// vector instructions at a million LJ molecules (477 a brick, 244 candidates and 76 entries each) about
+// 2,800 are the tests at 7 a candidate, 1,500 the entries at 11, 400 the windows.  Windows by two
+// binary searches and FP64 roots, tests by compare and select and store addresses by entry number took
+// 9,260.  Per build: 1,048,576 LJ molecules 266 -> 199 us, walls and slide (1,048,576)
+// 238 -> 183 us, cutoff 4 in bricks of one cell (55,296) 131 -> 98 us.
 typedef short s16x2 __attribute__((ext_vector_type(2)));
 
 struct NlqArgs {
@@ -632,8 +643,14 @@ struct NlqArgs {
     int* nbn;
     int* flags;
     int cap, maxnb, maxreg;
-    double ra2, xwin, h, inv_h;  // ra2, xwin, lo, hi: the radius of the pairs kept (as NlbArgs)
-    int lo, hi;
+    double ra2, h, inv_h;  // ra2: the radius of the pairs kept (as NlbArgs)
+    // quantised r^2 below lo is a pair, from hi on none: nhi = -hi, band = hi - lo, so that the signs
+    // of r^2 + nhi and of that + band are the two tests
+    int nhi, band;
+    // the x bins of the region's rows: 2^lb of them a cell, sb bins a unit of length, hb bins a grid
+    // step, slack bins added to each side of a window; ra2f: ra2 rounded up for the windows
+    int lb;
+    float sb, hb, slack, ra2f;
     double cs[3], hd[3];
     const int* order;
     // bond discovery (POLY): monomer fields in slot order, the bond lists, molecule numbers
@@ -647,8 +664,7 @@ struct NlqArgs {
 };
 
 __device__ inline int quantise(double x, double o, double inv_h) {
-    const int q = (int)floor((x - o) * inv_h + 0.5);
-    return min(max(q, 0), 32767);
+    return min(max((int)((x - o) * inv_h + 0.5), 0), 32767);  // (toward zero: below it is clamped)
 }
 
 // registers held to what lets three workgroups share a CU (its LDS region is a third of the
@@ -683,12 +699,16 @@ k_nlist_quant(NlqArgs a) {
     r.ic_off = ip;
     ip += g.B[0] * g.B[1] * g.B[2] + 1;
     r.ic_rc = ip;
+    ip += g.B[0] * g.B[1] * g.B[2];
+    uint16_t* const tab = (uint16_t*)ip;    // (nreg << lb) + 1: first molecule of each x bin
     const int brick = brick_of_block(a.order, blockIdx.x, gridDim.x);
     if (!stage_tables(r, g, brick, a.start, a.maxreg, a.flags)) return;
     const int bx = brick % g.nb[0], by = (brick / g.nb[0]) % g.nb[1], bz = brick / (g.nb[0] * g.nb[1]);
     const double ox = -a.hd[0] + (bx * g.B[0] - 1) * a.cs[0] - 2.0 * a.h;
     const double oy = -a.hd[1] + (by * g.B[1] - 1) * a.cs[1] - 2.0 * a.h;
     const double oz = -a.hd[2] + (bz * g.B[2] - 1) * a.cs[2] - 2.0 * a.h;
+    // first x bin of each region cell's row (the global cells have served)
+    for (int t = threadIdx.x; t < g.nreg; t += blockDim.x) r.gc[t] = (t / g.R[0] * g.R[0]) << a.lb;
     constexpr int SU = 6;  // molecules per thread and pass, loads first (as stage_region)
     for (int q0 = threadIdx.x; q0 < r.total; q0 += SU * blockDim.x) {
         int sl[SU], sc[SU];
@@ -703,15 +723,26 @@ k_nlist_quant(NlqArgs a) {
             py[k] = a.s.y[sl[k]];
             pz[k] = a.s.z[sl[k]];
         }
+        bool shifted = false;
+#pragma unroll
+        for (int k = 0; k < SU; ++k) shifted |= sc[k] != 13;
+        if (shifted) {  // (no molecule of a brick away from the domain's faces)
+#pragma unroll
+            for (int k = 0; k < SU; ++k) {
+                int sx, sy, sz;
+                decode_shift(sc[k], sx, sy, sz);
+                px[k] = img(px[k], sx, g.L[0]);
+                py[k] = img(py[k], sy, g.L[1]);
+                pz[k] = img(pz[k], sz, g.L[2]);
+            }
+        }
 #pragma unroll
         for (int k = 0; k < SU; ++k) {
             const int q = q0 + k * (int)blockDim.x;
             if (q >= r.total) break;
-            int sx, sy, sz;
-            decode_shift(sc[k], sx, sy, sz);
-            const int xq = quantise(img(px[k], sx, g.L[0]), ox, a.inv_h);
-            const int yq = quantise(img(py[k], sy, g.L[1]), oy, a.inv_h);
-            const int zq = quantise(img(pz[k], sz, g.L[2]), oz, a.inv_h);
+            const int xq = quantise(px[k], ox, a.inv_h);
+            const int yq = quantise(py[k], oy, a.inv_h);
+            const int zq = quantise(pz[k], oz, a.inv_h);
             // (POLY: z | low 17 bits of the chain id << 15)
             qv[q] = make_uint2((uint32_t)xq | ((uint32_t)yq << 16),
                                (uint32_t)zq | (POLY ? ((uint32_t)a.mono[sl[k]] & 0x1ffffu) << 15 : 0u));
@@ -724,9 +755,31 @@ k_nlist_quant(NlqArgs a) {
         a.btab[(size_t)brick * a.btab_stride + 1] = r.ni;
     }
     __syncthreads();
+    const int R0 = g.R[0], R1 = g.R[1], nbin = R0 << a.lb;
+    {
+        // The rows' x bins: bin e's entry is the first staged molecule of a bin >= e (rows and their
+        // molecules follow each other in the region layout).  A thread takes neighbouring molecules
+        // and writes, at each, the bins that begin there.
+        const int per = (r.total + (int)blockDim.x - 1) / (int)blockDim.x;
+        auto bin_of = [&](int q) {
+            const int b = (int)(((float)(qv[q].x & 0xffffu) - 2.0f) * a.hb);
+            return r.gc[r.rq[q]] + min(max(b, 0), nbin - 1);
+        };
+        const int qa = (int)threadIdx.x * per, qb = min(qa + per, r.total);
+        if (qa < qb) {
+            int e = qa ? bin_of(qa - 1) : -1;
+            for (int q = qa; q < qb; ++q)
+                for (const int eq = bin_of(q); e < eq;) tab[++e] = (uint16_t)q;
+            if (qb == r.total)
+                while (e < (g.nreg << a.lb)) tab[++e] = (uint16_t)qb;
+        } else if (r.total == 0) {
+            for (int e = threadIdx.x; e <= (g.nreg << a.lb); e += blockDim.x) tab[e] = 0;
+        }
+    }
+    __syncthreads();
     int wmax = 0;
     const size_t cap = a.cap;
-    const int R0 = g.R[0], R1 = g.R[1];
+    const int maxw = a.maxnb >> 2;
     const int nrounds = (r.ni + blockDim.x - 1) / blockDim.x;
     for (int round = 0; round < nrounds; ++round) {
         const int qi = round * blockDim.x + threadIdx.x;
@@ -790,8 +843,12 @@ k_nlist_quant(NlqArgs a) {
             const double ylo = -a.hd[1] + vy * a.cs[1], zlo = -a.hd[2] + vz * a.cs[2];
             const double gyl = fmax(yi - ylo - 1e-9, 0.0), gyh = fmax(ylo + a.cs[1] - yi - 1e-9, 0.0);
             const double gzl = fmax(zi - zlo - 1e-9, 0.0), gzh = fmax(zlo + a.cs[2] - zi - 1e-9, 0.0);
+            // (for the windows, in single precision: x in bins from the region's face)
+            const float fyl = (float)gyl, fyh = (float)gyh, fzl = (float)gzl, fzh = (float)gzh;
+            const float xb = (float)(xi - ox) * a.sb - 2.0f * a.hb;
+            const int bmin = (rx - 1) << a.lb, bmax = ((rx + 2) << a.lb) - 1;
             // nine runs of three x-consecutive region cells; each x window (of the radius of the
-            // pairs kept) widened by a grid step on both sides of its quantised bounds.  The runs
+            // pairs kept) is taken as whole bins of the rows' tables.  The runs
             // go nearest first: by the distance g^2 from the molecule to the run's y and z faces
             // (its top 28 bits), then by run number.  That order does not depend on the radius,
             // so a list of a smaller radius is the larger one's with the farther entries left out.
@@ -812,61 +869,51 @@ k_nlist_quant(NlqArgs a) {
                     w[k] = x < y ? x : y;
                     w[k + 1] = x < y ? y : x;
                 }
-            uint64_t word = 0;
+            // the last four entries (the first of them lowest), entries modulo 4 in the top two bits
+            // of c4, full words so far and where the next one goes
+            uint32_t wlo = 0, whi = 0, c4 = 0;
+            int nword = 0;
+            uint64_t* out = a.nbl + slot;
             for (int kk = 0; kk < 9; ++kk) {
                 const int k = (int)(w[kk] & 15u);
                 const int dz = k / 3 - 1, dy = k % 3 - 1;
-                const int c0 = (rx - 1) + R0 * ((ry + dy) + R1 * (rz + dz));
-                int jb = r.off[c0], je = r.off[c0 + 3];
-                const double gy = dy < 0 ? gyl : (dy > 0 ? gyh : 0.0);
-                const double gz = dz < 0 ? gzl : (dz > 0 ? gzh : 0.0);
-                const double w2 = a.ra2 - (gy * gy + gz * gz);
-                if (!(w2 > 0.0)) continue;
-                {
-                    const double xw = (dy == 0 && dz == 0) ? a.xwin : sqrt(w2) * (1.0 + 1e-9) + 1e-12;
-                    const int xl = (int)floor((xi - xw - ox) * a.inv_h) - 1;
-                    const int xh = (int)ceil((xi + xw - ox) * a.inv_h) + 1;
-                    int lo = jb, hi = je;
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if ((int)(qv[mid].x & 0xffffu) < xl) lo = mid + 1;
-                        else hi = mid;
-                    }
-                    jb = lo;
-                    hi = je;
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if ((int)(qv[mid].x & 0xffffu) <= xh) lo = mid + 1;
-                        else hi = mid;
-                    }
-                    je = lo;
-                }
+                const float gy = dy < 0 ? fyl : (dy > 0 ? fyh : 0.0f);
+                const float gz = dz < 0 ? fzl : (dz > 0 ? fzh : 0.0f);
+                const float w2 = a.ra2f - (gy * gy + gz * gz);
+                if (!(w2 > 0.0f)) continue;
+                const float xw = __builtin_amdgcn_sqrtf(w2) * a.sb + a.slack;
+                const int row = (R0 * ((ry + dy) + R1 * (rz + dz))) << a.lb;
+                const int jb = tab[row + min(max((int)(xb - xw), bmin), bmax)];
+                const int je = tab[row + min(max((int)(xb + xw), bmin), bmax) + 1];
                 for (int j0 = jb; j0 < je; j0 += 32) {
                     const int nn = min(32, je - j0);
                     // each test shifts its two bits in from the bottom (the first candidate ends
-                    // highest); one bit reversal afterwards puts candidate u at bit u
+                    // highest); one bit reversal afterwards puts candidate u at bit u.  Candidates go
+                    // by fours: those past the window's end read what follows in LDS, and their bits
+                    // are dropped
                     uint32_t m = 0, b = 0, sc = 0;
                     auto test = [&](int j) {
                         const uint2 wj = qv[j];
                         const s16x2 d1 = ixy - __builtin_bit_cast(s16x2, wj.x);
                         const int dz = izq - (int)(POLY ? wj.y & 0x7fffu : wj.y);
-                        const int r2q = __builtin_amdgcn_sdot2(d1, d1, __mul24(dz, dz), false);
-                        m = m + m + (uint32_t)(r2q < a.lo);
-                        b = b + b + (uint32_t)(r2q < a.hi);
+                        const int dq = __builtin_amdgcn_sdot2(d1, d1, __mul24(dz, dz) + a.nhi, false);
+                        m = __builtin_amdgcn_alignbit(m, (uint32_t)dq + (uint32_t)a.band, 31);
+                        b = __builtin_amdgcn_alignbit(b, (uint32_t)dq, 31);
                         if (POLY) sc = sc + sc + (uint32_t)((wj.y >> 15) == ich);
                     };
                     int u = 0;
-                    for (; u + 4 <= nn; u += 4) {
+                    do {
                         test(j0 + u);
                         test(j0 + u + 1);
                         test(j0 + u + 2);
                         test(j0 + u + 3);
-                    }
-                    for (; u < nn; ++u) test(j0 + u);
-                    m = __builtin_bitreverse32(m) >> (32 - nn);
-                    b = __builtin_bitreverse32(b) >> (32 - nn);
-                    if (POLY) sc = __builtin_bitreverse32(sc) >> (32 - nn);
-                    if (li >= j0 && li < j0 + nn) {
+                        u += 4;
+                    } while (u < nn);
+                    const uint32_t keep = 0xffffffffu >> (32 - nn);
+                    m = (__builtin_bitreverse32(m) >> (32 - u)) & keep;
+                    b = (__builtin_bitreverse32(b) >> (32 - u)) & keep;
+                    if (POLY) sc = (__builtin_bitreverse32(sc) >> (32 - u)) & keep;
+                    if (k == 4 && li >= j0 && li < j0 + nn) {
                         m &= ~(1u << (li - j0));
                         b &= ~(1u << (li - j0));
                     }
@@ -875,10 +922,15 @@ k_nlist_quant(NlqArgs a) {
                         const int u = __builtin_ctz(u8);
                         const int pk = ls[j0 + u];
                         const int sl = pk >> 5;
-                        int sx, sy, sz;
-                        decode_shift(pk & 31, sx, sy, sz);
-                        const double ddx = xi - img(a.s.x[sl], sx, g.L[0]), ddy = yi - img(a.s.y[sl], sy, g.L[1]),
-                                     ddz = zi - img(a.s.z[sl], sz, g.L[2]);
+                        double xj = a.s.x[sl], yj = a.s.y[sl], zj = a.s.z[sl];
+                        if ((pk & 31) != 13) {
+                            int sx, sy, sz;
+                            decode_shift(pk & 31, sx, sy, sz);
+                            xj = img(xj, sx, g.L[0]);
+                            yj = img(yj, sy, g.L[1]);
+                            zj = img(zj, sz, g.L[2]);
+                        }
+                        const double ddx = xi - xj, ddy = yi - yj, ddz = zi - zj;
                         const double r2 = (ddx * ddx + ddy * ddy) + ddz * ddz;
                         if (r2 < a.ra2) m |= 1u << u;
                     }
@@ -886,11 +938,15 @@ k_nlist_quant(NlqArgs a) {
                     // (POLY: the hits of the molecule's own chain, for the bond test below)
                     const uint32_t same = POLY ? m & sc : 0u;
                     while (m) {
-                        const int j = j0 + __builtin_ctz(m);
+                        const uint32_t j = (uint32_t)(j0 + __builtin_ctz(m));
                         m &= m - 1;
-                        word = (word >> 16) | ((uint64_t)(uint32_t)j << 48);
-                        if ((cnt & 3) == 3 && cnt < a.maxnb) a.nbl[(size_t)(cnt >> 2) * cap + slot] = word;
-                        ++cnt;
+                        wlo = __builtin_amdgcn_alignbit(whi, wlo, 16);
+                        whi = __builtin_amdgcn_alignbit(j, whi, 16);
+                        if (__builtin_uadd_overflow(c4, 0x40000000u, &c4)) {
+                            if (nword < maxw) *out = (uint64_t)whi << 32 | wlo;
+                            out += cap;
+                            ++nword;
+                        }
                     }
                     if (POLY) {
                         // hits of the molecule's own chain wait in registers (up to eight) for
@@ -905,7 +961,9 @@ k_nlist_quant(NlqArgs a) {
                     }
                 }
             }
-            if ((cnt & 3) != 0 && cnt < a.maxnb) a.nbl[(size_t)(cnt >> 2) * cap + slot] = word >> (16 * (4 - (cnt & 3)));
+            const int tail = (int)(c4 >> 30);
+            cnt = 4 * nword + tail;
+            if (tail != 0 && nword < maxw) *out = ((uint64_t)whi << 32 | wlo) >> (16 * (4 - tail));
             a.nbn[slot] = cnt < a.maxnb ? cnt : a.maxnb;
             if (POLY) {
                 flush_bonds();
@@ -957,7 +1015,7 @@ k_nlist_quant(NlqArgs a) {
 // What bounds it: the latency of one tile (windows, products, placing) where a wavefront has one or two,
 // the issue of about 1,700 instructions a tile where it has many; the products themselves are a
 // fiftieth of them.  A list build took, against k_nlist_quant, whose every lane scans its molecule's
-// windows alone: 25 -> 15 us (2,048 WCA molecules), 46 -> 19 us (5,148, bricks of 49), 54 -> 43 us
+// windows alone: 19 -> 14 us (2,048 WCA molecules), 35 -> 19 us (5,148, bricks of 49), 45 -> 43 us
 // (108,000, bricks of 222); but 73 -> 78 us at 500 molecules a brick, 265 -> 340 us at 1,048,576 (where
 // the scan keeps the vector units 93 % busy with as many instructions) and 131 -> 148 us at rc 4 (windows
 // of five blocks): bricks of at most 256 molecules (160 with bonds, 124 -> 100 us at 153 and 90 -> 95 us at
@@ -3260,7 +3318,6 @@ int launch_nlist(fm_ctx* c) {
         q.maxnb = a.maxnb;
         q.maxreg = a.maxreg;
         q.ra2 = a.ra2;
-        q.xwin = a.xwin;
         q.order = a.order;
         // the staging tables of the plain force launches, while the cells stay as binned
         q.btab = c->btab;
@@ -3276,11 +3333,26 @@ int launch_nlist(fm_ctx* c) {
         q.h = ext / 32700.0;
         q.inv_h = 1.0 / q.h;
         const double t = sqrt(a.ra2) / q.h, eps = 1.0 + 1e-6, r3 = sqrt(3.0);
-        q.lo = (int)floor(t * t - 2.0 * r3 * eps * t - 1e-9 * t * t) - 2;
-        q.hi = (int)ceil(t * t * (1.0 + 3e-9) + 2.0 * r3 * eps * t * (1.0 + 1e-9) + 3.0 * eps * eps) + 2;
+        const int lo = (int)floor(t * t - 2.0 * r3 * eps * t - 1e-9 * t * t) - 2;
+        const int hi = (int)ceil(t * t * (1.0 + 3e-9) + 2.0 * r3 * eps * t * (1.0 + 1e-9) + 3.0 * eps * eps) + 2;
+        q.nhi = -hi;
+        q.band = hi - lo;
         const int nbmax = g.B[0] * g.B[1] * g.B[2];
-        const size_t lds = (size_t)c->maxreg * (sizeof(uint2) + sizeof(int)) +
-                           (size_t)((c->maxreg + 1) / 2 + 4 * g.nreg + 1 + 2 * nbmax + 1) * sizeof(int);
+        const size_t lds0 = (size_t)c->maxreg * (sizeof(uint2) + sizeof(int)) +
+                            (size_t)((c->maxreg + 1) / 2 + 4 * g.nreg + 1 + 2 * nbmax + 1) * sizeof(int);
+        // sixteen x bins a cell (one to three molecules of a run each), fewer where they would take
+        // a workgroup from the CU
+        size_t lds = 0;
+        for (q.lb = 4; q.lb >= 0; --q.lb) {
+            lds = lds0 + ((((size_t)g.nreg << q.lb) + 1) * sizeof(uint16_t) + 7) / 8 * 8;
+            if (lds <= c->lds_limit && (q.lb == 0 || std::min(c->lds_cu / lds, (size_t)3) == std::min(c->lds_cu / lds0, (size_t)3)))
+                break;
+        }
+        q.lb = std::max(q.lb, 0);
+        q.sb = (float)((1 << q.lb) / c->cs[0]);
+        q.hb = (float)(q.h * (1 << q.lb) / c->cs[0]);
+        q.slack = (float)(2.5 * q.hb + 1e-3);
+        q.ra2f = (float)(a.ra2 * (1.0 + 1e-6));
         ktimer_begin(c, KT_NLIST);
         if (a.mono) k_nlist_quant<true><<<brick_count(c), FB_BLOCK, lds, c->stream>>>(q);
         else k_nlist_quant<false><<<brick_count(c), FB_BLOCK, lds, c->stream>>>(q);
