@@ -312,10 +312,10 @@ __device__ bool stage_region(Region& r, const BG& g, int brick, const int* start
 // slot and image shift of each staged molecule in the region layout (total and interior counts
 // first), then the slot and LDS index of each interior molecule.  No region tables are formed.
 // Ends with __syncthreads().
-// (type_src: the one-byte types of the staged molecules into r.ltype8 too; key_src: the owner keys
-// of the MOP tally, key_src[slot] << 1 | (image of a periodic shift), into r.lslot)
+// (type_src: the one-byte types of the staged molecules into r.ltype8 too; images: 1 for the image of
+// a periodic shift, 0 else, into r.lslot)
 __device__ bool stage_from_table(Region& r, const BG& g, const St& s, const int* T, int capm,
-                                 const int* type_src = nullptr, const int* key_src = nullptr) {
+                                 const int* type_src = nullptr, bool images = false) {
     r.total = T[0];
     r.ni = T[1];
     if (r.total > capm) return false;  // (a build that met a larger region halted its loop)
@@ -342,7 +342,7 @@ __device__ bool stage_from_table(Region& r, const BG& g, const St& s, const int*
             r.pos[3 * q + 1] = img(py[k], sy, g.L[1]);
             r.pos[3 * q + 2] = img(pz[k], sz, g.L[2]);
             if (type_src) r.ltype8[q] = (uint8_t)type_src[w[k] >> 5];
-            if (key_src) r.lslot[q] = (key_src[w[k] >> 5] << 1) | ((w[k] & 31) != 13 ? 1 : 0);
+            if (images) r.lslot[q] = (w[k] & 31) != 13 ? 1 : 0;
         }
     }
     __syncthreads();
@@ -2281,15 +2281,16 @@ __device__ inline void mop_entry_fast(const FbArgs& a, const double ri[3], const
 // half list) and every pair with a halo image from the molecule's side (so twice, once per end).
 // A pair's contribution is symmetric in its two ends (r_ij and the sign factor both change sign,
 // the crossed planes and the intercept are the same), so any rule that picks one end of each
-// unshifted pair tallies the same sum: the end with the higher molecule number.  Each staged
-// molecule's key is its molecule number << 1 | (its region cell is an image).
+// unshifted pair tallies the same sum: the end lower in y, which has only the planes above it to
+// look at.  Each staged molecule carries whether it is an image.
 struct P4K {
     double x[4], y[4], z[4];
     int k[4];
 };
+template <int NQ>
 __device__ __forceinline__ void lj_stage_k(P4K& p, const double* pos, const int* key, uint64_t w) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < NQ; ++q) {
         const int j = (int)((w >> (16 * q)) & 0xffffu);
         p.x[q] = pos[3 * j];
         p.y[q] = pos[3 * j + 1];
@@ -2301,27 +2302,33 @@ struct MopI {             // the i-molecule's side of the MOP test
     double ti;            // (y_i + halfdomain - shift) / planespacing
     double hps, inv_sp;   // halfdomain - shift, 1 / planespacing
     double bx, bz;        // the box's half widths in x and z, less 1e-12 relative
-    int keyi, nplanes;
+    int nplanes;
     bool in_i;            // molecule i strictly inside the box in x and z
     double* spxy;
     const double* planes;
-    // SLOTS: the (at most three) planes a pair of molecule i can cross, kb .. kb+2 (0-based plane
-    // numbers; a slot outside 0 .. nplanes-1 holds 1e300, where no pair crosses), their y, the
-    // sign of y_i against each, and the thread's sums of the contributions to each
-    int kb, sneg;          // sneg bit s: y_i lies below slot s's plane
-    double pl[3];
-    double c[3][3];
+    // NS: the (at most NS) planes above molecule i that a pair of it can cross, kb .. (0-based plane
+    // numbers; a slot below y_i or outside 0 .. nplanes-1 holds 1e300, where no pair crosses), their
+    // y, and the thread's sums of x^4 (2 x^3 - 1) r_ij over the entries that cross each
+    int kb;
+    double pl[2];
+    double c[2][3];
 };
-// SLOTS (when 2 rc < 3 planespacing, so a pair inside rc crosses at most three planes near
-// molecule i): the MOP tally without branches.  For each slot the reference's sign factor
-// sign(y_i - plane) - sign(y_j - plane) is zero unless the plane lies between the two molecules,
-// so every entry adds (acc r_ij) x (sign factor) to each slot's sums, with acc zero for an entry
-// beyond rc or not tallied from this end; the entries with a molecule near the box's x or z
-// faces (whose intercept factors need the reference's divisions) go through mop_entry_fast.
-template <bool SLOTS, int NQ = 4>
+// NS (2 when rc < 2 planespacing, so a pair inside rc crosses at most two planes above its lower end;
+// 0 for finer planes): the MOP tally without branches.  A slot's plane lies above y_i, so an entry
+// crosses it when y_j is not below it (the reference's sign factor is then -2, and 0 otherwise), and
+// adds its force term to the slot's sums, zero for an entry beyond rc; of an unshifted pair the upper
+// end finds nothing to add.  The entries with a molecule near the box's x or z faces (whose intercept
+// factors need the reference's divisions) and images below molecule i (whose own end is in another
+// place) go through mop_entry_fast.
+// What bounds it: instruction issue (four fifths of the time).  With three slots on both sides of the
+// molecule, the sign factors subtracted per slot and the owner found by molecule numbers a launch over
+// 1,048,576 molecules with 64 planes took 260 us; 233 us with two above.
+template <int NS, int NQ>
 __device__ __forceinline__ void lj_word_mop(const FbArgs& a, const P4K& p, int left, double xi, double yi,
                                             double zi, MopI& m, double& fx, double& fy, double& fz,
                                             double& pe, double& vt) {
+    double tq[NQ];
+    int slow = 0;  // bit q: entry q goes through mop_entry_fast
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const double rx = xi - p.x[q], ry = yi - p.y[q], rz = zi - p.z[q];
@@ -2332,45 +2339,53 @@ __device__ __forceinline__ void lj_word_mop(const FbArgs& a, const P4K& p, int l
         const double x2 = x * x;
         const double x3 = x * x2;
         const double x4 = x2 * x2;
-        const double t = x4 * fmaf64(2.0, x3, -1.0);
+        const double t = x4 * fmaf64(2.0, x3, -1.0);  // (zero for an entry beyond rc)
         fx = fmaf64(t, rx, fx);
         fy = fmaf64(t, ry, fy);
         fz = fmaf64(t, rz, fz);
         vt = fmaf64(t, r2, vt);
         const double e = 4.0 * (x3 * x3 - x3) - a.potshift;
         pe = pe + (in ? e : 0.0);
-        const int kj = p.k[q];
-        const bool own = ((m.keyi | kj) & 1) != 0 || (m.keyi >> 1) > (kj >> 1);
-        if constexpr (SLOTS) {
-            const bool ins = m.in_i && fabs(p.x[q]) < m.bx && fabs(p.z[q]) < m.bz;
-            // (t is zero for an entry beyond rc)
-            const double af = (own && ins) ? 24.0 * t : 0.0;
-            const double v[3] = {af * rx, af * ry, af * rz};
+        tq[q] = t;
+        // this end tallies it: an image, or molecule i the lower of the two
+        const bool up = yi < p.y[q];
+        bool own = in & ((p.k[q] != 0) | up);
+        if constexpr (NS > 0) {
+            const bool ins = m.in_i & (fabs(p.x[q]) < m.bx) & (fabs(p.z[q]) < m.bz);
 #pragma unroll
-            for (int s = 0; s < 3; ++s) {
-                const double f = (((m.sneg >> s) & 1) ? -1.0 : 1.0) - copysign(1.0, p.y[q] - m.pl[s]);
-#pragma unroll
-                for (int d = 0; d < 3; ++d) m.c[s][d] = fmaf64(v[d], f, m.c[s][d]);
+            for (int s = 0; s < NS; ++s) {
+                const double ts = ins & (p.y[q] >= m.pl[s]) ? t : 0.0;
+                m.c[s][0] = fmaf64(ts, rx, m.c[s][0]);
+                m.c[s][1] = fmaf64(ts, ry, m.c[s][1]);
+                m.c[s][2] = fmaf64(ts, rz, m.c[s][2]);
             }
-            if (!(in && own && !ins)) continue;
+            own = own & !(ins & up);
         }
-        // the whole numbers strictly between t_i and t_j, widened (see mop_entry_fast)
-        const double tj = (p.y[q] + m.hps) * m.inv_sp;
-        const int k0 = (int)ceil(fmin(m.ti, tj) - 1e-9), k1 = (int)floor(fmax(m.ti, tj) + 1e-9);
-        if (in && own && k0 <= k1 && k1 >= 0 && k0 < m.nplanes) {
-            // the pair law's magnitude 48 (x^7 - x^4/2) as the force sum takes it (within 1e-15)
-            const double acc = 24.0 * t;
-            const double ri[3] = {xi, yi, zi}, rj[3] = {p.x[q], p.y[q], p.z[q]}, rij[3] = {rx, ry, rz};
-            mop_entry_fast(a, ri, rj, rij, acc, m.spxy, m.planes, k0, k1,
-                           m.in_i && fabs(p.x[q]) < m.bx && fabs(p.z[q]) < m.bz);
+        slow |= (int)own << q;
+    }
+    if (slow != 0) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            if (!((slow >> q) & 1)) continue;
+            // the whole numbers strictly between t_i and t_j, widened (see mop_entry_fast)
+            const double tj = (p.y[q] + m.hps) * m.inv_sp;
+            const int k0 = (int)ceil(fmin(m.ti, tj) - 1e-9), k1 = (int)floor(fmax(m.ti, tj) + 1e-9);
+            if (k0 <= k1 && k1 >= 0 && k0 < m.nplanes) {
+                // the pair law's magnitude 48 (x^7 - x^4/2) as the force sum takes it (within 1e-15)
+                const double acc = 24.0 * tq[q];
+                const double ri[3] = {xi, yi, zi}, rj[3] = {p.x[q], p.y[q], p.z[q]};
+                const double rij[3] = {xi - p.x[q], yi - p.y[q], zi - p.z[q]};
+                mop_entry_fast(a, ri, rj, rij, acc, m.spxy, m.planes, k0, k1,
+                               m.in_i && fabs(p.x[q]) < m.bx && fabs(p.z[q]) < m.bz);
+            }
         }
     }
 }
 
 // The list loop with the MOP test per entry: one word at a time, the next word's index in flight.
-// With SLOTS the word's entries go one at a time (the nine plane sums hold registers that four
-// staged entries would need).
-template <bool SLOTS>
+// A word's entries go NQ at a time: two (233 us at 1,048,576 molecules; one at a time 239, and four
+// spill 18 registers), or one where bonds and tethers hold registers too.
+template <int NS, int NQ>
 __device__ __forceinline__ void lj_plain_mop(const FbArgs& a, const double* pos, const int* key,
                                              const uint64_t* row, int n, size_t cap, double xi, double yi,
                                              double zi, MopI& m, const Team& tm, double& fx, double& fy,
@@ -2381,21 +2396,11 @@ __device__ __forceinline__ void lj_plain_mop(const FbArgs& a, const double* pos,
     for (int kw = 4 * tm.t; kw < n; kw += 4 * T) {
         const uint64_t w = wn;
         if (kw + 4 * T < n) wn = row[(size_t)((kw >> 2) + T) * cap];
-        if constexpr (SLOTS) {
 #pragma unroll 1
-            for (int q = 0; q < 4; ++q) {
-                P4K p;
-                const int j = (int)((w >> (16 * q)) & 0xffffu);
-                p.x[0] = pos[3 * j];
-                p.y[0] = pos[3 * j + 1];
-                p.z[0] = pos[3 * j + 2];
-                p.k[0] = key[j];
-                lj_word_mop<true, 1>(a, p, n - kw - q, xi, yi, zi, m, sx, sy, sz, pe, vt);
-            }
-        } else {
+        for (int q = 0; q < 4; q += NQ) {
             P4K p;
-            lj_stage_k(p, pos, key, w);
-            lj_word_mop<SLOTS>(a, p, n - kw, xi, yi, zi, m, sx, sy, sz, pe, vt);
+            lj_stage_k<NQ>(p, pos, key, w >> (16 * q));
+            lj_word_mop<NS, NQ>(a, p, n - kw - q, xi, yi, zi, m, sx, sy, sz, pe, vt);
         }
     }
     fx = 24.0 * team_sum(sx, T);
@@ -2407,7 +2412,7 @@ __device__ __forceinline__ void lj_plain_mop(const FbArgs& a, const double* pos,
 
 // EXTRA: tethers (and bonds) in a pass of their own first, their force and virial parked in the launch's
 // output (what they read is then not held through the pair loop: 54 registers spilled otherwise)
-template <bool SLOTS, bool EXTRA>
+template <int NS, bool EXTRA>
 __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char* smem) {
     Region r;
     carve(r, smem, a.g, a.maxreg, true);
@@ -2416,16 +2421,14 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
     double* planes = spxy + 3 * a.nplanes;
     for (int t = threadIdx.x; t < a.nplanes; t += blockDim.x) planes[t] = a.planes[t];
     for (int t = threadIdx.x; t < 3 * a.nplanes; t += blockDim.x) spxy[t] = 0.0;
-    // staged from the list build's table when there is one, with the owner keys
+    // staged from the list build's table when there is one, with the image marks
     const int* tab = a.btab ? a.btab + (size_t)brick * a.btab_stride : nullptr;
     if (tab) {
-        if (!stage_from_table(r, a.g, a.s, tab, a.maxreg, nullptr, a.ext)) return;
+        if (!stage_from_table(r, a.g, a.s, tab, a.maxreg, nullptr, true)) return;
     } else {
-        if (!stage_region(r, a.g, brick, a.start, a.s, true, nullptr, a.cap, nullptr, nullptr, a.maxreg, a.flags,
-                          nullptr, a.ext))
+        if (!stage_region(r, a.g, brick, a.start, a.s, true, nullptr, a.cap, nullptr, nullptr, a.maxreg, a.flags))
             return;
-        // the staged molecule numbers become the owner keys
-        for (int t = threadIdx.x; t < r.total; t += blockDim.x) r.lslot[t] = (r.lslot[t] << 1) | (r.sh[r.rq[t]] != 13);
+        for (int t = threadIdx.x; t < r.total; t += blockDim.x) r.lslot[t] = r.sh[r.rq[t]] != 13;
         __syncthreads();
     }
     const size_t cap = a.cap;
@@ -2451,37 +2454,34 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
     m.nplanes = a.nplanes;
     m.spxy = spxy;
     m.planes = planes;
-    const double rct = sqrt(a.rc2) * m.inv_sp;  // rc in plane spacings
     const Team tm = team_lane(a.team);
     for (int q = tm.q0; q < r.ni; q += tm.dq) {
         int li, i;
         imol_tab(r, a.start, tab, a.maxreg, q, li, i);
         const double xi = r.pos[3 * li], yi = r.pos[3 * li + 1], zi = r.pos[3 * li + 2];
         m.ti = (yi + m.hps) * m.inv_sp;
-        m.keyi = r.lslot[li];
         m.in_i = fabs(xi) < m.bx && fabs(zi) < m.bz;
-        if constexpr (SLOTS) {
-            // the planes strictly within rc of y_i: t in (t_i - rc/spacing, t_i + rc/spacing)
-            m.kb = (int)floor(m.ti - rct - 1e-9) + 1;
-            m.sneg = 0;
+        if constexpr (NS > 0) {
+            // the planes above y_i, from the first whose t is not below t_i (either way within rounding)
+            m.kb = (int)floor(m.ti - 1e-9) + 1;
 #pragma unroll
-            for (int s = 0; s < 3; ++s) {
+            for (int s = 0; s < NS; ++s) {
                 const int k = m.kb + s;
-                m.pl[s] = (k >= 0 && k < a.nplanes) ? planes[k] : 1e300;
-                m.sneg |= (copysign(1.0, yi - m.pl[s]) < 0.0 ? 1 : 0) << s;
+                const double pl = k >= 0 && k < a.nplanes ? planes[k] : 1e300;
+                m.pl[s] = yi < pl ? pl : 1e300;
                 m.c[s][0] = m.c[s][1] = m.c[s][2] = 0.0;
             }
         }
         double fx, fy, fz, pe, vir;
-        lj_plain_mop<SLOTS>(a, r.pos, r.lslot, a.nbl + i, a.nbn[i], cap, xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
-        if constexpr (SLOTS) {
+        lj_plain_mop<NS, EXTRA ? 1 : 2>(a, r.pos, r.lslot, a.nbl + i, a.nbn[i], cap, xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
+        if constexpr (NS > 0) {
 #pragma unroll
-            for (int s = 0; s < 3; ++s) {
+            for (int s = 0; s < NS; ++s) {
                 const int k = m.kb + s;
                 if (k >= 0 && k < a.nplanes)
 #pragma unroll
                     for (int d = 0; d < 3; ++d)
-                        if (m.c[s][d] != 0.0) atomicAdd(&spxy[3 * k + d], m.c[s][d]);
+                        if (m.c[s][d] != 0.0) atomicAdd(&spxy[3 * k + d], -48.0 * m.c[s][d]);
             }
         }
         if (tm.t != 0) continue;
@@ -2826,16 +2826,16 @@ k_forces_brick_lj(FbArgs a) {
 
 // record steps with the MOP tally only (forces_body_mop): two workgroups per CU, as the LDS of
 // two regions allows
-template <bool SLOTS, bool EXTRA>
+template <int NS, bool EXTRA>
 __global__ __launch_bounds__(FB_BLOCK) __attribute__((amdgpu_waves_per_eu(FB_BLOCK / 128))) void
 k_forces_brick_mop(FbArgs a) {
     extern __shared__ __align__(16) char smem[];
     if (halted(a.halt, a.step)) return;
-    forces_body_mop<SLOTS, EXTRA>(a, brick_of_block(a.order, blockIdx.x, gridDim.x), smem);
+    forces_body_mop<NS, EXTRA>(a, brick_of_block(a.order, blockIdx.x, gridDim.x), smem);
 }
 
-// a pair inside rc crosses at most three planes near molecule i when 2 rc < 3 spacings
-__host__ __device__ inline bool mop_slots(const FbArgs& a) { return 2.0 * sqrt(a.rc2) / a.spacing < 3.0 - 1e-6; }
+// a pair inside rc crosses at most two planes above its lower end when rc < 2 spacings
+__host__ __device__ inline bool mop_slots(const FbArgs& a) { return sqrt(a.rc2) / a.spacing < 2.0 - 1e-6; }
 // a record step of an LJ domain whose only tally beyond PE and virial is MOP
 __host__ __device__ inline bool mop_record(const FbArgs& a) {
     return a.rec && a.pxy != nullptr && a.cv == nullptr && a.rf == nullptr;
@@ -2942,8 +2942,8 @@ k_forces_brick_multi_mop(const FbArgs* descs, const int2* table) {
     const FbArgs& a = descs[t.x];
     if (skip_domain(a)) return;
     if (!a.rec) forces_body<false, false, EXTRA, false, false, true>(a, t.y, smem);
-    else if (mop_slots(a)) forces_body_mop<true, EXTRA>(a, t.y, smem);
-    else forces_body_mop<false, EXTRA>(a, t.y, smem);
+    else if (mop_slots(a)) forces_body_mop<2, EXTRA>(a, t.y, smem);
+    else forces_body_mop<0, EXTRA>(a, t.y, smem);
 }
 
 // Mixed precision: image coordinates and differences in FP64, the pair law and the per-molecule
@@ -3560,10 +3560,10 @@ int launch_forces(fm_ctx* c, int iter, bool kick, bool cond, int next, bool* fus
     // both precisions; with tethers or bonds in the forces for FP64 only)
     if ((kind == 0 || kind == 1 || kind == 4) && mop_record(a)) {
         if (extra) {
-            if (mop_slots(a)) k_forces_brick_mop<true, true><<<grid, blk, lds, c->stream>>>(a);
-            else k_forces_brick_mop<false, true><<<grid, blk, lds, c->stream>>>(a);
-        } else if (mop_slots(a)) k_forces_brick_mop<true, false><<<grid, blk, lds, c->stream>>>(a);
-        else k_forces_brick_mop<false, false><<<grid, blk, lds, c->stream>>>(a);
+            if (mop_slots(a)) k_forces_brick_mop<2, true><<<grid, blk, lds, c->stream>>>(a);
+            else k_forces_brick_mop<0, true><<<grid, blk, lds, c->stream>>>(a);
+        } else if (mop_slots(a)) k_forces_brick_mop<2, false><<<grid, blk, lds, c->stream>>>(a);
+        else k_forces_brick_mop<0, false><<<grid, blk, lds, c->stream>>>(a);
         ktimer_end(c, KT_FORCES);
         LAUNCH_CHECK();
         return 0;
