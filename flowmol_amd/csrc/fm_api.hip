@@ -179,7 +179,8 @@ static int alloc_nlist(fm_ctx* c, int maxnb) {
     if (c->nbl) hipFree(c->nbl);
     c->nbl = nullptr;
     c->maxnb = (maxnb + 3) & ~3;
-    return dalloc(&c->nbl, (size_t)(c->maxnb / 4) * c->cap);
+    // (whole groups of a team's rows: ListRow)
+    return dalloc(&c->nbl, (size_t)((c->maxnb / 4 + c->team - 1) / c->team * c->team) * c->cap);
 }
 
 // a build met a list of `need` entries: room for a quarter more

@@ -333,14 +333,25 @@ __device__ bool stage_from_table(Region& r, const BG& g, const St& s, const int*
             py[k] = s.y[sl];
             pz[k] = s.z[sl];
         }
+        bool shifted = false;
+#pragma unroll
+        for (int k = 0; k < SU; ++k) shifted |= (w[k] & 31) != 13;
+        if (shifted) {  // (no molecule of a brick away from the domain's faces)
+#pragma unroll
+            for (int k = 0; k < SU; ++k) {
+                int sx, sy, sz;
+                decode_shift(w[k] & 31, sx, sy, sz);
+                px[k] = img(px[k], sx, g.L[0]);
+                py[k] = img(py[k], sy, g.L[1]);
+                pz[k] = img(pz[k], sz, g.L[2]);
+            }
+        }
 #pragma unroll
         for (int k = 0; k < SU; ++k) {
             const int q = min(q0 + k * (int)blockDim.x, r.total - 1);
-            int sx, sy, sz;
-            decode_shift(w[k] & 31, sx, sy, sz);
-            r.pos[3 * q] = img(px[k], sx, g.L[0]);
-            r.pos[3 * q + 1] = img(py[k], sy, g.L[1]);
-            r.pos[3 * q + 2] = img(pz[k], sz, g.L[2]);
+            r.pos[3 * q] = px[k];
+            r.pos[3 * q + 1] = py[k];
+            r.pos[3 * q + 2] = pz[k];
             if (type_src) r.ltype8[q] = (uint8_t)type_src[w[k] >> 5];
             if (images) r.lslot[q] = (w[k] & 31) != 13 ? 1 : 0;
         }
@@ -1425,6 +1436,7 @@ struct FbArgs {
     const double* planes;
     int* flags;
     int cap, maxreg;
+    int maxw;              // words a molecule's list has room for
     int team;              // lanes that share a molecule's list (a power of two up to 16; team_of)
     int rec, ev;
     int kick;              // fused simulation_move_particles_vv(2): v += (0.5*dt)*a
@@ -1629,42 +1641,70 @@ __device__ __forceinline__ V team_sum(V v, int T) {
     return v;
 }
 
+// A lane's list words: word k is in row t + k T of the list (T lanes a molecule, t the lane's).  k is
+// the same for the whole wavefront, so a row's address is scalar arithmetic and the lane's part of it
+// one register, held from the start.  A lane past its own end reads the row as it is (the word is not
+// used); k is held within the rows that the list has (alloc_nlist allocates whole groups of T).
+// With a 64-bit multiply, an addition and a minimum a load, the image shifts of staging worked out
+// for every molecule and the state read between the stores of the step's end a force launch took 481 us
+// at 4,194,304 LJ molecules, 43.0 at 131,072 beads, 22.1 at 108,000 LJ; now 460, 41.2, 21.2.  The
+// longest list of the wavefront as k's limit saves the rows past it and costs as much in shuffles.
+__device__ __forceinline__ size_t wave_uniform(size_t v) {
+    return (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) |
+           (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32;
+}
+struct ListRow {
+    typedef const __attribute__((address_space(1))) char* Global;  // (the empty asm below hides it)
+    Global nbl;
+    size_t step;    // bytes of T rows
+    uint32_t off;   // of the lane's first word
+    int last;       // last group of T rows
+    __device__ __forceinline__ ListRow(const FbArgs& a, int i, const Team& tm)
+        : nbl((Global)wave_uniform((size_t)a.nbl)), step(wave_uniform((size_t)a.cap * tm.T * sizeof(uint64_t))),
+          off((uint32_t)((tm.t * a.cap + i) * sizeof(uint64_t))),
+          last(__builtin_amdgcn_readfirstlane((a.maxw + tm.T - 1) / tm.T - 1)) {}
+    __device__ __forceinline__ uint64_t operator[](int k) const {
+        Global p = nbl + (size_t)min(k, last) * step;
+        asm("" : "+s"(p));  // (the row's address stays scalar)
+        return *(const __attribute__((address_space(1))) uint64_t*)(p + off);
+    }
+};
+
 // REC: also the molecule's PE and virial (lj_word_rec).
 template <bool REC = false>
-__device__ __forceinline__ void lj_plain(const double* pos, const uint64_t* row, int n, size_t cap, double xi,
+__device__ __forceinline__ void lj_plain(const double* pos, const ListRow& row, int n, double xi,
                                          double yi, double zi, double rc2, const Team& tm, double& fx, double& fy,
                                          double& fz, double potshift = 0.0, double* pe_out = nullptr,
                                          double* vir_out = nullptr) {
     double sx = 0, sy = 0, sz = 0;
     double pe = 0.0, vt = 0.0;
     P4 pa, pb;
-    // At the top of each pass pa holds the positions of word k = kw/4, w1 is the lane's next word and
-    // w2 the one after (in flight).  Word loads past the end re-read the last word (the row always has
-    // at least one word), so no load sits behind a branch and each wait is for the oldest load;
-    // a pass always evaluates both words (the second one masked off past the end) so that the
-    // loop body is one block and the loads stay ahead of their uses.
-    const int lastw = n > 0 ? (n - 1) >> 2 : 0, T = tm.T, T4 = 4 * T;
-    uint64_t w0 = row[(size_t)min(tm.t, lastw) * cap];
-    lj_stage(pa, pos, 4 * tm.t < n ? w0 : 0);
-    uint64_t w1 = row[(size_t)min(tm.t + T, lastw) * cap];
-    uint64_t w2 = row[(size_t)min(tm.t + 2 * T, lastw) * cap];
-    for (int kw = 4 * tm.t; kw < n; kw += 2 * T4) {
-        const int k = kw >> 2;
-        lj_stage(pb, pos, kw + T4 < n ? w1 : 0);
+    // At the top of each pass pa holds the positions of the lane's word k, w1 is its next word and w2
+    // the one after (in flight); `left` counts its entries from word k on.  No load sits behind a
+    // branch, so each wait is for the oldest load; a pass always evaluates both words (the second one
+    // masked off past the end) so that the loop body is one block and the loads stay ahead of their uses.
+    const int T = tm.T, T4 = 4 * T;
+    int left = n - 4 * tm.t;
+    const uint64_t w0 = row[0];
+    lj_stage(pa, pos, left > 0 ? w0 : 0);
+    uint64_t w1 = row[1];
+    uint64_t w2 = row[2];
+    for (int k = 0; left > 0; k += 2, left -= 2 * T4) {
+        lj_stage(pb, pos, left > T4 ? w1 : 0);
         // both words two ahead are loaded here, at the top of the pass: the wait the compiler
         // places at the loop head is then for loads a whole pass old
         const uint64_t wk2 = w2;
-        w1 = row[(size_t)min(k + 3 * T, lastw) * cap];
-        w2 = row[(size_t)min(k + T4, lastw) * cap];
+        w1 = row[k + 3];
+        w2 = row[k + 4];
         __builtin_amdgcn_sched_barrier(0);  // keep the reads above the evaluation
-        if constexpr (REC) lj_word_rec(pa, n - kw, xi, yi, zi, rc2, potshift, sx, sy, sz, pe, vt);
-        else lj_word(pa, n - kw, xi, yi, zi, rc2, sx, sy, sz);
-        lj_stage(pa, pos, kw + 2 * T4 < n ? wk2 : 0);
+        if constexpr (REC) lj_word_rec(pa, left, xi, yi, zi, rc2, potshift, sx, sy, sz, pe, vt);
+        else lj_word(pa, left, xi, yi, zi, rc2, sx, sy, sz);
+        lj_stage(pa, pos, left > 2 * T4 ? wk2 : 0);
         __builtin_amdgcn_sched_barrier(0);
         // the second word only when a lane of the wavefront has entries in it
-        if (__builtin_amdgcn_ballot_w64(kw + T4 < n) != 0ull) {
-            if constexpr (REC) lj_word_rec(pb, n - kw - T4, xi, yi, zi, rc2, potshift, sx, sy, sz, pe, vt);
-            else lj_word(pb, n - kw - T4, xi, yi, zi, rc2, sx, sy, sz);
+        if (__builtin_amdgcn_ballot_w64(left > T4) != 0ull) {
+            if constexpr (REC) lj_word_rec(pb, left - T4, xi, yi, zi, rc2, potshift, sx, sy, sz, pe, vt);
+            else lj_word(pb, left - T4, xi, yi, zi, rc2, sx, sy, sz);
         }
     }
     fx = 24.0 * team_sum(sx, T);
@@ -1687,17 +1727,43 @@ __device__ __forceinline__ const FbArgs& fargs_again() {
     return *(const FbArgs*)kp;
 }
 
+// The force of molecule i, and the kick of a fused simulation_move_particles_vv(2) (its reads before
+// the first store, as below)
+__device__ __forceinline__ void store_force(const FbArgs& a, int i, double fx, double fy, double fz) {
+    double vx, vy, vz;
+    if (a.kick) {
+        vx = a.s.vx[i];
+        vy = a.s.vy[i];
+        vz = a.s.vz[i];
+    }
+    a.s.ax[i] = fx;
+    a.s.ay[i] = fy;
+    a.s.az[i] = fz;
+    if (a.kick) {
+        a.s.vx[i] = vx + a.hdt * fx;
+        a.s.vy[i] = vy + a.hdt * fy;
+        a.s.vz[i] = vz + a.hdt * fz;
+    }
+}
+
 // simulation_move_particles_vv(2) of this step, then (1) of the next step and the rdisp update of
 // rebuild criterion 2 (the arithmetic of k_pass2 and k_pass1_disp), the state after them written
 // to s2; the first lane of the wavefront that sees a displacement beyond the threshold raises the
 // rebuild flag with the next step's number.  KEEP_V (record steps): v at the end of this step stays
 // in s for the record-step sums (no other thread of the launch reads this molecule's velocity).
+// x, y, z: the molecule's stored position (its staged one: interior cells carry no image shift).
 template <bool KEEP_V>
-__device__ __forceinline__ void vv_pass2_pass1(const FbArgs& a, int i, double fx, double fy, double fz) {
-    const double ux = a.s.vx[i] + a.hdt * fx, uy = a.s.vy[i] + a.hdt * fy, uz = a.s.vz[i] + a.hdt * fz;
-    a.s2.x[i] = a.s.x[i] + a.dt * ux + a.hdt2 * fx;
-    a.s2.y[i] = a.s.y[i] + a.dt * uy + a.hdt2 * fy;
-    a.s2.z[i] = a.s.z[i] + a.dt * uz + a.hdt2 * fz;
+__device__ __forceinline__ void vv_pass2_pass1(const FbArgs& a, int i, double x, double y, double z, double fx,
+                                               double fy, double fz) {
+    // everything is read before the first store: a read after one that may be of the same memory
+    // would wait for its own round trip
+    const size_t cp = a.cap;
+    const double vx = a.s.vx[i], vy = a.s.vy[i], vz = a.s.vz[i];
+    double d0 = a.fresh ? 0.0 : a.rd[i], d1 = a.fresh ? 0.0 : a.rd[i + cp], d2 = a.fresh ? 0.0 : a.rd[i + 2 * cp];
+    const double ux = vx + a.hdt * fx, uy = vy + a.hdt * fy, uz = vz + a.hdt * fz;
+    a.s2.x[i] = x + a.dt * ux + a.hdt2 * fx;
+    a.s2.y[i] = y + a.dt * uy + a.hdt2 * fy;
+    a.s2.z[i] = z + a.dt * uz + a.hdt2 * fz;
     const double wx = ux + a.hdt * fx, wy = uy + a.hdt * fy, wz = uz + a.hdt * fz;
     a.s2.vx[i] = wx;
     a.s2.vy[i] = wy;
@@ -1705,8 +1771,6 @@ __device__ __forceinline__ void vv_pass2_pass1(const FbArgs& a, int i, double fx
     a.s2.ax[i] = fx;
     a.s2.ay[i] = fy;
     a.s2.az[i] = fz;
-    const size_t cp = a.cap;
-    double d0 = a.fresh ? 0.0 : a.rd[i], d1 = a.fresh ? 0.0 : a.rd[i + cp], d2 = a.fresh ? 0.0 : a.rd[i + 2 * cp];
     d0 = d0 + wx * a.dt;
     d1 = d1 + wy * a.dt;
     d2 = d2 + wz * a.dt;
@@ -1852,11 +1916,11 @@ __device__ __forceinline__ void forces_body(const FbArgs& a, int brick, char* sm
         const uint64_t* row = a.nbl + i;
         bool looped = false;  // the pairs went through the branch-free loop
         if constexpr (!MIE && !RECORD && !VIR) {
-            lj_plain(r.pos, row, n, cap, xi, yi, zi, a.rc2, tm, fx, fy, fz);
+            lj_plain(r.pos, ListRow(a, i, tm), n, xi, yi, zi, a.rc2, tm, fx, fy, fz);
             looped = true;
         } else if constexpr (!MIE && RECORD && VIR && !EXTRA) {
             if (simple_rec) {  // PE and virial only
-                lj_plain<true>(r.pos, row, n, cap, xi, yi, zi, a.rc2, tm, fx, fy, fz, a.potshift, &pe, &vir);
+                lj_plain<true>(r.pos, ListRow(a, i, tm), n, xi, yi, zi, a.rc2, tm, fx, fy, fz, a.potshift, &pe, &vir);
                 looped = true;
             }
         }
@@ -1945,19 +2009,12 @@ __device__ __forceinline__ void forces_body(const FbArgs& a, int brick, char* sm
         if constexpr (EXTRA) bond_tether_forces<RECORD, VIR>(a, i, xi, yi, zi, inv_mi, do_rf, rf, fx, fy, fz, vir);
         if constexpr (P1) {  // (k_forces_brick_plain only: its one argument is the FbArgs)
             const FbArgs& b = fargs_again();
-            vv_pass2_pass1<RECORD>(b, i, fx, fy, fz);
+            vv_pass2_pass1<RECORD>(b, i, xi, yi, zi, fx, fy, fz);
             if (VIR) b.vir[i] = vir;
             if (RECORD) b.pe_lj[i] = pe;
             continue;
         }
-        a.s.ax[i] = fx;
-        a.s.ay[i] = fy;
-        a.s.az[i] = fz;
-        if (a.kick) {
-            a.s.vx[i] = a.s.vx[i] + a.hdt * fx;
-            a.s.vy[i] = a.s.vy[i] + a.hdt * fy;
-            a.s.vz[i] = a.s.vz[i] + a.hdt * fz;
-        }
+        store_force(a, i, fx, fy, fz);
         if (VIR) a.vir[i] = vir;
         if (RECORD) {
             a.pe_lj[i] = pe;
@@ -2102,29 +2159,29 @@ __device__ __forceinline__ void mie_word(const P4M& p, int left, double xi, doub
 
 // The list loop of lj_plain (two words in flight, the word after them loading) over mie_word.
 template <int NT, int NB, bool REC>
-__device__ __forceinline__ void mie_plain(const double* pos, const uint8_t* lt, const uint64_t* row, int n,
-                                          size_t cap, double xi, double yi, double zi, const MieRow<NT, REC>& m,
+__device__ __forceinline__ void mie_plain(const double* pos, const uint8_t* lt, const ListRow& row, int n,
+                                          double xi, double yi, double zi, const MieRow<NT, REC>& m,
                                           const Team& tm, double& fx, double& fy, double& fz, double& pe,
                                           double& vt) {
     double sx = 0, sy = 0, sz = 0, spe = 0, svt = 0;
     P4M pa, pb;
-    const int lastw = n > 0 ? (n - 1) >> 2 : 0, T = tm.T, T4 = 4 * T;
-    const uint64_t w0 = row[(size_t)min(tm.t, lastw) * cap];
-    mie_stage(pa, pos, lt, 4 * tm.t < n ? w0 : 0);
-    uint64_t w1 = row[(size_t)min(tm.t + T, lastw) * cap];
-    uint64_t w2 = row[(size_t)min(tm.t + 2 * T, lastw) * cap];
-    for (int kw = 4 * tm.t; kw < n; kw += 2 * T4) {
-        const int k = kw >> 2;
-        mie_stage(pb, pos, lt, kw + T4 < n ? w1 : 0);
+    const int T = tm.T, T4 = 4 * T;
+    int left = n - 4 * tm.t;
+    const uint64_t w0 = row[0];
+    mie_stage(pa, pos, lt, left > 0 ? w0 : 0);
+    uint64_t w1 = row[1];
+    uint64_t w2 = row[2];
+    for (int k = 0; left > 0; k += 2, left -= 2 * T4) {
+        mie_stage(pb, pos, lt, left > T4 ? w1 : 0);
         const uint64_t wk2 = w2;
-        w1 = row[(size_t)min(k + 3 * T, lastw) * cap];
-        w2 = row[(size_t)min(k + T4, lastw) * cap];
+        w1 = row[k + 3];
+        w2 = row[k + 4];
         __builtin_amdgcn_sched_barrier(0);
-        mie_word<NT, NB, REC>(pa, n - kw, xi, yi, zi, m, sx, sy, sz, spe, svt);
-        mie_stage(pa, pos, lt, kw + 2 * T4 < n ? wk2 : 0);
+        mie_word<NT, NB, REC>(pa, left, xi, yi, zi, m, sx, sy, sz, spe, svt);
+        mie_stage(pa, pos, lt, left > 2 * T4 ? wk2 : 0);
         __builtin_amdgcn_sched_barrier(0);
-        if (__builtin_amdgcn_ballot_w64(kw + T4 < n) != 0ull)
-            mie_word<NT, NB, REC>(pb, n - kw - T4, xi, yi, zi, m, sx, sy, sz, spe, svt);
+        if (__builtin_amdgcn_ballot_w64(left > T4) != 0ull)
+            mie_word<NT, NB, REC>(pb, left - T4, xi, yi, zi, m, sx, sy, sz, spe, svt);
     }
     fx = team_sum(sx, T);
     fy = team_sum(sy, T);
@@ -2211,7 +2268,7 @@ __device__ __forceinline__ void forces_body_mie(const FbArgs& a, int brick, char
         mie_row<NT, NB, REC>(a, ti, m);
         const double inv_mi = 1.0 / a.mie[7 * T2 + ti];
         double fx, fy, fz, pe, vir;
-        mie_plain<NT, NB, REC>(r.pos, r.ltype8, a.nbl + i, a.nbn[i], a.cap, xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
+        mie_plain<NT, NB, REC>(r.pos, r.ltype8, ListRow(a, i, tm), a.nbn[i], xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
         if (tm.t != 0) continue;
         const FbArgs& b = KA ? fargs_again() : a;  // the arguments below: not held through the pair loop
         fx = fx * inv_mi;
@@ -2228,17 +2285,10 @@ __device__ __forceinline__ void forces_body_mie(const FbArgs& a, int brick, char
             b.pe_lj[i] = pe;
         }
         if constexpr (P1) {
-            vv_pass2_pass1<REC>(b, i, fx, fy, fz);
+            vv_pass2_pass1<REC>(b, i, xi, yi, zi, fx, fy, fz);
             continue;
         }
-        b.s.ax[i] = fx;
-        b.s.ay[i] = fy;
-        b.s.az[i] = fz;
-        if (b.kick) {
-            b.s.vx[i] = b.s.vx[i] + b.hdt * fx;
-            b.s.vy[i] = b.s.vy[i] + b.hdt * fy;
-            b.s.vz[i] = b.s.vz[i] + b.hdt * fz;
-        }
+        store_force(b, i, fx, fy, fz);
     }
 }
 
@@ -2387,20 +2437,21 @@ __device__ __forceinline__ void lj_word_mop(const FbArgs& a, const P4K& p, int l
 // spill 18 registers), or one where bonds and tethers hold registers too.
 template <int NS, int NQ>
 __device__ __forceinline__ void lj_plain_mop(const FbArgs& a, const double* pos, const int* key,
-                                             const uint64_t* row, int n, size_t cap, double xi, double yi,
+                                             const ListRow& row, int n, double xi, double yi,
                                              double zi, MopI& m, const Team& tm, double& fx, double& fy,
                                              double& fz, double& pe_out, double& vir_out) {
     double sx = 0, sy = 0, sz = 0, pe = 0.0, vt = 0.0;
     const int T = tm.T;
-    uint64_t wn = 4 * tm.t < n ? row[(size_t)tm.t * cap] : 0;
-    for (int kw = 4 * tm.t; kw < n; kw += 4 * T) {
+    int left = n - 4 * tm.t;
+    uint64_t wn = row[0];
+    for (int k = 0; left > 0; ++k, left -= 4 * T) {
         const uint64_t w = wn;
-        if (kw + 4 * T < n) wn = row[(size_t)((kw >> 2) + T) * cap];
+        wn = row[k + 1];
 #pragma unroll 1
         for (int q = 0; q < 4; q += NQ) {
             P4K p;
             lj_stage_k<NQ>(p, pos, key, w >> (16 * q));
-            lj_word_mop<NS, NQ>(a, p, n - kw - q, xi, yi, zi, m, sx, sy, sz, pe, vt);
+            lj_word_mop<NS, NQ>(a, p, left - q, xi, yi, zi, m, sx, sy, sz, pe, vt);
         }
     }
     fx = 24.0 * team_sum(sx, T);
@@ -2473,7 +2524,7 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
             }
         }
         double fx, fy, fz, pe, vir;
-        lj_plain_mop<NS, EXTRA ? 1 : 2>(a, r.pos, r.lslot, a.nbl + i, a.nbn[i], cap, xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
+        lj_plain_mop<NS, EXTRA ? 1 : 2>(a, r.pos, r.lslot, ListRow(a, i, tm), a.nbn[i], xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
         if constexpr (NS > 0) {
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
@@ -2491,14 +2542,7 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
             fz = fz + a.s.az[i];
             vir = vir + a.vir[i];
         }
-        a.s.ax[i] = fx;
-        a.s.ay[i] = fy;
-        a.s.az[i] = fz;
-        if (a.kick) {
-            a.s.vx[i] = a.s.vx[i] + a.hdt * fx;
-            a.s.vy[i] = a.s.vy[i] + a.hdt * fy;
-            a.s.vz[i] = a.s.vz[i] + a.hdt * fz;
-        }
+        store_force(a, i, fx, fy, fz);
         a.vir[i] = vir;
         a.pe_lj[i] = pe;
     }
@@ -2678,7 +2722,7 @@ __device__ __forceinline__ void lj_word32(const P4F& p, int kw, int left, float 
 // (tab: the brick's staging table when the region was staged from it, for the image shifts)
 template <bool REC>
 __device__ __forceinline__ void lj_plain32(const FbArgs& a, const Region& r, const int* tab, const float4* p4, int i,
-                                           const uint64_t* row, int n, size_t cap, float xi, float yi, float zi,
+                                           int n, float xi, float yi, float zi,
                                            double& fx, double& fy, double& fz, double& pe, double& vir) {
     float sx = 0.f, sy = 0.f, sz = 0.f;
     double vt = 0.0;
@@ -2687,19 +2731,19 @@ __device__ __forceinline__ void lj_plain32(const FbArgs& a, const Region& r, con
     uint32_t bl0 = 0, bl1 = 0;
     int nb = 0;
     P4F pa, pb;
-    const int lastw = n > 0 ? (n - 1) >> 2 : 0;
-    uint64_t w0 = row[0];
+    const ListRow row(a, i, Team{0, 0, 0, 1});
+    const uint64_t w0 = row[0];
     uint64_t wa = n > 0 ? w0 : 0;
     lj_stage32(pa, p4, wa);
-    uint64_t w1 = row[(size_t)min(1, lastw) * cap];
-    uint64_t w2 = row[(size_t)min(2, lastw) * cap];
-    for (int kw = 0; kw < n; kw += 8) {
-        const int k = kw >> 2;
+    uint64_t w1 = row[1];
+    uint64_t w2 = row[2];
+    for (int k = 0; 4 * k < n; k += 2) {
+        const int kw = 4 * k;
         const uint64_t wb = kw + 4 < n ? w1 : 0;
         lj_stage32(pb, p4, wb);
         const uint64_t wk2 = w2;
-        w1 = row[(size_t)min(k + 3, lastw) * cap];
-        w2 = row[(size_t)min(k + 4, lastw) * cap];
+        w1 = row[k + 3];
+        w2 = row[k + 4];
         __builtin_amdgcn_sched_barrier(0);
         lj_word32<REC>(pa, kw, n - kw, xi, yi, zi, rc2f, band, sx, sy, sz, bl0, bl1, nb, a.potshift, &pe, &vt);
         wa = kw + 8 < n ? wk2 : 0;
@@ -2722,7 +2766,7 @@ __device__ __forceinline__ void lj_plain32(const FbArgs& a, const Region& r, con
                 const uint64_t packed = ((uint64_t)bl1 << 32) | bl0;
                 e = (int)((packed >> (12 * b)) & 0xfffu);
             }
-            const int j = (int)((row[(size_t)(e >> 2) * cap] >> (16 * (e & 3))) & 0xffffu);
+            const int j = (int)((a.nbl[(size_t)(e >> 2) * a.cap + i] >> (16 * (e & 3))) & 0xffffu);
             const float4 v = p4[j];
             const float dx = xi - v.x, dy = yi - v.y, dz = zi - v.z;
             if (!(fabsf(r2_32(dx, dy, dz) - rc2f) < band)) continue;
@@ -2764,23 +2808,17 @@ __device__ __forceinline__ void forces_body32(const FbArgs& a, int brick, char* 
         }
         const float4 me = p4[li];
         double fx, fy, fz, pe, vir;
-        lj_plain32<REC>(a, r, tab, p4, i, a.nbl + i, a.nbn[i], cap, me.x, me.y, me.z, fx, fy, fz, pe, vir);
+        lj_plain32<REC>(a, r, tab, p4, i, a.nbn[i], me.x, me.y, me.z, fx, fy, fz, pe, vir);
         if constexpr (REC) {
             a.vir[i] = vir;
             a.pe_lj[i] = pe;
         }
         if constexpr (P1) {  // (k_forces_brick_plain32 only: its one argument is the FbArgs)
-            vv_pass2_pass1<REC>(fargs_again(), i, fx, fy, fz);
+            const FbArgs& b = fargs_again();
+            vv_pass2_pass1<REC>(b, i, b.s.x[i], b.s.y[i], b.s.z[i], fx, fy, fz);
             continue;
         }
-        a.s.ax[i] = fx;
-        a.s.ay[i] = fy;
-        a.s.az[i] = fz;
-        if (a.kick) {
-            a.s.vx[i] = a.s.vx[i] + a.hdt * fx;
-            a.s.vy[i] = a.s.vy[i] + a.hdt * fy;
-            a.s.vz[i] = a.s.vz[i] + a.hdt * fz;
-        }
+        store_force(a, i, fx, fy, fz);
     }
 }
 
@@ -3039,14 +3077,7 @@ __device__ __forceinline__ void forces_body_mixed(const FbArgs& a, int brick, ch
                 for (int d = 0; d < 3; ++d) T[i + d * cap] = T[i + d * cap] + T[i + (3 + d) * cap] * a.dt;
             }
         }
-        a.s.ax[i] = dfx;
-        a.s.ay[i] = dfy;
-        a.s.az[i] = dfz;
-        if (a.kick) {
-            a.s.vx[i] = a.s.vx[i] + a.hdt * dfx;
-            a.s.vy[i] = a.s.vy[i] + a.hdt * dfy;
-            a.s.vz[i] = a.s.vz[i] + a.hdt * dfz;
-        }
+        store_force(a, i, dfx, dfy, dfz);
         if (VIR) a.vir[i] = vir;
         if (RECORD) a.pe_lj[i] = pe;
     }
@@ -3437,6 +3468,7 @@ int make_fargs(fm_ctx* c, int iter, bool kick, void* out, size_t* lds_out, int* 
     a.flags = c->d_flags;
     a.cap = c->cap;
     a.maxreg = c->maxreg;
+    a.maxw = c->maxnb / 4;
     a.team = c->team;
     const int tplot = c->p.tplot, teval = c->p.teval;
     a.step = iter;
