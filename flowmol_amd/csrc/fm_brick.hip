@@ -766,15 +766,17 @@ k_nlist_quant(NlqArgs a) {
         a.btab[(size_t)brick * a.btab_stride + 1] = r.ni;
     }
     __syncthreads();
-    const int R0 = g.R[0], R1 = g.R[1], nbin = R0 << a.lb;
+    const int R0 = g.R[0], R1 = g.R[1];
     {
         // The rows' x bins: bin e's entry is the first staged molecule of a bin >= e (rows and their
         // molecules follow each other in the region layout).  A thread takes neighbouring molecules
-        // and writes, at each, the bins that begin there.
+        // and writes, at each, the bins that begin there.  A molecule's bin is one of its own cell's
+        // (its quantised x may lie beyond a face): the windows end at the faces of three cells, and
+        // they are all of the molecules of those.
         const int per = (r.total + (int)blockDim.x - 1) / (int)blockDim.x;
         auto bin_of = [&](int q) {
-            const int b = (int)(((float)(qv[q].x & 0xffffu) - 2.0f) * a.hb);
-            return r.gc[r.rq[q]] + min(max(b, 0), nbin - 1);
+            const int b = (int)(((float)(qv[q].x & 0xffffu) - 2.0f) * a.hb), c = r.rq[q];
+            return min(max(r.gc[c] + b, c << a.lb), ((c + 1) << a.lb) - 1);
         };
         const int qa = (int)threadIdx.x * per, qb = min(qa + per, r.total);
         if (qa < qb) {

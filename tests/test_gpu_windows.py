@@ -57,3 +57,33 @@ def test_windows_keep_the_neighbour_set(precision, fill, n, brick):
     g.assign_to_neighbourlist()
     assert np.array_equal(canonical_pairs(*o.neighbourlist()), canonical_pairs(*g.neighbourlist()))
     g.close()
+
+
+def at_faces(columns, seed):
+    """Columns along x of five molecules, one beside a face of each cell, up to 2e-4 to either side: half
+    a step of the list build's quantised grid and less.  Next ones are 2.8, the list radius and the side
+    of a cell, apart within 4e-4."""
+    rng = np.random.default_rng(seed)
+    yz = np.repeat(rng.uniform(0.01, 13.99, (columns, 2)), 5, axis=0) + rng.uniform(-2e-3, 2e-3, (5 * columns, 2))
+    x = 2.8 * np.tile(np.arange(5), columns) + rng.uniform(1e-6, 2e-4, 5 * columns) * rng.choice([-1.0, 1.0], 5 * columns)
+    r = np.column_stack([np.where(x < 0.0, x + 14.0, x), yz]) - 7.0
+    return r[rng.permutation(r.shape[0])]
+
+
+@pytest.mark.parametrize("precision", [FM_PREC_FP64, FM_PREC_MIXED])
+@pytest.mark.parametrize("columns,brick", [(400, (3, 3, 3)), (600, (2, 3, 4)), (300, (5, 2, 3)), (40, (1, 1, 1))])
+def test_pairs_beside_the_cells_faces(precision, columns, brick):
+    r = at_faces(columns, seed=columns)
+    p = config.make_params((14.0, 14.0, 14.0), r.shape[0] / 14.0 ** 3, 2.5, tplot=10)
+    p.precision = precision
+    p.brick[0], p.brick[1], p.brick[2] = brick
+    say(f"case: {r.shape[0]} molecules beside the faces, brick {brick}, precision {precision}")
+    o, g = Oracle(p, r, np.zeros_like(r)), MDContext(p, r, np.zeros_like(r))
+    for x in (o, g):
+        x.assign_to_cell()
+    o.updateborders(1)
+    o.assign_to_neighbourlist()
+    g.messenger_updateborders(1)
+    g.assign_to_neighbourlist()
+    assert np.array_equal(canonical_pairs(*o.neighbourlist()), canonical_pairs(*g.neighbourlist()))
+    g.close()
