@@ -1014,7 +1014,9 @@ k_nlist_quant(NlqArgs a) {
 // give it eight consecutive ones (an octet), whose sign bits are a byte of its hit mask, and so that
 // octet o always falls to the molecule's lane o mod 4.  A value nearer to zero than the error bound
 // below is decided by the reference's FP64 test (rij2 < rneighbr2, src/linklist.f90:717-720,750-754)
-// on the positions in HBM, so the set is the FP64 set exactly.  Each lane then places its hits in LDS
+// on the positions in HBM, so the set is the FP64 set exactly.  The reference looks at the 27 cells
+// around a molecule's own: where the list radius may reach past the next cell (unequal skins, a bond
+// length beyond rc) the candidates of a run are held to the molecule's three cells.  Each lane then places its hits in LDS
 // behind those of the molecule's lanes before it, and the words of four entries go to HBM for
 // neighbouring slots together.
 //
@@ -1102,7 +1104,9 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <bool POLY>
+// CELLS: cells no longer along x than the list radius, so that the tile's x window may pass a molecule's
+// three (a launch of its own: the test costs the list build of 108,000 molecules 1.5 us of 43)
+template <bool POLY, bool CELLS>
 __global__ __launch_bounds__(FB_BLOCK) __attribute__((amdgpu_waves_per_eu(FB_BLOCK / 128))) void k_nlist_tile(NltArgs a) {
     extern __shared__ __align__(16) char smem[];
     const BG& g = a.g;
@@ -1230,6 +1234,12 @@ __global__ __launch_bounds__(FB_BLOCK) __attribute__((amdgpu_waves_per_eu(FB_BLO
         nb = __builtin_amdgcn_readfirstlane(nb);
         const int li = li0 + min(c, n16 - 1);
         const bool act = c < n16;
+        auto own_cell = [&] {  // the molecule's region cell in its row
+            int x = 1;
+            for (int k = 1; k < ex; ++k) x += li >= r.off[rowc + 1 + k] ? 1 : 0;
+            return x;
+        };
+        const int rx = CELLS ? own_cell() : 0;
         const float wi = pos[4 * li + 3], q2 = 2.0f * sqrtf(wi) + a.rn;
         const float band = (28.0f / 16777216.0f) * (q2 * q2 + ra2f + a.hext * a.rn);
         const float pv = pos[4 * li + gl], bop = gl < 3 ? -2.0f * pv : 1.0f;
@@ -1270,6 +1280,10 @@ __global__ __launch_bounds__(FB_BLOCK) __attribute__((amdgpu_waves_per_eu(FB_BLO
                 }
             }
             if (k == 4 && (unsigned)(li - jl) < 8u) m &= ~(1u << (li - jl));  // not itself
+            if constexpr (CELLS) {  // those of the molecule's own three cells of the run
+                const int* const off = r.off + R0 * ((ry + k % 3 - 1) + R1 * (rz + k / 3 - 1)) + rx;
+                m &= 0xffu << min(max(off[-1] - jl, 0), 8) & 0xffu >> (8 - min(max(off[2] - jl, 0), 8));
+            }
             return m;
         };
         uint16_t* const row = lb + c * a.maxnb;
@@ -1337,9 +1351,7 @@ __global__ __launch_bounds__(FB_BLOCK) __attribute__((amdgpu_waves_per_eu(FB_BLO
         wmax = max(wmax, act ? cnt : 0);
         wave_sync();
         const int n = min(cnt, a.maxnb);
-        int rc = rowc + 1;
-        for (int k = 1; k < ex; ++k) rc += li >= r.off[rowc + 1 + k] ? 1 : 0;
-        const int slot = r.cst[rc] + (li - r.off[rc]);
+        const int rc = rowc + (CELLS ? rx : own_cell()), slot = r.cst[rc] + (li - r.off[rc]);
         if (act) {
             for (int w = gl; 4 * w < n; w += 4) {
                 uint64_t word = *(const uint64_t*)(row + 4 * w);
@@ -3326,9 +3338,13 @@ int launch_nlist(fm_ctx* c) {
         q.rn = (float)(sqrt(a.ra2) * (1.0 + 1e-6));
         q.xw = (float)(sqrt(a.ra2) * (1.0 + 1e-6) + 1e-6 * h);
         const dim3 grid(brick_count(c)), blk(64 * nw);
+        const bool cells = sqrt(a.ra2) * (1.0 + 1e-9) > c->cs[0];
         ktimer_begin(c, KT_NLIST);
-        if (a.mono) k_nlist_tile<true><<<grid, blk, tile_lds, c->stream>>>(q);
-        else k_nlist_tile<false><<<grid, blk, tile_lds, c->stream>>>(q);
+        if (a.mono) {
+            if (cells) k_nlist_tile<true, true><<<grid, blk, tile_lds, c->stream>>>(q);
+            else k_nlist_tile<true, false><<<grid, blk, tile_lds, c->stream>>>(q);
+        } else if (cells) k_nlist_tile<false, true><<<grid, blk, tile_lds, c->stream>>>(q);
+        else k_nlist_tile<false, false><<<grid, blk, tile_lds, c->stream>>>(q);
         LAUNCH_CHECK();
         ktimer_end(c, KT_NLIST);
         c->btab_valid = true;

@@ -87,3 +87,54 @@ def test_pairs_beside_the_cells_faces(precision, columns, brick):
     g.assign_to_neighbourlist()
     assert np.array_equal(canonical_pairs(*o.neighbourlist()), canonical_pairs(*g.neighbourlist()))
     g.close()
+
+
+# Cells shorter than the list radius: the reference looks at the 27 cells around a molecule's own, so
+# a pair nearer than the radius whose cells are two apart is in no list.
+@pytest.mark.parametrize("precision", [FM_PREC_FP64, FM_PREC_MIXED])
+@pytest.mark.parametrize("n,brick", [(700, (1, 1, 1)), (900, (2, 1, 1)), (1600, (5, 1, 2)), (1500, (3, 1, 1)),
+                                     (2500, (3, 3, 3)), (3000, (5, 2, 2))])
+def test_unequal_skins(precision, n, brick):
+    rng = np.random.default_rng(n)
+    L = np.array([12.5, 14.75, 14.75])      # 5 cells of 2.5, 2.95 and 2.95; list radius 2.8
+    r = rng.uniform(-0.5, 0.5, (n, 3)) * L
+    p = config.make_params(L, n / L.prod(), 2.5, tplot=10)
+    p.precision = precision
+    for d, skin in enumerate((0.0, 0.45, 0.45)):
+        p.delta_rneighbr[d] = skin
+    p.brick[0], p.brick[1], p.brick[2] = brick
+    say(f"case: {n} molecules, cells of 2.5, radius 2.8, brick {brick}, precision {precision}")
+    o, g = Oracle(p, r, np.zeros_like(r)), MDContext(p, r, np.zeros_like(r))
+    for x in (o, g):
+        x.assign_to_cell()
+    o.updateborders(1)
+    o.assign_to_neighbourlist()
+    g.messenger_updateborders(1)
+    g.assign_to_neighbourlist()
+    assert np.array_equal(canonical_pairs(*o.neighbourlist()), canonical_pairs(*g.neighbourlist()))
+    g.close()
+
+
+@pytest.mark.parametrize("brick", [(1, 1, 1), (3, 2, 2), (7, 1, 3), (7, 9, 4)])
+def test_bond_length_beyond_the_cells(brick):
+    p, r, v, moltype, mono = config.config_polymer((6, 8, 6), seed=12)
+    p.rcutoff = config.WCA_CUT              # cells of 1.436 and 1.49, list radius R_0 = 1.5
+    rng = np.random.default_rng(7)
+    r = r + rng.uniform(-1.0, 1.0, r.shape) * (0.15, 0.03, 0.03)
+    L = np.array([p.domain[d] for d in range(3)])
+    r = np.where(r < -0.5 * L, r + L, np.where(r >= 0.5 * L, r - L, r))
+    p.brick[0], p.brick[1], p.brick[2] = brick
+    say(f"case: chains, cells of 1.44, radius 1.5, brick {brick}")
+    o, g = Oracle(p, r, v), MDContext(p, r, v)
+    for x in (o, g):
+        x.set_moltype(moltype)
+        x.set_monomers(*mono)
+        x.assign_to_cell()
+    o.updateborders(1)
+    o.assign_to_neighbourlist()
+    g.messenger_updateborders(1)
+    g.assign_to_neighbourlist()
+    assert np.array_equal(canonical_pairs(*o.neighbourlist()), canonical_pairs(*g.neighbourlist()))
+    canon = lambda b, s: sorted((i, int(x), int(y)) for i in range(b.shape[0]) for x, y in zip(b[i], s[i]) if x >= 0)
+    assert canon(*o.bonds()) == canon(*g.bonds())
+    g.close()
