@@ -280,13 +280,62 @@ static void default_brick(const fm_params* p, const int nc[3], double occ, int o
 // expected list.  Measured at 5,148 molecules (1x1x1 bricks of 25, 73 entries): 1 lane 19.5 us a step,
 // 2 15.6, 4 14.9, 8 14.3, 16 15.4; at 55,296 with rc 4 (bricks of 76, 266 entries): 1 lane 89 us, 2 71.7,
 // 4 71.9, 16 80; 131,072 beads (bricks of 306): 1 lane 71.9 us, 2 68.5, 4 71.4.  One lane in mixed
-// precision (FP32 sums).
-static int team_of(const fm_ctx* c, double occ, double entries) {
-    if (c->p.precision == FM_PREC_MIXED) return 1;
-    const double I = (double)c->brick[0] * c->brick[1] * c->brick[2] * occ;
+// precision (FP32 sums).  A lane's place in a group of T rows of the list is a 32-bit byte offset (ListRow):
+// T * capacity words are at most 2^32 bytes.
+static int team_of(const fm_params* p, const int brick[3], double occ, double entries, int cap) {
+    if (p->precision == FM_PREC_MIXED) return 1;
+    const double I = (double)brick[0] * brick[1] * brick[2] * occ;
     int T = 1;
-    while (T < 16 && 2 * T * I <= (T == 1 ? 1.4 * FB_BLOCK : 0.5 * FB_BLOCK) && 2 * T * 8 <= entries) T *= 2;
+    while (T < 16 && 2 * T * I <= (T == 1 ? 1.4 * FB_BLOCK : 0.5 * FB_BLOCK) && 2 * T * 8 <= entries &&
+           2 * T * (uint64_t)cap * sizeof(uint64_t) <= (1ull << 32))
+        T *= 2;
     return T;
+}
+
+// The cells of a context, what it expects in them and in a list, and the shape of its launches
+struct Layout {
+    int nc[3];
+    size_t ncell;
+    double rn;        // list radius
+    double occ;       // molecules a cell
+    double entries;   // of a full list at the mean density
+    int brick[3];
+    int team;
+    bool tile_list;   // the rule of k_nlist_tile
+};
+
+static int plan_layout(const fm_params* p, int np, int cap, Layout* l) {
+    // set_parameters_cells (src/setup_set_parameters.f90:1848-1903)
+    l->rn = p->rcutoff + (p->delta_rneighbr[0] + p->delta_rneighbr[1] + p->delta_rneighbr[2]) / 3.0;
+    if (p->potential_flag == 1 && l->rn < p->R_0) l->rn = p->R_0;
+    for (int d = 0; d < 3; ++d) {
+        l->nc[d] = (int)floor(p->domain[d] / (p->rcutoff + p->delta_rneighbr[d]));
+        if (l->nc[d] < 3)
+            return fm_set_error(FM_EINVAL, "ERROR - DOMAIN SHOULD HAVE AT LEAST 3 CELLS, IN X, Y AND Z - INCREASE NUMBER OF UNITS IN INPUT");
+    }
+    l->ncell = (size_t)l->nc[0] * l->nc[1] * l->nc[2];
+    l->occ = std::max(1.0, (double)np / l->ncell);
+    const double dens = std::max(p->density, np / (p->domain[0] * p->domain[1] * p->domain[2]));
+    l->entries = 4.0 / 3.0 * M_PI * l->rn * l->rn * l->rn * dens;
+    if (p->brick[0] > 0 && p->brick[1] > 0 && p->brick[2] > 0) {
+        for (int d = 0; d < 3; ++d) l->brick[d] = std::min(p->brick[d], l->nc[d]);
+    } else {
+        default_brick(p, l->nc, l->occ, l->brick);
+    }
+    l->team = team_of(p, l->brick, l->occ, l->entries, cap);
+    l->tile_list = p->precision == FM_PREC_FP64 && l->occ <= 40.0 &&
+                   l->brick[0] * l->brick[1] * l->brick[2] * l->occ <= (p->potential_flag == 1 ? 160.0 : 256.0);
+    return 0;
+}
+
+// The launch shape fm_init gives a context: cells per brick, lanes per molecule of the force launches
+extern "C" int fm_default_layout(const fm_params* p, int32_t np, int32_t capacity, int32_t brick[3], int32_t* team) {
+    if (!p || np < 0 || !(p->rcutoff > 0.0)) return fm_set_error(FM_EINVAL, "bad argument");
+    Layout l;
+    TRY(plan_layout(p, np, std::max(std::max(np, capacity), 1), &l));
+    for (int d = 0; d < 3 && brick; ++d) brick[d] = l.brick[d];
+    if (team) *team = l.team;
+    return 0;
 }
 
 // Block curve of sort_mols: SORT_FLAG 1 numbers the blocks x fastest
@@ -392,32 +441,27 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
         return fm_set_error(FM_EINVAL, "capacity %d exceeds 2^27 molecules per context", c->cap);
     }
 
-    // set_parameters_cells (src/setup_set_parameters.f90:1848-1903)
     for (int d = 0; d < 3; ++d) c->half[d] = 0.5 * p->domain[d];
-    double rneighbr = p->rcutoff + (p->delta_rneighbr[0] + p->delta_rneighbr[1] + p->delta_rneighbr[2]) / 3.0;
-    c->rn2 = rneighbr * rneighbr;
-    if (p->potential_flag == 1 && rneighbr < p->R_0) {
-        rneighbr = p->R_0;
-        c->rn2 = p->R_0 * p->R_0;
-    }
-    for (int d = 0; d < 3; ++d) c->nc[d] = (int)floor(p->domain[d] / (p->rcutoff + p->delta_rneighbr[d]));
-    if (c->nc[0] < 3 || c->nc[1] < 3 || c->nc[2] < 3) {
+    Layout lay;
+    if (int rc = plan_layout(p, np, c->cap, &lay)) {
         free_ctx(c);
-        return fm_set_error(FM_EINVAL, "ERROR - DOMAIN SHOULD HAVE AT LEAST 3 CELLS, IN X, Y AND Z - INCREASE NUMBER OF UNITS IN INPUT");
+        return rc;
     }
-    for (int d = 0; d < 3; ++d) c->cs[d] = p->domain[d] / c->nc[d];
-    c->ncell = c->nc[0] * c->nc[1] * c->nc[2];
+    c->rn2 = lay.rn * lay.rn;
+    for (int d = 0; d < 3; ++d) {
+        c->nc[d] = lay.nc[d];
+        c->cs[d] = p->domain[d] / c->nc[d];
+        c->brick[d] = lay.brick[d];
+    }
+    c->ncell = (int)lay.ncell;
+    c->team = lay.team;
+    c->tile_list = lay.tile_list;
     c->rc2 = p->rcutoff * p->rcutoff;
     {
         double rc = p->rcutoff, x3 = rc * (rc * rc), x6 = x3 * x3, x12 = x6 * x6;
         c->potshift = 4.0 * (1.0 / x12 - 1.0 / x6);
     }
     c->dmin = std::min(p->delta_rneighbr[0], std::min(p->delta_rneighbr[1], p->delta_rneighbr[2]));
-    if (p->brick[0] > 0 && p->brick[1] > 0 && p->brick[2] > 0) {
-        for (int d = 0; d < 3; ++d) c->brick[d] = std::min(p->brick[d], c->nc[d]);
-    } else {
-        default_brick(p, c->nc, std::max(1.0, (double)np / c->ncell), c->brick);
-    }
     {
         hipDeviceProp_t prop;
         if (hipGetDeviceProperties(&prop, dev) == hipSuccess) {
@@ -430,17 +474,8 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
 
     // neighbour capacity: 1.5x the expected count at the mean density, plus margin
     int maxnb = p->max_neighbours;
-    const double dens = std::max(p->density, np / (p->domain[0] * p->domain[1] * p->domain[2]));
-    const double expect = 4.0 / 3.0 * M_PI * rneighbr * rneighbr * rneighbr * dens;
-    {
-        const double occ = std::max(1.0, (double)np / c->ncell);
-        c->team = team_of(c, occ, expect);
-        // (the rule of k_nlist_tile)
-        c->tile_list = p->precision == FM_PREC_FP64 && occ <= 40.0 &&
-                       c->brick[0] * c->brick[1] * c->brick[2] * occ <= (p->potential_flag == 1 ? 160.0 : 256.0);
-    }
     if (maxnb <= 0) {
-        maxnb = (int)(1.5 * expect) + 32;
+        maxnb = (int)(1.5 * lay.entries) + 32;
         maxnb = (maxnb + 3) & ~3;
     }
 

@@ -54,3 +54,30 @@ def test_forces_and_tallies(liquid, brick, tally):
         if it == 0 and p.pressure_outflag:
             assert np.abs(g.rfmol() - o.rfmol()).max() <= 10 * TOL * np.abs(o.rfmol()).max()
     g.close()
+
+
+@pytest.mark.parametrize("capacity", [0, 2 ** 26 + 1])   # 16 lanes, and 4 where 8 would pass 32-bit offsets
+@pytest.mark.parametrize("it", [0, 1])                   # a record step, a step without tallies
+def test_sixteen_lanes_and_a_capacity_beyond_32_bit_offsets(capacity, it):
+    import torch
+
+    if capacity and torch.cuda.mem_get_info()[0] < 60 * 2 ** 30:
+        pytest.skip("needs 60 GiB of device memory")
+    p, r, v = config.config_fcc((8, 8, 8), 0.4, 2.5, seed=19, tplot=4)
+    r = r + np.random.default_rng(19).uniform(-0.2, 0.2, r.shape)
+    L = np.array([p.domain[d] for d in range(3)])
+    r = np.where(r < -0.5 * L, r + L, np.where(r >= 0.5 * L, r - L, r))
+    p.density = 1.6                         # (the rule's expectation: 147 entries; the lists hold half)
+    p.max_neighbours = 96
+    p.brick[0] = p.brick[1] = p.brick[2] = 1
+    say(f"case: 2048 LJ, bricks of ten, capacity {capacity}, step {it}")
+    o, g = Oracle(p, r, v), MDContext(p, r, v, capacity=capacity)
+    o.setup()
+    g.setup(1)
+    o.compute_forces(it)
+    g.simulation_compute_forces(it)
+    assert rel_force_err(g.state()[2], o.state()[2], o.force_scale()) < TOL
+    if it == 0:
+        for ref, got in zip(o.molecular(), g.molecular()):
+            assert np.abs(got - ref).max() <= TOL * np.abs(ref).max()
+    g.close()

@@ -4,6 +4,9 @@ import itertools
 import numpy as np
 import pytest
 
+from flowmol_amd import config
+from flowmol_amd._abi import iptr
+from flowmol_amd._lib import check, load
 from flowmol_amd.md import FB_BLOCK, brick_candidates
 
 
@@ -60,3 +63,25 @@ def test_random_walk_chains():
     assert list(sub[:8]) == list(range(1, 9)) and list(funcy[:8]) == [1, 2, 2, 2, 2, 2, 2, 1]
     _, r2, _, _, _ = config.config_polymer(nunits=(8, 8, 8), init="random_walk", seed=9)
     assert np.array_equal(r, r2)
+
+
+def layout(p, nmol, capacity=0):
+    """(brick, lanes per molecule) that a context of these parameters gets."""
+    brick, team = np.zeros(3, np.int32), np.zeros(1, np.int32)
+    check(load().fm_default_layout(p, nmol, capacity, iptr(brick), iptr(team)))
+    return tuple(int(x) for x in brick), int(team[0])
+
+
+@pytest.mark.parametrize("density,lanes", [(0.8, 8), (1.6, 16)])   # 73 and 147 expected entries
+def test_lanes_keep_the_list_offsets_within_32_bits(density, lanes):
+    """A lane's place in its team's rows of the list is a 32-bit byte offset: however large the capacity
+    that fm_init takes (below 2^27), lanes x capacity x 8 bytes are at most 2^32."""
+    p, r, _ = config.config_fcc((8, 8, 8), 0.4, 2.5, seed=1, tplot=10)
+    p.density = density
+    p.brick[0] = p.brick[1] = p.brick[2] = 1
+    nmol = r.shape[0]                      # 2,048 in 6^3 cells: ten a brick
+    assert layout(p, nmol)[1] == lanes
+    for capacity in (2 ** 24, 2 ** 25, 2 ** 25 + 1, 2 ** 26, 2 ** 26 + 1, 2 ** 27 - 1):
+        team = layout(p, nmol, capacity)[1]
+        assert 1 <= team <= lanes and team * capacity * 8 <= 2 ** 32
+        assert team == lanes or 2 * team * capacity * 8 > 2 ** 32
