@@ -564,10 +564,12 @@ __global__ __launch_bounds__(FM_BLOCK) void k_bin_count(WrapArgs a, BinArgs b) {
         if (ok) {
             cell = c[0] + b.nc[0] * (c[1] + b.nc[1] * c[2]);
         } else {
-            // counted in cell 0 so that the permutation stays complete; the error stops the run
+            // counted in some cell so that the permutation stays complete; the error stops the run.
+            // (All over the box: k_bin_order ranks a cell in n^2 / 64 steps of one wavefront, a minute
+            // for a million molecules in one cell)
             // (WRAP: the renumbering that follows turns ~slot into the molecule's number)
             set_err(a.flags, FM_EESCAPE, WRAP ? ~i : a.ext[i]);
-            cell = 0;
+            cell = i % (b.nc[0] * b.nc[1] * b.nc[2]);
         }
         b.cell_of[i] = cell;
     }

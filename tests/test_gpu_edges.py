@@ -49,3 +49,25 @@ def test_domain_below_three_cells_is_rejected():
     with pytest.raises(FlowmolHipError) as e:
         MDContext(p, r, v)
     assert "3 CELLS" in str(e.value).upper()
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_a_state_of_escaped_molecules_is_refused_at_once(bad):
+    """A million molecules that are nowhere: the binning keeps them in one cell, whose order is not
+    worked out (a minute by one wavefront), and the error names one of them."""
+    import time
+
+    p, r, v = config.config_fcc((64, 64, 64), 0.8, 2.5, seed=3, tplot=10)
+    q = np.full_like(r, bad)
+    say(f"case: 1048576 molecules at {bad}")
+    g = MDContext(p, r, v)
+    g.upload_state(q, v)
+    t = time.perf_counter()
+    with pytest.raises(FlowmolHipError) as e:
+        g.assign_to_cell()
+    assert e.value.code == FM_EESCAPE
+    assert time.perf_counter() - t < 5.0
+    g.upload_state(r, v)      # the context goes on with a good state
+    g.setup(0)
+    assert np.isfinite(g.state()[2]).all()
+    g.close()
