@@ -70,7 +70,7 @@ SIGNATURES = {
     "fm_batch_size": (C.c_int, [_vp, _ip]),
     "fm_batch_get_iter": (C.c_int, [_vp, _vp, _ip]),
     "fm_memory_footprint": (C.c_int, [C.POINTER(FmParams), _i32, _lp]),
-    "fm_default_layout": (C.c_int, [C.POINTER(FmParams), _i32, _i32, _ip, _ip]),
+    "fm_default_layout": (C.c_int, [C.POINTER(FmParams), _i32, _i32, _i32, _ip, _ip]),
     "fm_synchronize": (C.c_int, [_vp]),
     "fm_kernel_timing": (C.c_int, [_vp, _i32]),
     "fm_get_kernel_timing": (C.c_int, [_vp, C.c_char_p, _i32, _dp, _lp, _i32, _ip]),

@@ -216,15 +216,16 @@ static int set_brick(fm_ctx* c, const int b[3]) {
 // Brick shape: the least estimated time of a force launch, among the shapes whose expected molecule
 // count fits one pass of the workgroup (15/16 of its threads).  A workgroup's time goes with the
 // molecules R that it stages (its cells and one halo layer; about 11 ns a molecule and 3 us beside
-// them, the pair loop running under the staging of the CU's other workgroup), and 512 workgroups run
-// at once, two on a CU where the staged regions leave room for two.  So a large domain takes the
+// them, the pair loop running under the staging of the CU's other workgroup), and two workgroups run
+// at once on each of the device's CUs where the staged regions leave room for two (512 on the 256 CUs
+// of a whole MI355X, 64 on a partition of 32).  So a large domain takes the
 // shape with the least halo per cell (1,048,576 molecules: 3x3x3 cells, 2197 bricks), and one whose
 // bricks would leave workgroup slots empty takes smaller ones, as many as the slots.  Measured, a step
 // of 108,000 molecules (rc 2.5): 3x3x3 (216 bricks) 48.5 us, 3x2x2 (486) 37.1, 2x2x2 (729) 45.5; of
 // 55,296 with rc 4: 2x3x1 78.6 us, 1x1x1 (729, two on a CU) 67.5, 2x1x1 (405, one on a CU) 83; of 5,148:
 // 3x3x2 27.3 us, 1x2x1 (120) 18.5 and with teams of lanes 14.6, 1x1x1 (210) 14.3: single cells of few
 // molecules are left out (each molecule would be staged 27 times over for nothing).
-static void choose_brick(const int nc[3], double occ, int out[3]) {
+static void choose_brick(const int nc[3], double occ, int cus, int out[3]) {
     const double target = FB_BLOCK * 15.0 / 16.0;
     double best = -1.0;
     out[0] = out[1] = out[2] = 1;
@@ -237,7 +238,7 @@ static void choose_brick(const int nc[3], double occ, int out[3]) {
                 const double R = (bx + 2) * (by + 2) * (bz + 2) * occ;
                 const double nb = (double)((nc[0] + bx - 1) / bx) * ((nc[1] + by - 1) / by) * ((nc[2] + bz - 1) / bz);
                 // (27 B a staged molecule with its share of the tables; the largest region 15 % above the mean)
-                const double slots = 256.0 * (R * 1.15 * 27.0 <= 80.0 * 1024.0 ? 2 : 1);
+                const double slots = (double)cus * (R * 1.15 * 27.0 <= 80.0 * 1024.0 ? 2 : 1);
                 const double cost = (nb <= slots ? 1.0 : nb / slots + 0.2) * (R + 300.0);
                 // (of equal ones the longest along x, the order of the slots)
                 if (best < 0.0 || cost <= best * (1.0 + 1e-12)) {
@@ -270,9 +271,22 @@ static void choose_brick_halo(const int nc[3], double occ, int out[3]) {
             }
 }
 
-static void default_brick(const fm_params* p, const int nc[3], double occ, int out[3]) {
+static void default_brick(const fm_params* p, const int nc[3], double occ, int cus, int out[3]) {
     if (p->precision == FM_PREC_MIXED) choose_brick_halo(nc, occ, out);
-    else choose_brick(nc, occ, out);
+    else choose_brick(nc, occ, cus, out);
+}
+
+#define MAX_CUS 256  // of a whole MI355X
+
+// CUs of the current device; those of a whole one where there is none (host-only use)
+static int device_cus() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
+        (void)hipGetLastError();
+        return MAX_CUS;
+    }
+    return cus;
 }
 
 // Lanes per molecule of the force launches: two where a brick's molecules leave over a quarter of the
@@ -304,7 +318,7 @@ struct Layout {
     bool tile_list;   // the rule of k_nlist_tile
 };
 
-static int plan_layout(const fm_params* p, int np, int cap, Layout* l) {
+static int plan_layout(const fm_params* p, int np, int cap, int cus, Layout* l) {
     // set_parameters_cells (src/setup_set_parameters.f90:1848-1903)
     l->rn = p->rcutoff + (p->delta_rneighbr[0] + p->delta_rneighbr[1] + p->delta_rneighbr[2]) / 3.0;
     if (p->potential_flag == 1 && l->rn < p->R_0) l->rn = p->R_0;
@@ -320,7 +334,7 @@ static int plan_layout(const fm_params* p, int np, int cap, Layout* l) {
     if (p->brick[0] > 0 && p->brick[1] > 0 && p->brick[2] > 0) {
         for (int d = 0; d < 3; ++d) l->brick[d] = std::min(p->brick[d], l->nc[d]);
     } else {
-        default_brick(p, l->nc, l->occ, l->brick);
+        default_brick(p, l->nc, l->occ, cus, l->brick);
     }
     l->team = team_of(p, l->brick, l->occ, l->entries, cap);
     l->tile_list = p->precision == FM_PREC_FP64 && l->occ <= 40.0 &&
@@ -329,10 +343,11 @@ static int plan_layout(const fm_params* p, int np, int cap, Layout* l) {
 }
 
 // The launch shape fm_init gives a context: cells per brick, lanes per molecule of the force launches
-extern "C" int fm_default_layout(const fm_params* p, int32_t np, int32_t capacity, int32_t brick[3], int32_t* team) {
-    if (!p || np < 0 || !(p->rcutoff > 0.0)) return fm_set_error(FM_EINVAL, "bad argument");
+extern "C" int fm_default_layout(const fm_params* p, int32_t np, int32_t capacity, int32_t compute_units,
+                                 int32_t brick[3], int32_t* team) {
+    if (!p || np < 0 || compute_units < 0 || !(p->rcutoff > 0.0)) return fm_set_error(FM_EINVAL, "bad argument");
     Layout l;
-    TRY(plan_layout(p, np, std::max(std::max(np, capacity), 1), &l));
+    TRY(plan_layout(p, np, std::max(std::max(np, capacity), 1), compute_units > 0 ? compute_units : device_cus(), &l));
     for (int d = 0; d < 3 && brick; ++d) brick[d] = l.brick[d];
     if (team) *team = l.team;
     return 0;
@@ -443,7 +458,7 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
 
     for (int d = 0; d < 3; ++d) c->half[d] = 0.5 * p->domain[d];
     Layout lay;
-    if (int rc = plan_layout(p, np, c->cap, &lay)) {
+    if (int rc = plan_layout(p, np, c->cap, device_cus(), &lay)) {
         free_ctx(c);
         return rc;
     }
@@ -633,7 +648,8 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
     return 0;
 }
 
-// Device bytes fm_init allocates for these parameters (admission control by HBM footprint).
+// Device bytes fm_init allocates for these parameters (admission control by HBM footprint).  Host
+// arithmetic only: no device is asked (bricks as on the most CUs, the smallest and so the largest tables).
 extern "C" int fm_memory_footprint(const fm_params* p, int32_t np, int64_t* bytes) {
     if (!p || !bytes || np < 0) return fm_set_error(FM_EINVAL, "bad argument");
     int nc[3];
@@ -668,7 +684,7 @@ extern "C" int fm_memory_footprint(const fm_params* p, int32_t np, int64_t* byte
         if (p->brick[0] > 0 && p->brick[1] > 0 && p->brick[2] > 0) {
             for (int d = 0; d < 3; ++d) br[d] = std::min(p->brick[d], nc[d]);
         } else {
-            default_brick(p, nc, std::max(1.0, (double)np / ncell), br);
+            default_brick(p, nc, std::max(1.0, (double)np / ncell), MAX_CUS, br);
         }
         double halo = 1.0;
         for (int d = 0; d < 3; ++d) halo *= (br[d] + 2.0) / br[d];

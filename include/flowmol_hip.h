@@ -300,8 +300,10 @@ int  fm_batch_get_iter(const fm_batch* b, const fm_ctx* ctx, int32_t* iter);
 /* device bytes fm_init would allocate (admission control by HBM footprint) */
 int  fm_memory_footprint(const fm_params* p, int32_t np, int64_t* bytes);
 /* the launch shape fm_init would choose (or takes from p->brick): cells per LDS brick, and lanes per
-   molecule of the force launches.  Either output may be null. */
-int  fm_default_layout(const fm_params* p, int32_t np, int32_t capacity, int32_t brick[3], int32_t* team);
+   molecule of the force launches, on a device of compute_units CUs (0: the current device's, or
+   256 without one).  Either output may be null. */
+int  fm_default_layout(const fm_params* p, int32_t np, int32_t capacity, int32_t compute_units,
+                       int32_t brick[3], int32_t* team);
 
 /* ---- timing / synchronisation -------------------------------------------------------------- */
 int  fm_synchronize(fm_ctx* ctx);

@@ -65,10 +65,10 @@ def test_random_walk_chains():
     assert np.array_equal(r, r2)
 
 
-def layout(p, nmol, capacity=0):
+def layout(p, nmol, capacity=0, compute_units=0):
     """(brick, lanes per molecule) that a context of these parameters gets."""
     brick, team = np.zeros(3, np.int32), np.zeros(1, np.int32)
-    check(load().fm_default_layout(p, nmol, capacity, iptr(brick), iptr(team)))
+    check(load().fm_default_layout(p, nmol, capacity, compute_units, iptr(brick), iptr(team)))
     return tuple(int(x) for x in brick), int(team[0])
 
 
@@ -85,3 +85,15 @@ def test_lanes_keep_the_list_offsets_within_32_bits(density, lanes):
         team = layout(p, nmol, capacity)[1]
         assert 1 <= team <= lanes and team * capacity * 8 <= 2 ** 32
         assert team == lanes or 2 * team * capacity * 8 > 2 ** 32
+
+
+def test_default_bricks_are_as_many_as_the_device_runs_at_once():
+    """108,000 molecules in 18^3 cells: the largest bricks (24 cells) are too few for the 512 workgroups of
+    256 CUs, which get smaller ones, and enough for a partition of 32 or 64 CUs, which keeps them."""
+    p, r, _ = config.config_fcc((30, 30, 30), 0.8, 2.5, seed=1, tplot=10)
+    cells, bricks = {}, {}
+    for cus in (32, 64, 256):
+        shape = layout(p, r.shape[0], compute_units=cus)[0]
+        cells[cus], bricks[cus] = np.prod(shape), np.prod([-(-18 // b) for b in shape])
+    assert cells[32] == cells[64] == 24
+    assert cells[256] < 24 and 400 <= bricks[256] <= 512
