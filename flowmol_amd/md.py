@@ -20,7 +20,7 @@ import ctypes as C
 
 import numpy as np
 
-from ._abi import FM_ENSEMBLE_TAG_MOVE, FM_MAX_FUNCY, FmMacros, dptr, iptr
+from ._abi import FM_ENSEMBLE_TAG_MOVE, FM_MAX_FUNCY, FmMacros, FmParams, dptr, iptr
 from ._lib import check, load
 
 
@@ -318,11 +318,19 @@ class MDContext:
 FB_BLOCK = 512  # threads of one brick workgroup (FB_BLOCK of the brick kernels)
 
 
-def brick_candidates(ncells, nmol, max_candidates=4):
+def default_brick(params, nmol):
+    """The brick shape that a context of `nmol` molecules gets: params.brick where it is set, else the
+    library's choice for the cells, the occupancy, the precision and the device."""
+    b = np.zeros(3, np.int32)
+    check(load().fm_default_layout(C.byref(params), int(nmol), 0, 0, iptr(b), None))
+    return tuple(int(x) for x in b)
+
+
+def brick_candidates(ncells, nmol, max_candidates=4, default=None):
     """Brick shapes (cells along x, y, z) whose expected molecule count fits one pass of a
-    workgroup (15/16 of FB_BLOCK threads), least staged halo per cell first.  The first one is the
-    library's default for a large domain; a domain of fewer bricks than the device runs at once gets a
-    smaller one by default."""
+    workgroup (15/16 of FB_BLOCK threads), least staged halo per cell first.  `default` (the library's
+    FP64 choice when not given) is always among them: a domain of fewer bricks than the device runs
+    at once does best with smaller ones than the least halo asks for."""
     nc = [int(x) for x in ncells]
     occ = max(1.0, nmol / float(nc[0] * nc[1] * nc[2]))
     target = FB_BLOCK * 15.0 / 16.0
@@ -335,12 +343,23 @@ def brick_candidates(ncells, nmol, max_candidates=4):
                     continue
                 out.append((P / ((bx + 2) * (by + 2) * (bz + 2)), (bx, by, bz)))
     # a stable sort: equal halo efficiency keeps the enumeration order, as the library's choice
-    return [b for _, b in sorted(out, key=lambda t: -t[0])][:max(1, int(max_candidates))]
+    out.sort(key=lambda t: -t[0])
+    if default is None:
+        p = FmParams()
+        for d in range(3):
+            p.domain[d] = nc[d]   # cells of side one
+        p.rcutoff = 1.0
+        default = default_brick(p, nmol)
+    keep = max(1, int(max_candidates))
+    head = [b for _, b in out[:keep]]
+    if default not in head:
+        head = [b for _, b in out if b in head[:keep - 1] or b == default]
+    return head
 
 
 def tune_brick(params, r, v, a=None, steps=20, warmup=5, max_candidates=4, prepare=None):
     """Time `steps` fused velocity Verlet steps (after `warmup` more, list rebuilds included) of the
-    same state on a fresh context per candidate brick shape; returns (fastest shape, {shape:
+    same state on a fresh context per candidate brick shape, the default one among them; returns (fastest shape, {shape:
     seconds per step}).  `params` is not changed: set params.brick to the shape to use it.
     prepare(ctx), when given, loads what the state needs beyond r, v, a (molecule types, monomer
     data, tags) into each fresh context before its setup."""
@@ -350,7 +369,10 @@ def tune_brick(params, r, v, a=None, steps=20, warmup=5, max_candidates=4, prepa
     nc = probe.geometry()["ncells"]
     probe.close()
     times = {}
-    for b in brick_candidates(nc, np.asarray(r).reshape(-1, 3).shape[0], max_candidates):
+    nmol = np.asarray(r).reshape(-1, 3).shape[0]
+    plain = type(params).from_buffer_copy(params)
+    plain.brick[0] = plain.brick[1] = plain.brick[2] = 0
+    for b in brick_candidates(nc, nmol, max_candidates, default_brick(plain, nmol)):
         p = type(params).from_buffer_copy(params)
         p.brick[0], p.brick[1], p.brick[2] = b
         g = MDContext(p, r, v, a)

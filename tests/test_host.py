@@ -5,9 +5,9 @@ import numpy as np
 import pytest
 
 from flowmol_amd import config
-from flowmol_amd._abi import iptr
+from flowmol_amd._abi import FM_PREC_MIXED, iptr
 from flowmol_amd._lib import check, load
-from flowmol_amd.md import FB_BLOCK, brick_candidates
+from flowmol_amd.md import FB_BLOCK, brick_candidates, default_brick
 
 
 @pytest.mark.parametrize("ncells,nmol", [((39, 39, 39), 1048576), ((4, 4, 4), 2048), ((9, 9, 9), 2048),
@@ -97,3 +97,19 @@ def test_default_bricks_are_as_many_as_the_device_runs_at_once():
         cells[cus], bricks[cus] = np.prod(shape), np.prod([-(-18 // b) for b in shape])
     assert cells[32] == cells[64] == 24
     assert cells[256] < 24 and 400 <= bricks[256] <= 512
+
+
+@pytest.mark.parametrize("units,density,rc", [((8, 8, 8), 0.8, 2.5), ((11, 13, 9), 0.8, 2.5), ((16, 16, 16), 0.8, 2.5),
+                                              ((30, 30, 30), 0.8, 2.5), ((24, 24, 24), 0.8, 4.0), ((64, 64, 64), 0.8, 2.5),
+                                              ((12, 12, 12), 0.8, 1.1225)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_the_tuner_times_the_default_brick(units, density, rc, mixed):
+    p, r, _ = config.config_fcc(units, density, rc, seed=1, tplot=10, precision=FM_PREC_MIXED if mixed else 0)
+    nmol, cells = r.shape[0], [int(p.domain[d] // (rc + 0.3)) for d in range(3)]
+    default = layout(p, nmol)[0]
+    assert default_brick(p, nmol) == default
+    for k in (1, 2, 3, 6):
+        got = brick_candidates(cells, nmol, k, default)
+        assert default in got and len(got) == k == len(set(got))
+        if not mixed:
+            assert got == brick_candidates(cells, nmol, k)
