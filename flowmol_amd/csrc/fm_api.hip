@@ -175,12 +175,14 @@ static void free_ctx(fm_ctx* c) {
     delete c;
 }
 
+// rows of four entries of a list, in whole groups of a team's (ListRow)
+static size_t list_rows(int maxnb, int team) { return (size_t)(maxnb / 4 + team - 1) / team * team; }
+
 static int alloc_nlist(fm_ctx* c, int maxnb) {
     if (c->nbl) hipFree(c->nbl);
     c->nbl = nullptr;
     c->maxnb = (maxnb + 3) & ~3;
-    // (whole groups of a team's rows: ListRow)
-    return dalloc(&c->nbl, (size_t)((c->maxnb / 4 + c->team - 1) / c->team * c->team) * c->cap);
+    return dalloc(&c->nbl, list_rows(c->maxnb, c->team) * c->cap);
 }
 
 // a build met a list of `need` entries: room for a quarter more
@@ -648,61 +650,72 @@ extern "C" int fm_init(const fm_params* p, int32_t np, int32_t capacity, fm_ctx*
     return 0;
 }
 
+// Capacity of a staged region of a small brick over the mean region, at most
+#define REGION_HEADROOM 1.6
+
 // Device bytes fm_init allocates for these parameters (admission control by HBM footprint).  Host
 // arithmetic only: no device is asked (bricks as on the most CUs, the smallest and so the largest tables).
 extern "C" int fm_memory_footprint(const fm_params* p, int32_t np, int64_t* bytes) {
-    if (!p || !bytes || np < 0) return fm_set_error(FM_EINVAL, "bad argument");
-    int nc[3];
-    for (int d = 0; d < 3; ++d) {
-        nc[d] = (int)floor(p->domain[d] / (p->rcutoff + p->delta_rneighbr[d]));
-        if (nc[d] < 3) return fm_set_error(FM_EINVAL, "fewer than 3 cells");
-    }
-    const size_t ncell = (size_t)nc[0] * nc[1] * nc[2];
+    if (!p || !bytes || np < 0 || !(p->rcutoff > 0.0)) return fm_set_error(FM_EINVAL, "bad argument");
     const size_t cap = std::max(np, 1);
-    double rneighbr = p->rcutoff + (p->delta_rneighbr[0] + p->delta_rneighbr[1] + p->delta_rneighbr[2]) / 3.0;
-    if (p->potential_flag == 1 && rneighbr < p->R_0) rneighbr = p->R_0;
+    Layout l;
+    TRY(plan_layout(p, np, (int)cap, MAX_CUS, &l));
+    const size_t ncell = l.ncell;
     int maxnb = p->max_neighbours;
-    if (maxnb <= 0) {
-        const double vol = p->domain[0] * p->domain[1] * p->domain[2];
-        const double dens = std::max(p->density, np / vol);
-        maxnb = (int)(1.5 * (4.0 / 3.0 * M_PI * rneighbr * rneighbr * rneighbr * dens)) + 32;
-    }
+    if (maxnb <= 0) maxnb = (int)(1.5 * l.entries) + 32;
     maxnb = (maxnb + 3) & ~3;
-    size_t b = 0;
-    b += 2 * 9 * cap * 8 + 3 * cap * 8 + 9 * cap * 8;          // state copies, rdisp, staging
-    b += (2 + 1 + 1 + 1 + 1 + 1 + 2) * cap * 4 + cap / 8;       // ext, slot_of, cell_of, bin_pos, perm, nbn, sendmols scratch
-    b += 3 * cap * 8;                                           // pe_lj, pe_poly, vir
-    b += (size_t)(maxnb / 4) * cap * 8;                         // neighbour words
-    b += 3 * (ncell + 1) * 4;                                   // cell counts, starts, cursors
-    b += cap * 4 + 4 * 1024 * 1024;                             // scan/select temporary, reductions
-    b += 8 * 1024 * 1024;                                       // the allocator's rounding of ~45 buffers
+    // 2 MiB for the staging tables' rounding (they are counted as they are, below) and 8 MiB for the
+    // small buffers and the tables' growth
+    size_t b = 10u << 20;
+    auto buf = [&](size_t n, size_t count = 1) {  // (buffers of a MiB and more take whole 2 MiB pages)
+        const size_t page = 2u << 20;
+        b += count * (n < page / 2 ? n : (n + page - 1) / page * page);
+    };
+    buf(9 * cap * 8, 3);                                // state copies, staging
+    buf(3 * cap * 8);                                   // rdisp
+    buf(cap * 4, 9);                                    // ext, slot_of, cell_of, bin_pos, perm, nbn, sendmols scratch
+    buf(cap * 8, 3);                                    // pe_lj, pe_poly, vir
+    buf(cap / 8 + 16);                                  // leavers
+    buf(cap / 4 + 64);                                  // reductions
+    size_t rows = maxnb / 4;
+    for (int T = 1; T <= 16 && 8 * T <= std::max(l.entries, 8.0); T *= 2)  // (whichever team the bricks get: team_of)
+        rows = std::max(rows, list_rows(maxnb, T));
+    buf(rows * cap * 8);                                // neighbour words
+    buf((ncell + 1) * 4, 3);                            // cell counts, starts, bricks
     {
-        // staging tables: 10 B per molecule of region capacity per brick (1.125 of the capacity);
-        // the regions hold each molecule prod((B+2)/B) times over, and the capacity is up to
-        // 1.6 times the mean region
-        int br[3];
-        if (p->brick[0] > 0 && p->brick[1] > 0 && p->brick[2] > 0) {
-            for (int d = 0; d < 3; ++d) br[d] = std::min(p->brick[d], nc[d]);
-        } else {
-            default_brick(p, nc, std::max(1.0, (double)np / ncell), MAX_CUS, br);
+        // staging tables: 10 B per molecule of region capacity per brick (1.125 of the capacity); the
+        // capacity is up to REGION_HEADROOM times the mean region (size_regions)
+        double mean = (double)cap / ncell, nbrick = 1.0;
+        for (int d = 0; d < 3; ++d) {
+            mean *= l.brick[d] + 2.0;
+            nbrick *= (l.nc[d] + l.brick[d] - 1) / l.brick[d];
         }
-        double halo = 1.0;
-        for (int d = 0; d < 3; ++d) halo *= (br[d] + 2.0) / br[d];
-        b += (size_t)(10.0 * 1.125 * 1.6 * halo * (double)cap) + 4096;
+        b += (size_t)(10.0 * 1.125 * REGION_HEADROOM * mean * nbrick) + 4096;
     }
-    if (p->potential_flag == 1) b += FM_MAX_FUNCY * cap * 4 + cap * 4 + 2 * 7 * cap * 4;
-    if (p->mie_potential == 1) b += 2 * cap * 4;
-    if (p->ensemble == FM_ENSEMBLE_TAG_MOVE) b += 2 * cap * 4 + 2 * 6 * cap * 8;
-    if (p->pressure_outflag == 1) b += 9 * cap * 8;
+    if (p->potential_flag == 1) {
+        buf(FM_MAX_FUNCY * cap * 4);
+        buf(cap * 4);
+        buf(8 * cap * 4, 2);
+    }
+    if (p->mie_potential == 1) buf(cap * 4, 2);
+    if (p->ensemble == FM_ENSEMBLE_TAG_MOVE) {
+        buf(cap * 4, 2);
+        buf(6 * cap * 8, 2);
+    }
+    if (p->pressure_outflag == 1) buf(9 * cap * 8);
     if (p->vflux_outflag >= 1 && p->vflux_outflag <= 3) b += 4 * (size_t)std::max(p->nplanes, 0) * 8;
-    if (p->sort_flag != 0) b += 4 * cap * 4 + 2 * (ncell + 1) * 4 + cap * 8 + 8192;  // keys, values, curve, counts, sort temporary
+    if (p->sort_flag != 0) {  // keys, values, curve, counts, sort temporary
+        buf(cap * 4, 4);
+        buf((ncell + 1) * 4, 2);
+        buf(cap * 8 + 8192);
+    }
     if (p->vflux_outflag == 4) {
         size_t nbo = 1;
         for (int d = 0; d < 3; ++d) {
-            const int nb = std::max((int)(p->binspercell[d] * nc[d]), 1);
-            nbo *= (size_t)(nb + 2 * (int)ceil((double)nb / nc[d]));
+            const int nb = std::max((int)(p->binspercell[d] * l.nc[d]), 1);
+            nbo *= (size_t)(nb + 2 * (int)ceil((double)nb / l.nc[d]));
         }
-        b += 9 * nbo * 8;
+        buf(9 * nbo * 8);
     }
     *bytes = (int64_t)b;
     return 0;
@@ -1094,11 +1107,15 @@ static int size_regions(fm_ctx* c, int measured) {
         return size_brick_tables(c);
     }
     // (registers hold the brick kernels to three workgroups per CU: small regions take a third of the
-    // LDS, up to half as much again as measured, and seldom meet a larger region)
+    // LDS, up to half as much again as measured or REGION_HEADROOM times the mean region, which the
+    // memory estimate counts on, and seldom meet a larger one)
     const size_t wgs = std::min<size_t>(std::max<size_t>(c->lds_cu / need, 1), 3);
     const size_t budget = std::min(c->lds_limit, (c->lds_cu / wgs) & ~(size_t)1023);
     // largest m in [m0, 65536] with region_bytes(m) <= budget
-    int lo = m0, hi = wgs < 3 ? 65536 : std::min(65536, m0 + m0 / 2);
+    double mean = (double)c->np / c->ncell;
+    for (int d = 0; d < 3; ++d) mean *= c->brick[d] + 2.0;
+    const int room = std::max((int)(REGION_HEADROOM * mean), m0 + m0 / 8);
+    int lo = m0, hi = wgs < 3 ? 65536 : std::min({65536, m0 + m0 / 2, room});
     while (lo < hi) {
         const int mid = lo + (hi - lo + 1) / 2;
         if (region_bytes(c, mid) <= budget) lo = mid;

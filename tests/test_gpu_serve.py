@@ -6,7 +6,7 @@ import pytest
 
 from flowmol_amd import config
 from flowmol_amd.md import MDContext
-from flowmol_amd.serve import Batch, ReplicaServer, couette_request, make_context
+from flowmol_amd.serve import Batch, ReplicaServer, couette_request, make_context, memory_footprint
 
 pytestmark = pytest.mark.gpu
 
@@ -278,3 +278,28 @@ def test_polymer_batch_members_match_alone():
     b.close()
     for g in ctx:
         g.close()
+
+
+@pytest.mark.parametrize("units,brick,density,rc", [
+    ((72, 72, 72), (1, 1, 1), 0.8, 2.5), ((50, 50, 50), (2, 1, 1), 0.8, 2.5), ((50, 50, 50), (0, 0, 0), 0.8, 2.5),
+    ((36, 36, 36), (2, 2, 2), 0.4, 2.5), ((40, 40, 40), (1, 1, 1), 0.8, 1.1225)])
+def test_footprint_covers_the_device_memory(units, brick, density, rc):
+    """What the admission counts is at least what a context takes, lists and staging tables included."""
+    import torch
+
+    p, r, v = config.config_fcc(units, density, rc, seed=5, tplot=10)
+    for d in range(3):
+        p.brick[d] = brick[d]
+    say(f"case: {r.shape[0]} molecules, brick {brick}, density {density}, cutoff {rc}")
+    warm = MDContext(*config.config_fcc((6, 6, 6), 0.8, 2.5, seed=1, tplot=10))   # (what the process keeps)
+    warm.setup(0)
+    free = torch.cuda.mem_get_info()[0]
+    g = MDContext(p, r, v)
+    g.setup(0)
+    g.run_vv(1, 40)
+    g.synchronize()
+    used = free - torch.cuda.mem_get_info()[0]
+    print(f"used {used / 2**20:.1f} MiB, estimated {memory_footprint(p, r.shape[0]) / 2**20:.1f} MiB", flush=True)
+    assert 0 < used <= memory_footprint(p, r.shape[0])
+    g.close()
+    warm.close()
