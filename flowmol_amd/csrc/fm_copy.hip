@@ -24,6 +24,7 @@
 #define NSLOTS 12
 #define POOL_SETS 4
 #define COPY_THREADS 6
+#define COPY_SEGS 4          // segments of a call
 #define COPY_MIN (4u << 20)  // below this the threads cost more than they save
 
 namespace {
@@ -89,6 +90,18 @@ int plain_copy(fm_ctx* c, const CopySeg* seg, int nseg, bool to_host) {
             else FM_HIP(hipMemcpyAsync(seg[k].dev, seg[k].host, seg[k].bytes, hipMemcpyHostToDevice, c->stream));
         }
     return 0;
+}
+
+// Memory that the runtime knows (pinned, managed or a device's): the device copies it by itself, at the
+// link's rate (72 MB, the state of 1,048,576 molecules: 1.40 ms; through the slots 2.04), and a thread
+// here may not be able to touch it.
+bool runtime_memory(const void* p) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type != hipMemoryTypeUnregistered;
 }
 
 // One transfer.  issued: chunks whose device copy is queued (their slot's event recorded); moved[i]:
@@ -186,9 +199,22 @@ void copy_pool_release() {
 // Copies the segments between the device and the host, in stream order.  Host data is in place (to the
 // device: no longer needed) when it returns, unless the transfer is small: then after the stream's
 // next synchronisation, which every caller does.
-int copy_segments(fm_ctx* c, const CopySeg* seg, int nseg, bool to_host) {
+int copy_segments(fm_ctx* c, const CopySeg* all, int n_all, bool to_host) {
     size_t total = 0;
-    for (int k = 0; k < nseg; ++k) total += seg[k].host ? seg[k].bytes : 0;
+    for (int k = 0; k < n_all; ++k) total += all[k].host ? all[k].bytes : 0;
+    if (total < COPY_MIN) return plain_copy(c, all, n_all, to_host);
+    CopySeg seg[COPY_SEGS];
+    int nseg = 0;
+    total = 0;
+    for (int k = 0; k < n_all; ++k) {
+        if (!all[k].host || !all[k].bytes) continue;
+        if (n_all > COPY_SEGS || runtime_memory(all[k].host)) {
+            if (int rc = plain_copy(c, all + k, 1, to_host)) return rc;
+        } else {
+            seg[nseg++] = all[k];
+            total += all[k].bytes;
+        }
+    }
     if (total < COPY_MIN) return plain_copy(c, seg, nseg, to_host);
     SlotSet* s = borrow(c->dev);
     if (!s) return plain_copy(c, seg, nseg, to_host);

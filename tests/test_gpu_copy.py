@@ -1,5 +1,6 @@
 """Host transfers of any size: states below and above the size that passes through the pinned slots, with
 remainders of a slot, from several threads at once, come back as they went."""
+import ctypes as C
 import sys
 import threading
 
@@ -7,6 +8,7 @@ import numpy as np
 import pytest
 
 from flowmol_amd import config
+from flowmol_amd._lib import check, load
 from flowmol_amd.md import MDContext
 
 pytestmark = pytest.mark.gpu
@@ -53,3 +55,32 @@ def test_round_trips_from_seven_threads():
     for t in th:
         t.join()
     assert not failed, failed
+
+
+def placed(x, where):
+    """A copy of x in the named kind of memory, with the object that keeps it and its address."""
+    import torch
+
+    t = torch.from_numpy(np.ascontiguousarray(x))
+    t = {"pinned": lambda: t.pin_memory(), "device": lambda: t.cuda(), "plain": lambda: t.clone()}[where]()
+    torch.cuda.synchronize()
+    return t, C.cast(t.data_ptr(), C.POINTER(C.c_double))
+
+
+@pytest.mark.parametrize("where", [("pinned",) * 3, ("device",) * 3, ("plain", "pinned", "device"),
+                                   ("pinned", "plain", "plain")])
+def test_arrays_that_the_runtime_knows(where):
+    """Pinned and device memory is copied by the device itself, whatever its size, beside plain arrays of
+    the same call."""
+    p, r, v = config.config_fcc((50, 50, 50), 0.8, 2.5, seed=8, tplot=10)   # 12 MB an array
+    rng = np.random.default_rng(8)
+    src = [rng.uniform(-1.0, 1.0, r.shape) for _ in range(3)]
+    say(f"case: 500000 molecules, arrays {where}")
+    g = MDContext(p, r, v)
+    given = [placed(x, w) for x, w in zip(src, where)]
+    got = [placed(np.zeros_like(x), w) for x, w in zip(src, where)]
+    check(load().fm_upload_state(g._h, r.shape[0], *[a for _, a in given]))
+    check(load().fm_download_state(g._h, *[a for _, a in got]))
+    for x, (t, _) in zip(src, got):
+        assert np.array_equal(t.cpu().numpy(), x)
+    g.close()
