@@ -5,9 +5,16 @@
 // through pinned slots: the calling thread queues the device copies in order, and a few threads move
 // each slot to or from the caller's memory as it is ready (the same 72 MB: 3.7 ms, of which the link takes most).
 //
-// The pinned slots belong to a pool of the process: a transfer borrows a set and gives it back before it
-// returns, at most POOL_SETS exist, and the pool is freed with the last context.  A transfer that finds
-// no set, or no thread, is done by the plain copy.
+// The pinned memory belongs to a pool of the process: a transfer borrows a set and gives it back before
+// it returns, at most POOL_SETS exist (of up to 24 MiB each, as much as a transfer has needed), and the
+// pool is freed with the last context.  A transfer that finds no set, or no thread, is done by the
+// plain copy.
+//
+// Slots of 4 MiB where there are enough of them for the threads: in the first 15 ms after a context is made
+// the device takes about 170 us for 2 MiB and 230 for 4, however the copies are queued (55 and 105 later
+// on), so the first reading of 1,048,576 molecules took 8.2 ms in slots of 2 MiB, by the plain copy 5.9 and
+// in slots of 4 MiB 5.8; later ones 2.07, 4.24 and 1.87 ms.  7.8 MB take 340 us in slots of 2 MiB, 370 in
+// slots of 4.
 #include "fm_internal.h"
 
 #include <string.h>
@@ -20,18 +27,24 @@
 #include <thread>
 #include <vector>
 
-#define SLOT_BYTES (2u << 20)
-#define NSLOTS 12
+#define UNIT_BYTES (2u << 20)  // a slot is one or two of these
+#define NUNITS 12
+#define TWO_UNITS (24u << 20)  // two from this size on
 #define POOL_SETS 4
 #define COPY_THREADS 6
 #define COPY_SEGS 4          // segments of a call
-#define COPY_MIN (4u << 20)  // below this the threads cost more than they save
+// Below these the threads cost more than they save.  Us by the plain copy and through the slots: to the
+// host 4.5 MB 290 and 240, 7.8 MB 480 and 340; to the device 4.5 MB 197 and 240, 7.8 MB 315 and 338, 12.3 MB
+// 475 and 470, 18.4 MB 670 and 605
+#define COPY_MIN_HOST (4u << 20)
+#define COPY_MIN_DEVICE (12u << 20)
 
 namespace {
 
 struct SlotSet {
-    char* p = nullptr;           // NSLOTS x SLOT_BYTES, pinned
-    hipEvent_t ev[NSLOTS] = {};  // the device copy of each slot
+    char* p = nullptr;           // n x UNIT_BYTES, pinned
+    hipEvent_t ev[NUNITS] = {};  // the device copy of each slot
+    int n = 0;
     int dev = -1;
     bool busy = false;
 };
@@ -47,12 +60,31 @@ void free_set(SlotSet* s) {
     delete s;
 }
 
-SlotSet* borrow(int dev) {
+// a set of fewer units than wanted gets that many, in one allocation (six take 1.5 ms longer to free); if
+// they cannot be had it keeps what it has
+void grow_set(SlotSet* s, int want) {
+    if (s->n >= want) return;
+    char* p = nullptr;
+    bool ok = hipHostMalloc((void**)&p, (size_t)want * UNIT_BYTES, hipHostMallocDefault) == hipSuccess;
+    for (int k = 0; ok && k < want; ++k)
+        ok = s->ev[k] || hipEventCreateWithFlags(&s->ev[k], hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+    } else {
+        std::swap(p, s->p);
+        s->n = want;
+    }
+    if (p) hipHostFree(p);
+}
+
+// a set with at least one unit, `want` of them if they can be had
+SlotSet* borrow(int dev, int want) {
     std::lock_guard<std::mutex> lock(g_mu);
     SlotSet** room = nullptr;
     for (SlotSet*& s : g_sets) {
         if (!s) room = &s;
         else if (!s->busy && s->dev == dev) {
+            grow_set(s, want);
             s->busy = true;
             return s;
         }
@@ -61,10 +93,8 @@ SlotSet* borrow(int dev) {
     SlotSet* s = new (std::nothrow) SlotSet();
     if (!s) return nullptr;
     s->dev = dev;
-    bool ok = hipHostMalloc((void**)&s->p, (size_t)NSLOTS * SLOT_BYTES, hipHostMallocDefault) == hipSuccess;
-    for (int k = 0; ok && k < NSLOTS; ++k) ok = hipEventCreateWithFlags(&s->ev[k], hipEventDisableTiming) == hipSuccess;
-    if (!ok) {
-        (void)hipGetLastError();
+    grow_set(s, want);
+    if (s->n == 0) {
         free_set(s);
         return nullptr;
     }
@@ -111,6 +141,7 @@ struct Transfer {
     SlotSet* s;
     std::vector<Chunk> ch;
     bool to_host;
+    size_t slot_bytes, ring;     // and slots in use
     std::atomic<size_t> next{0}, issued{0};
     std::vector<std::atomic<char>> moved;
     std::atomic<int> failed{0};
@@ -147,14 +178,14 @@ struct Transfer {
         for (;;) {
             const size_t i = next.fetch_add(1);
             if (i >= ch.size()) return;
-            const size_t slot = i % NSLOTS;
-            char* pin = s->p + slot * SLOT_BYTES;
+            const size_t slot = i % ring;
+            char* pin = s->p + slot * slot_bytes;
             if (to_host) {
                 if (!until_issued(i + 1) || !device_done(slot)) return;
                 memcpy(ch[i].host, pin, ch[i].n);
             } else {
-                // (the slot's copy of NSLOTS chunks ago has left it)
-                if (i >= NSLOTS && (!until_issued(i - NSLOTS + 1) || !device_done(slot))) return;
+                // (the slot's copy of `ring` chunks ago has left it)
+                if (i >= ring && (!until_issued(i - ring + 1) || !device_done(slot))) return;
                 memcpy(pin, ch[i].host, ch[i].n);
             }
             moved[i].store(1, std::memory_order_release);
@@ -164,9 +195,9 @@ struct Transfer {
     // the calling thread: the device side in order
     bool issue() {
         for (size_t i = 0; i < ch.size(); ++i) {
-            const size_t slot = i % NSLOTS;
-            char* pin = s->p + slot * SLOT_BYTES;
-            if (to_host ? (i >= NSLOTS && !until_moved(i - NSLOTS)) : !until_moved(i)) return false;
+            const size_t slot = i % ring;
+            char* pin = s->p + slot * slot_bytes;
+            if (to_host ? (i >= ring && !until_moved(i - ring)) : !until_moved(i)) return false;
             const hipError_t e = to_host
                                      ? hipMemcpyAsync(pin, ch[i].dev, ch[i].n, hipMemcpyDeviceToHost, c->stream)
                                      : hipMemcpyAsync(ch[i].dev, pin, ch[i].n, hipMemcpyHostToDevice, c->stream);
@@ -202,7 +233,8 @@ void copy_pool_release() {
 int copy_segments(fm_ctx* c, const CopySeg* all, int n_all, bool to_host) {
     size_t total = 0;
     for (int k = 0; k < n_all; ++k) total += all[k].host ? all[k].bytes : 0;
-    if (total < COPY_MIN) return plain_copy(c, all, n_all, to_host);
+    const size_t least = to_host ? COPY_MIN_HOST : COPY_MIN_DEVICE;
+    if (total < least) return plain_copy(c, all, n_all, to_host);
     CopySeg seg[COPY_SEGS];
     int nseg = 0;
     total = 0;
@@ -215,18 +247,19 @@ int copy_segments(fm_ctx* c, const CopySeg* all, int n_all, bool to_host) {
             total += all[k].bytes;
         }
     }
-    if (total < COPY_MIN) return plain_copy(c, seg, nseg, to_host);
-    SlotSet* s = borrow(c->dev);
+    if (total < least) return plain_copy(c, seg, nseg, to_host);
+    SlotSet* s = borrow(c->dev, (int)std::min<size_t>(NUNITS, total / UNIT_BYTES + 2));
     if (!s) return plain_copy(c, seg, nseg, to_host);
+    const size_t slot_bytes = total >= TWO_UNITS && s->n >= 2 ? 2 * UNIT_BYTES : UNIT_BYTES;
     int rc = 0;
     std::vector<std::thread> th;
     try {
         std::vector<Chunk> ch;
         for (int k = 0; k < nseg; ++k)
             for (size_t o = 0; seg[k].host && o < seg[k].bytes;) {
-                // (chunks end where the host's 2 MB pages do: no two threads take the fault of one page)
+                // (chunks end where the host's 2 MiB pages do: no two threads take the fault of one page)
                 char* h = (char*)seg[k].host + o;
-                const size_t n = std::min<size_t>(SLOT_BYTES - ((uintptr_t)h & (SLOT_BYTES - 1)), seg[k].bytes - o);
+                const size_t n = std::min<size_t>(slot_bytes - ((uintptr_t)h & (slot_bytes - 1)), seg[k].bytes - o);
                 ch.push_back({h, (char*)seg[k].dev + o, n});
                 o += n;
             }
@@ -235,6 +268,8 @@ int copy_segments(fm_ctx* c, const CopySeg* all, int n_all, bool to_host) {
         t.s = s;
         t.ch.swap(ch);
         t.to_host = to_host;
+        t.slot_bytes = slot_bytes;
+        t.ring = (size_t)s->n * UNIT_BYTES / slot_bytes;
         const size_t want = std::min<size_t>(COPY_THREADS, t.ch.size() / 2);
         th.reserve(want);
         try {

@@ -84,3 +84,12 @@ def test_arrays_that_the_runtime_knows(where):
     for x, (t, _) in zip(src, got):
         assert np.array_equal(t.cpu().numpy(), x)
     g.close()
+
+
+# 8 MB an array is where slots of one unit (2 MiB) become slots of two; 4 MB an array where uploads stage
+@pytest.mark.parametrize("n", [174762, 174763, 349525, 349526, 1100001])
+def test_round_trip_at_the_slot_sizes(n):
+    say(f"case: {n} molecules up and down, twice")
+    failed = []
+    round_trip(n, n, 2, failed)
+    assert not failed, failed
