@@ -138,3 +138,28 @@ def test_bond_length_beyond_the_cells(brick):
     canon = lambda b, s: sorted((i, int(x), int(y)) for i in range(b.shape[0]) for x, y in zip(b[i], s[i]) if x >= 0)
     assert canon(*o.bonds()) == canon(*g.bonds())
     g.close()
+
+
+# The list build by matrix tiles (FP64, small bricks): runs whose windows are empty, end within an octet, and
+# take more than four blocks of 32 candidates, lists longer than the capacity first allocated.
+@pytest.mark.parametrize("side", [2.8, 2.9])     # of a cell: the list radius itself, and more
+@pytest.mark.parametrize("n,rows,brick", [(15, 1, (1, 1, 1)), (17, 1, (3, 1, 1)), (130, 1, (1, 1, 1)), (600, 1, (1, 1, 1)),
+                                          (1200, 1, (1, 1, 1)), (1000, 2, (2, 1, 1)), (1600, 3, (1, 2, 1))])
+def test_tiles_with_long_and_short_runs(n, rows, brick, side):
+    rng = np.random.default_rng(n)
+    L = 5.0 * side
+    r = rng.uniform(0.0, L, (n, 3))
+    r[:, 1:] = side * (rng.integers(0, rows, (n, 2)) + rng.uniform(0.01, 0.99, (n, 2)))
+    r -= 0.5 * L
+    p = config.make_params((L, L, L), n / L ** 3, 2.5, tplot=10)
+    p.brick[0], p.brick[1], p.brick[2] = brick
+    say(f"case: {n} molecules in {rows}^2 rows of cells of {side}, brick {brick}")
+    o, g = Oracle(p, r, np.zeros_like(r)), MDContext(p, r, np.zeros_like(r))
+    for x in (o, g):
+        x.assign_to_cell()
+    o.updateborders(1)
+    o.assign_to_neighbourlist()
+    g.messenger_updateborders(1)
+    g.assign_to_neighbourlist()
+    assert np.array_equal(canonical_pairs(*o.neighbourlist()), canonical_pairs(*g.neighbourlist()))
+    g.close()
