@@ -2386,13 +2386,28 @@ struct MopI {             // the i-molecule's side of the MOP test
 // place) go through mop_entry_fast.
 // What bounds it: instruction issue (four fifths of the time).  With three slots on both sides of the
 // molecule, the sign factors subtracted per slot and the owner found by molecule numbers a launch over
-// 1,048,576 molecules with 64 planes took 260 us; 233 us with two above.
+// 1,048,576 molecules with 64 planes took 260 us; 233 us with two above.  Finer planes tally each entry as
+// it is met: 361 us with 100 planes, 413 with 128, 847 with 256 (365, 420 and 853 with the entries marked
+// first and tallied after their word).
 template <int NS, int NQ>
 __device__ __forceinline__ void lj_word_mop(const FbArgs& a, const P4K& p, int left, double xi, double yi,
                                             double zi, MopI& m, double& fx, double& fy, double& fz,
                                             double& pe, double& vt) {
     double tq[NQ];
     int slow = 0;  // bit q: entry q goes through mop_entry_fast
+    auto tally = [&](int q) {
+        // the whole numbers strictly between t_i and t_j, widened (see mop_entry_fast)
+        const double tj = (p.y[q] + m.hps) * m.inv_sp;
+        const int k0 = (int)ceil(fmin(m.ti, tj) - 1e-9), k1 = (int)floor(fmax(m.ti, tj) + 1e-9);
+        if (k0 <= k1 && k1 >= 0 && k0 < m.nplanes) {
+            // the pair law's magnitude 48 (x^7 - x^4/2) as the force sum takes it (within 1e-15)
+            const double acc = 24.0 * tq[q];
+            const double ri[3] = {xi, yi, zi}, rj[3] = {p.x[q], p.y[q], p.z[q]};
+            const double rij[3] = {xi - p.x[q], yi - p.y[q], zi - p.z[q]};
+            mop_entry_fast(a, ri, rj, rij, acc, m.spxy, m.planes, k0, k1,
+                           m.in_i && fabs(p.x[q]) < m.bx && fabs(p.z[q]) < m.bz);
+        }
+    };
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const double rx = xi - p.x[q], ry = yi - p.y[q], rz = zi - p.z[q];
@@ -2413,7 +2428,7 @@ __device__ __forceinline__ void lj_word_mop(const FbArgs& a, const P4K& p, int l
         tq[q] = t;
         // this end tallies it: an image, or molecule i the lower of the two
         const bool up = yi < p.y[q];
-        bool own = in & ((p.k[q] != 0) | up);
+        const bool own = in & ((p.k[q] != 0) | up);
         if constexpr (NS > 0) {
             const bool ins = m.in_i & (fabs(p.x[q]) < m.bx) & (fabs(p.z[q]) < m.bz);
 #pragma unroll
@@ -2423,32 +2438,19 @@ __device__ __forceinline__ void lj_word_mop(const FbArgs& a, const P4K& p, int l
                 m.c[s][1] = fmaf64(ts, ry, m.c[s][1]);
                 m.c[s][2] = fmaf64(ts, rz, m.c[s][2]);
             }
-            own = own & !(ins & up);
-        }
-        slow |= (int)own << q;
+            slow |= (int)(own & !(ins & up)) << q;
+        } else if (own) tally(q);
     }
-    if (slow != 0) {
+    if (NS > 0 && slow != 0) {
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            if (!((slow >> q) & 1)) continue;
-            // the whole numbers strictly between t_i and t_j, widened (see mop_entry_fast)
-            const double tj = (p.y[q] + m.hps) * m.inv_sp;
-            const int k0 = (int)ceil(fmin(m.ti, tj) - 1e-9), k1 = (int)floor(fmax(m.ti, tj) + 1e-9);
-            if (k0 <= k1 && k1 >= 0 && k0 < m.nplanes) {
-                // the pair law's magnitude 48 (x^7 - x^4/2) as the force sum takes it (within 1e-15)
-                const double acc = 24.0 * tq[q];
-                const double ri[3] = {xi, yi, zi}, rj[3] = {p.x[q], p.y[q], p.z[q]};
-                const double rij[3] = {xi - p.x[q], yi - p.y[q], zi - p.z[q]};
-                mop_entry_fast(a, ri, rj, rij, acc, m.spxy, m.planes, k0, k1,
-                               m.in_i && fabs(p.x[q]) < m.bx && fabs(p.z[q]) < m.bz);
-            }
-        }
+        for (int q = 0; q < NQ; ++q)
+            if ((slow >> q) & 1) tally(q);
     }
 }
 
 // The list loop with the MOP test per entry: one word at a time, the next word's index in flight.
 // A word's entries go NQ at a time: two (233 us at 1,048,576 molecules; one at a time 239, and four
-// spill 18 registers), or one where bonds and tethers hold registers too.
+// spill 18 registers), four without plane slots, or one where bonds and tethers hold registers too.
 template <int NS, int NQ>
 __device__ __forceinline__ void lj_plain_mop(const FbArgs& a, const double* pos, const int* key,
                                              const ListRow& row, int n, double xi, double yi,
@@ -2538,7 +2540,7 @@ __device__ __forceinline__ void forces_body_mop(const FbArgs& a, int brick, char
             }
         }
         double fx, fy, fz, pe, vir;
-        lj_plain_mop<NS, EXTRA ? 1 : 2>(a, r.pos, r.lslot, ListRow(a, i, tm), a.nbn[i], xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
+        lj_plain_mop<NS, EXTRA ? 1 : (NS > 0 ? 2 : 4)>(a, r.pos, r.lslot, ListRow(a, i, tm), a.nbn[i], xi, yi, zi, m, tm, fx, fy, fz, pe, vir);
         if constexpr (NS > 0) {
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
