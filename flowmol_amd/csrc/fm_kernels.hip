@@ -850,6 +850,35 @@ __global__ __launch_bounds__(FM_BLOCK) void k_bin_order(PermArgs a) {
     if (PER == 2 && c0 + 1 < a.ncell) order_cell(a, c0 + 1, lkey + w0, lext + w0);
 }
 
+// Cells of few molecules: a thread per molecule, which reads the keys of its cell's others itself (any cell
+// size).  A wavefront of k_bin_order would hold two of these cells and move their molecules with a few of
+// its lanes.  A binning, us by k_bin_order and by this: 1,048,576 molecules at 0.22 a cell 728 and 110, 1.1
+// 272 and 90, 4.4 115 and 79, 7.5 89 and 76, 10.1 81 and 77, 13 73 and 81, 17.7 68 and 83; 4,000,000 WCA (2.3)
+// 635 and 262; but 108,000 at 10 a cell 25 and 32, 32,000 WCA 26 and 28, 2,048 (2.8) 21 and 23.5, where a
+// launch has few wavefronts either way.  So up to eleven a cell from SPARSE_CELLS cells on (108,000 at 6.1 a
+// cell, 17,576 cells: 27.5 and 27.9).
+#define SPARSE_OCC 11
+#define SPARSE_CELLS 16384
+__global__ __launch_bounds__(FM_BLOCK) void k_bin_order_sparse(PermArgs a, const int* cell_of, int np) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= np) return;
+    Moved m;
+    load_molecule(a, k, m);
+    const int c = cell_of[m.o], b = a.start[c], n = a.start[c + 1] - b;
+    if (k == b) {
+        a.count[c] = 0;  // (an empty cell's is zero)
+        if (n > a.maxcell) set_err(a.flags, FM_EOVERFLOW, c);
+    }
+    const long long key = xkey(m.f[0]);
+    int rank = 0;
+    for (int q = 0; q < n; ++q) {
+        const int u = a.perm[b + q];
+        const long long o = xkey(a.src[u]);
+        if (o < key || (o == key && u != m.o && a.ext_src[u] < m.e)) ++rank;
+    }
+    store_molecule(a, m, b + rank, c);
+}
+
 // ---- macroscopic sums, src/simulation_record.f90:1205-1314 ------------------------------------
 // 7 sums per block: pe_lj, pe_poly, pe_lj+pe_poly, vir, mv2, vsum, msum ; + max(pe).  Each thread
 // sums MACRO_MPT molecules a grid apart (in that order), then the wavefront and the workgroup.
@@ -1410,7 +1439,9 @@ int launch_bin(fm_ctx* c, bool keep_acc, bool send, const int* reset, int nreset
     // below 32), one above that
     const int per = (size_t)c->np <= 24 * (size_t)c->ncell ? 2 : 1;
     const int nsort = nblocks((size_t)((c->ncell + per - 1) / per) * 64);
-    if (per == 2) k_bin_order<2><<<nsort, FM_BLOCK, 0, c->stream>>>(a);
+    if (c->ncell >= SPARSE_CELLS && (size_t)c->np <= SPARSE_OCC * (size_t)c->ncell)
+        k_bin_order_sparse<<<nblocks(c->np), FM_BLOCK, 0, c->stream>>>(a, cell_tmp, c->np);
+    else if (per == 2) k_bin_order<2><<<nsort, FM_BLOCK, 0, c->stream>>>(a);
     else k_bin_order<1><<<nsort, FM_BLOCK, 0, c->stream>>>(a);
     ktimer_end(c, KT_BIN);
     LAUNCH_CHECK();

@@ -102,3 +102,65 @@ def test_renumbering_of_any_leaver_count(count, corners):
         g.close()
     for ref, got in zip(*ends):
         assert np.array_equal(ref, got, equal_nan=True)
+
+
+def sparse(cells, seed):
+    """A box of cells^3 cells of side 2.8, nearly all empty: clumps of up to 130 molecules in cells here
+    and there, with many at equal x, and single molecules."""
+    rng = np.random.default_rng(seed)
+    r = []
+    for k in [1, 2, 3, 5, 31, 32, 33, 63, 64, 65, 130] * 12 + [1] * 2000:
+        q = rng.uniform(0.01, 2.79, (k, 3))
+        if k > 3:
+            q[:, 0] = np.linspace(0.1, 2.7, 6)[rng.integers(0, 6, k)]
+        r.append(2.8 * (rng.integers(0, cells, 3) - 0.5 * cells) + q)
+    r = np.concatenate(r)
+    return r[rng.permutation(r.shape[0])]
+
+
+@pytest.mark.parametrize("cells", [26, 66])      # the scan of the counts by itself, and from the chunks' sums
+def test_cells_of_few_molecules(cells):
+    r = sparse(cells, seed=cells)
+    L = 2.8 * cells + 1e-9
+    p = config.make_params((L, L, L), r.shape[0] / L ** 3, 2.5, tplot=10, ensemble=FM_ENSEMBLE_TAG_MOVE)
+    p.brick[0] = p.brick[1] = p.brick[2] = 3
+    say(f"case: {r.shape[0]} molecules in {cells}^3 cells")
+    rng = np.random.default_rng(1)
+    tag = rng.choice(np.array([0, FM_TAG_FIXED_SLIDE], np.int32), r.shape[0])
+    o, g = Oracle(p, r, np.zeros_like(r)), MDContext(p, r, np.zeros_like(r))
+    g.set_tags(tag, r + 1.0)
+    for x in (o, g):
+        x.assign_to_cell()
+    assert np.array_equal(g.cells(), o.cells())
+    for got, ref in zip(g.state()[:2] + (g.labels()[0], g.rtether()), (r, np.zeros_like(r), tag, r + 1.0)):
+        assert np.array_equal(got, ref)
+    o.updateborders(1)
+    o.assign_to_neighbourlist()
+    g.messenger_updateborders(1)
+    g.assign_to_neighbourlist()
+    assert np.array_equal(canonical_pairs(*o.neighbourlist()), canonical_pairs(*g.neighbourlist()))
+    for _ in range(2):                            # the counts are ready for the next binning
+        g.assign_to_cell()
+        assert np.array_equal(g.cells(), o.cells())
+    g.close()
+
+
+def test_gas_loop_equals_the_routines():
+    """A gas of two molecules a cell, rebuilt every third step: the fused loop's rebuilds (leavers wrapped and
+    counted in one launch) against the routines', bit for bit."""
+    say("case: 32000 molecules at density 0.1, 30 steps")
+    p, r, v = config.config_fcc((20, 20, 20), 0.08, 2.5, seed=4, tplot=3)
+    r = r + np.random.default_rng(2).uniform(-0.2, 0.2, r.shape)
+    L = np.array([p.domain[d] for d in range(3)])
+    r = np.where(r < -0.5 * L, r + L, np.where(r >= 0.5 * L, r - L, r))
+    a, b = MDContext(p, r, 3.0 * v), MDContext(p, r, 3.0 * v)
+    assert np.prod(a.geometry()["ncells"]) >= 16384
+    a.setup(0)
+    b.setup(0)
+    a.run_vv(1, 30)
+    for it in range(1, 31):
+        b.md_advance_vv(it)
+    for x, y in zip(a.state(), b.state()):
+        assert np.array_equal(x, y)
+    a.close()
+    b.close()
