@@ -1450,7 +1450,6 @@ struct FbArgs {
     const double* planes;
     int* flags;
     int cap, maxreg;
-    int maxw;              // words a molecule's list has room for
     int team;              // lanes that share a molecule's list (a power of two up to 16; team_of)
     int rec, ev;
     int kick;              // fused simulation_move_particles_vv(2): v += (0.5*dt)*a
@@ -1658,11 +1657,14 @@ __device__ __forceinline__ V team_sum(V v, int T) {
 // A lane's list words: word k is in row t + k T of the list (T lanes a molecule, t the lane's).  k is
 // the same for the whole wavefront, so a row's address is scalar arithmetic and the lane's part of it
 // one register, held from the start.  A lane past its own end reads the row as it is (the word is not
-// used); k is held within the rows that the list has (alloc_nlist allocates whole groups of T).
+// used); a row that no lane of the wavefront needs is not read, but one it holds already (alloc_nlist
+// allocates whole groups of T, and a word that a lane has lies in one).
 // With a 64-bit multiply, an addition and a minimum a load, the image shifts of staging worked out
 // for every molecule and the state read between the stores of the step's end a force launch took 481 us
-// at 4,194,304 LJ molecules, 43.0 at 131,072 beads, 22.1 at 108,000 LJ; now 460, 41.2, 21.2.  The
-// longest list of the wavefront as k's limit saves the rows past it and costs as much in shuffles.
+// at 4,194,304 LJ molecules, 43.0 at 131,072 beads, 22.1 at 108,000 LJ; now 460, 41.2, 21.2.
+// Where lists are short the rows past every list of a wavefront, two words ahead, are a tenth of the
+// launch's traffic: with them the launch that carries pass 1 took 71 us at 1,048,576 WCA molecules (ten
+// entries each) and 85 with rc 1.6, without 57 and 72.
 __device__ __forceinline__ size_t wave_uniform(size_t v) {
     return (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) |
            (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32;
@@ -1672,15 +1674,17 @@ struct ListRow {
     Global nbl;
     size_t step;    // bytes of T rows
     uint32_t off;   // of the lane's first word
-    int last;       // last group of T rows
     __device__ __forceinline__ ListRow(const FbArgs& a, int i, const Team& tm)
         : nbl((Global)wave_uniform((size_t)a.nbl)), step(wave_uniform((size_t)a.cap * tm.T * sizeof(uint64_t))),
-          off((uint32_t)((tm.t * a.cap + i) * sizeof(uint64_t))),
-          last(__builtin_amdgcn_readfirstlane((a.maxw + tm.T - 1) / tm.T - 1)) {}
+          off((uint32_t)((tm.t * a.cap + i) * sizeof(uint64_t))) {}
     __device__ __forceinline__ uint64_t operator[](int k) const {
-        Global p = nbl + (size_t)min(k, last) * step;
+        Global p = nbl + (size_t)k * step;
         asm("" : "+s"(p));  // (the row's address stays scalar)
         return *(const __attribute__((address_space(1))) uint64_t*)(p + off);
+    }
+    // word k when a lane needs it, else word `have` again
+    __device__ __forceinline__ uint64_t ahead(int k, bool need, int have) const {
+        return (*this)[__builtin_amdgcn_ballot_w64(need) != 0ull ? k : have];
     }
 };
 
@@ -1701,15 +1705,15 @@ __device__ __forceinline__ void lj_plain(const double* pos, const ListRow& row, 
     int left = n - 4 * tm.t;
     const uint64_t w0 = row[0];
     lj_stage(pa, pos, left > 0 ? w0 : 0);
-    uint64_t w1 = row[1];
-    uint64_t w2 = row[2];
+    uint64_t w1 = row.ahead(1, left > T4, 0);
+    uint64_t w2 = row.ahead(2, left > 2 * T4, 0);
     for (int k = 0; left > 0; k += 2, left -= 2 * T4) {
         lj_stage(pb, pos, left > T4 ? w1 : 0);
         // both words two ahead are loaded here, at the top of the pass: the wait the compiler
         // places at the loop head is then for loads a whole pass old
         const uint64_t wk2 = w2;
-        w1 = row[k + 3];
-        w2 = row[k + 4];
+        w1 = row.ahead(k + 3, left > 3 * T4, k);
+        w2 = row.ahead(k + 4, left > 4 * T4, k);
         __builtin_amdgcn_sched_barrier(0);  // keep the reads above the evaluation
         if constexpr (REC) lj_word_rec(pa, left, xi, yi, zi, rc2, potshift, sx, sy, sz, pe, vt);
         else lj_word(pa, left, xi, yi, zi, rc2, sx, sy, sz);
@@ -2183,13 +2187,13 @@ __device__ __forceinline__ void mie_plain(const double* pos, const uint8_t* lt, 
     int left = n - 4 * tm.t;
     const uint64_t w0 = row[0];
     mie_stage(pa, pos, lt, left > 0 ? w0 : 0);
-    uint64_t w1 = row[1];
-    uint64_t w2 = row[2];
+    uint64_t w1 = row.ahead(1, left > T4, 0);
+    uint64_t w2 = row.ahead(2, left > 2 * T4, 0);
     for (int k = 0; left > 0; k += 2, left -= 2 * T4) {
         mie_stage(pb, pos, lt, left > T4 ? w1 : 0);
         const uint64_t wk2 = w2;
-        w1 = row[k + 3];
-        w2 = row[k + 4];
+        w1 = row.ahead(k + 3, left > 3 * T4, k);
+        w2 = row.ahead(k + 4, left > 4 * T4, k);
         __builtin_amdgcn_sched_barrier(0);
         mie_word<NT, NB, REC>(pa, left, xi, yi, zi, m, sx, sy, sz, spe, svt);
         mie_stage(pa, pos, lt, left > 2 * T4 ? wk2 : 0);
@@ -2462,7 +2466,7 @@ __device__ __forceinline__ void lj_plain_mop(const FbArgs& a, const double* pos,
     uint64_t wn = row[0];
     for (int k = 0; left > 0; ++k, left -= 4 * T) {
         const uint64_t w = wn;
-        wn = row[k + 1];
+        wn = row.ahead(k + 1, left > 4 * T, k);
 #pragma unroll 1
         for (int q = 0; q < 4; q += NQ) {
             P4K p;
@@ -2751,15 +2755,15 @@ __device__ __forceinline__ void lj_plain32(const FbArgs& a, const Region& r, con
     const uint64_t w0 = row[0];
     uint64_t wa = n > 0 ? w0 : 0;
     lj_stage32(pa, p4, wa);
-    uint64_t w1 = row[1];
-    uint64_t w2 = row[2];
+    uint64_t w1 = row.ahead(1, n > 4, 0);
+    uint64_t w2 = row.ahead(2, n > 8, 0);
     for (int k = 0; 4 * k < n; k += 2) {
         const int kw = 4 * k;
         const uint64_t wb = kw + 4 < n ? w1 : 0;
         lj_stage32(pb, p4, wb);
         const uint64_t wk2 = w2;
-        w1 = row[k + 3];
-        w2 = row[k + 4];
+        w1 = row.ahead(k + 3, n - kw > 12, k);
+        w2 = row.ahead(k + 4, n - kw > 16, k);
         __builtin_amdgcn_sched_barrier(0);
         lj_word32<REC>(pa, kw, n - kw, xi, yi, zi, rc2f, band, sx, sy, sz, bl0, bl1, nb, a.potshift, &pe, &vt);
         wa = kw + 8 < n ? wk2 : 0;
@@ -3488,7 +3492,6 @@ int make_fargs(fm_ctx* c, int iter, bool kick, void* out, size_t* lds_out, int* 
     a.flags = c->d_flags;
     a.cap = c->cap;
     a.maxreg = c->maxreg;
-    a.maxw = c->maxnb / 4;
     a.team = c->team;
     const int tplot = c->p.tplot, teval = c->p.teval;
     a.step = iter;
