@@ -635,7 +635,7 @@ __global__ __launch_bounds__(FB_BLOCK) void k_nlist_brick(NlbArgs a) {
 // cover the rounding of the FP64 test itself, so the set is the FP64 set exactly.
 //
 // A molecule's candidates are an x window of each of its nine runs, as whole x bins: the first
-// molecule of each bin of the rows of region cells (sixteen bins a cell) stands in an LDS table, built
+// molecule of each bin of the rows of region cells (up to sixteen bins a cell) stands in an LDS table, built
 // once a brick, so a window costs one square root and two LDS reads.  The windows only leave out
 // molecules that cannot be pairs; the bins widen them by about a twentieth.
 // What bounds it: instruction issue (VALU busy nine tenths of the time).  Of a wavefront's 5,900
@@ -3395,10 +3395,14 @@ int launch_nlist(fm_ctx* c) {
         const int nbmax = g.B[0] * g.B[1] * g.B[2];
         const size_t lds0 = (size_t)c->maxreg * (sizeof(uint2) + sizeof(int)) +
                             (size_t)((c->maxreg + 1) / 2 + 4 * g.nreg + 1 + 2 * nbmax + 1) * sizeof(int);
-        // sixteen x bins a cell (one to three molecules of a run each), fewer where they would take
-        // a workgroup from the CU
+        // x bins a cell: up to sixteen, two a molecule (more than that are empty, and writing the table costs
+        // more than the windows save: 1,048,576 molecules, us a build with 16, 4 and 1: 0.22 a cell 501, 455
+        // and 422; 2.4 (WCA) 135, 126 and 131; 17.7 219, 228 and 275), and fewer where they would take a
+        // workgroup from the CU
         size_t lds = 0;
-        for (q.lb = 4; q.lb >= 0; --q.lb) {
+        q.lb = 0;
+        while (q.lb < 4 && (size_t)(1 << q.lb) * c->ncell <= (size_t)c->np) ++q.lb;
+        for (; q.lb >= 0; --q.lb) {
             lds = lds0 + ((((size_t)g.nreg << q.lb) + 1) * sizeof(uint16_t) + 7) / 8 * 8;
             if (lds <= c->lds_limit && (q.lb == 0 || std::min(c->lds_cu / lds, (size_t)3) == std::min(c->lds_cu / lds0, (size_t)3)))
                 break;
