@@ -34,10 +34,11 @@
 #define COPY_THREADS 6
 #define COPY_SEGS 4          // segments of a call
 // Below these the threads cost more than they save.  Us by the plain copy and through the slots: to the
-// host 4.5 MB 290 and 240, 7.8 MB 480 and 340; to the device 4.5 MB 197 and 240, 7.8 MB 315 and 338, 12.3 MB
-// 475 and 470, 18.4 MB 670 and 605
+// host 4.5 MB 290 and 240, 7.8 MB 480 and 340; to the device 4.5 MB 197 and 240, 12.3 MB 475 and 470, 24 MB
+// from the arrays of the transfer before 715 and 770, 30 MB 920 and 870, 37 MB 1,400 and 1,020 (from new
+// arrays the slots gain from 13 MB on)
 #define COPY_MIN_HOST (4u << 20)
-#define COPY_MIN_DEVICE (12u << 20)
+#define COPY_MIN_DEVICE (24u << 20)
 
 namespace {
 

@@ -86,7 +86,8 @@ def test_arrays_that_the_runtime_knows(where):
     g.close()
 
 
-# 8 MB an array is where slots of one unit (2 MiB) become slots of two; 4 MB an array where uploads stage
+# 8 MiB an array (349,525 molecules) is where slots of one unit (2 MiB) become slots of two and where uploads
+# begin to pass through them
 @pytest.mark.parametrize("n", [174762, 174763, 349525, 349526, 1100001])
 def test_round_trip_at_the_slot_sizes(n):
     say(f"case: {n} molecules up and down, twice")
