@@ -7,8 +7,8 @@
 //
 // The pinned memory belongs to a pool of the process: a transfer borrows a set and gives it back before
 // it returns, at most POOL_SETS exist (of up to 24 MiB each, as much as a transfer has needed), and the
-// pool is freed with the last context.  A transfer that finds no set, or no thread, is done by the
-// plain copy.
+// pool is freed with the last context.  Downloads make and grow the sets, uploads use what is there.  A
+// transfer that finds no set, or no thread, is done by the plain copy.
 //
 // Slots of 4 MiB where there are enough of them for the threads: in the first 15 ms after a context is made
 // the device takes about 170 us for 2 MiB and 230 for 4, however the copies are queued (55 and 105 later
@@ -78,19 +78,20 @@ void grow_set(SlotSet* s, int want) {
     if (p) hipHostFree(p);
 }
 
-// a set with at least one unit, `want` of them if they can be had
-SlotSet* borrow(int dev, int want) {
+// a set with at least one unit, `want` of them if they can be had; without `grow` a set of that many or none
+// (the pinned memory costs 2 ms, more than an upload of a context's only state gains by it)
+SlotSet* borrow(int dev, int want, bool grow) {
     std::lock_guard<std::mutex> lock(g_mu);
     SlotSet** room = nullptr;
     for (SlotSet*& s : g_sets) {
         if (!s) room = &s;
-        else if (!s->busy && s->dev == dev) {
+        else if (!s->busy && s->dev == dev && (grow || s->n >= want)) {
             grow_set(s, want);
             s->busy = true;
             return s;
         }
     }
-    if (!room) return nullptr;
+    if (!room || !grow) return nullptr;
     SlotSet* s = new (std::nothrow) SlotSet();
     if (!s) return nullptr;
     s->dev = dev;
@@ -249,7 +250,7 @@ int copy_segments(fm_ctx* c, const CopySeg* all, int n_all, bool to_host) {
         }
     }
     if (total < least) return plain_copy(c, seg, nseg, to_host);
-    SlotSet* s = borrow(c->dev, (int)std::min<size_t>(NUNITS, total / UNIT_BYTES + 2));
+    SlotSet* s = borrow(c->dev, (int)std::min<size_t>(NUNITS, total / UNIT_BYTES + 2), to_host);
     if (!s) return plain_copy(c, seg, nseg, to_host);
     const size_t slot_bytes = total >= TWO_UNITS && s->n >= 2 ? 2 * UNIT_BYTES : UNIT_BYTES;
     int rc = 0;
