@@ -222,34 +222,51 @@ static int set_brick(fm_ctx* c, const int b[3]) {
 // at once on each of the device's CUs where the staged regions leave room for two (512 on the 256 CUs
 // of a whole MI355X, 64 on a partition of 32).  So a large domain takes the
 // shape with the least halo per cell (1,048,576 molecules: 3x3x3 cells, 2197 bricks), and one whose
-// bricks would leave workgroup slots empty takes smaller ones, as many as the slots.  Measured, a step
-// of 108,000 molecules (rc 2.5): 3x3x3 (216 bricks) 48.5 us, 3x2x2 (486) 37.1, 2x2x2 (729) 45.5; of
-// 55,296 with rc 4: 2x3x1 78.6 us, 1x1x1 (729, two on a CU) 67.5, 2x1x1 (405, one on a CU) 83; of 5,148:
-// 3x3x2 27.3 us, 1x2x1 (120) 18.5 and with teams of lanes 14.6, 1x1x1 (210) 14.3: single cells of few
-// molecules are left out (each molecule would be staged 27 times over for nothing).
+// bricks would leave workgroup slots empty takes smaller ones, as many as the slots.  Measured, us a step
+// with its rebuilds (the rule's choice first): 108,000 molecules, rc 2.5: 3x2x2 (486 bricks) 30.9, 2x2x2
+// (729) 36.5, 3x3x2 (324) 36.7, 2x3x4 (least halo) 40.3; rc 4, 55,296: 3x1x1 (243, one on a CU) 44.7, 1x1x1
+// (729, two on a CU) 54.5, 2x1x1 (405, one on a CU) 63.7, 3x2x1 62.7; 256,000: 3x2x1 172.6, 3x1x1 175.6, 1x1x1
+// 225.  Single cells of few molecules are left out (each molecule would be staged 27 times over for
+// nothing).
+//
+// The work of all workgroups together, which is what a batch of domains in one launch costs, stays within
+// 1.4 times the least, or BRICK_WORK staged molecules above it.  Without that the smallest bricks won where
+// they gain a lone domain little: us a step without it and with it, of one domain and of 32 in a batch:
+// 2,048 WCA molecules 12.2 and 11.8, 243 and 171; 6,912 WCA 13.1 and 12.9, 294 and 201; 6,912 LJ 13.9 and
+// 15.3, 250 and 217; 16,384 LJ 16.2 and 20.1, 359 and 255; 32,000 LJ 19.8 and 20.3, 460 and 337; 32,000 at
+// density 0.2 20.3 and 21.7, 512 and 390.  (With least-halo bricks, one lane a molecule and no tiles they took
+// 18.2 and 189, 20.0 and 213, 27.4 and 233, 29.0 and 270, 29.8 and 342, 28.8 and 390.)
+#define BRICK_WORK 80000.0
 static void choose_brick(const int nc[3], double occ, int cus, int out[3]) {
     const double target = FB_BLOCK * 15.0 / 16.0;
-    double best = -1.0;
+    double least = 0.0, best = -1.0;
     out[0] = out[1] = out[2] = 1;
-    for (int bx = 1; bx <= std::min(nc[0], 12); ++bx)
-        for (int by = 1; by <= std::min(nc[1], 12); ++by)
-            for (int bz = 1; bz <= std::min(nc[2], 12); ++bz) {
-                const int P = bx * by * bz;
-                if (P > 1 && P * occ > target) continue;
-                if (P == 1 && occ < 48.0 && 2.0 * occ <= target) continue;
-                const double R = (bx + 2) * (by + 2) * (bz + 2) * occ;
-                const double nb = (double)((nc[0] + bx - 1) / bx) * ((nc[1] + by - 1) / by) * ((nc[2] + bz - 1) / bz);
-                // (27 B a staged molecule with its share of the tables; the largest region 15 % above the mean)
-                const double slots = (double)cus * (R * 1.15 * 27.0 <= 80.0 * 1024.0 ? 2 : 1);
-                const double cost = (nb <= slots ? 1.0 : nb / slots + 0.2) * (R + 300.0);
-                // (of equal ones the longest along x, the order of the slots)
-                if (best < 0.0 || cost <= best * (1.0 + 1e-12)) {
-                    best = cost;
-                    out[0] = bx;
-                    out[1] = by;
-                    out[2] = bz;
+    for (int pass = 0; pass < 2; ++pass)
+        for (int bx = 1; bx <= std::min(nc[0], 12); ++bx)
+            for (int by = 1; by <= std::min(nc[1], 12); ++by)
+                for (int bz = 1; bz <= std::min(nc[2], 12); ++bz) {
+                    const int P = bx * by * bz;
+                    if (P > 1 && P * occ > target) continue;
+                    const double R = (bx + 2) * (by + 2) * (bz + 2) * occ;
+                    const double nb = (double)((nc[0] + bx - 1) / bx) * ((nc[1] + by - 1) / by) * ((nc[2] + bz - 1) / bz);
+                    const double work = nb * (R + 300.0);
+                    if (pass == 0) {
+                        if (least == 0.0 || work < least) least = work;
+                        continue;
+                    }
+                    if (P == 1 && occ < 48.0 && 2.0 * occ <= target) continue;
+                    if (work > std::max(1.4 * least, least + BRICK_WORK)) continue;
+                    // (27 B a staged molecule with its share of the tables; the largest region 15 % above the mean)
+                    const double slots = (double)cus * (R * 1.15 * 27.0 <= 80.0 * 1024.0 ? 2 : 1);
+                    const double cost = (nb <= slots ? 1.0 : nb / slots + 0.2) * (R + 300.0);
+                    // (of equal ones the longest along x, the order of the slots)
+                    if (best < 0.0 || cost <= best * (1.0 + 1e-12)) {
+                        best = cost;
+                        out[0] = bx;
+                        out[1] = by;
+                        out[2] = bz;
+                    }
                 }
-            }
 }
 
 // The shape with the least halo per cell (mixed precision, whose FP32 sums depend on the shape: the
@@ -294,8 +311,8 @@ static int device_cus() {
 // Lanes per molecule of the force launches: two where a brick's molecules leave over a quarter of the
 // workgroup's threads idle, more while they take at most half of them and a lane keeps two words of the
 // expected list.  Measured at 5,148 molecules (1x1x1 bricks of 25, 73 entries): 1 lane 19.5 us a step,
-// 2 15.6, 4 14.9, 8 14.3, 16 15.4; at 55,296 with rc 4 (bricks of 76, 266 entries): 1 lane 89 us, 2 71.7,
-// 4 71.9, 16 80; 131,072 beads (bricks of 306): 1 lane 71.9 us, 2 68.5, 4 71.4.  One lane in mixed
+// 2 15.6, 4 14.9, 8 14.3, 16 15.4; at 55,296 with rc 4 (1x1x1 bricks of 76 given, 266 entries): 1 lane 89 us,
+// 2 71.7, 4 71.9, 16 80; 131,072 beads (bricks of 306): 1 lane 71.9 us, 2 68.5, 4 71.4.  One lane in mixed
 // precision (FP32 sums).  A lane's place in a group of T rows of the list is a 32-bit byte offset (ListRow):
 // T * capacity words are at most 2^32 bytes.
 static int team_of(const fm_params* p, const int brick[3], double occ, double entries, int cap) {
@@ -1348,7 +1365,10 @@ static int rebuild_lists_queued(fm_ctx* c, bool resets, bool keep_acc);
 // of the full list (the cell windows and the runs are those of the list radius), and an entry
 // beyond rc adds exactly zero to every force, PE and virial sum, so each sum is the full list's,
 // bit for bit.  Only for pairs that all end at rc: no bonds, no Mie tables; and one lane per molecule
-// (teams deal a list's words to their lanes, so leaving entries out changes the partial sums).
+// (teams deal a list's words to their lanes, so leaving entries out changes the partial sums).  Teams
+// give more than the shorter list where a brick leaves lanes idle: walls and slide, a rebuild every step, 1,536
+// molecules 97 us a step (one lane and the shorter list 179), 8,064 59 (80), 32,000 108 (130), 108,000 146
+// (144).
 static bool skinless_lists(const fm_ctx* c) { return c->p.potential_flag == 0 && c->p.mie_potential == 0 && c->team == 1; }
 
 static int rebuild_lists_for(fm_ctx* c, bool read_once, bool queued) {

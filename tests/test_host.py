@@ -113,3 +113,21 @@ def test_the_tuner_times_the_default_brick(units, density, rc, mixed):
         assert default in got and len(got) == k == len(set(got))
         if not mixed:
             assert got == brick_candidates(cells, nmol, k)
+
+
+@pytest.mark.parametrize("units,density,rc", [(8, 0.8, 1.1225), (12, 0.8, 1.1225), (20, 0.8, 1.1225), (12, 0.8, 2.5),
+                                              (16, 0.8, 2.5), (20, 0.8, 2.5), (30, 0.8, 2.5), (20, 0.2, 2.5), (13, 0.8, 4.0)])
+def test_default_bricks_do_not_multiply_the_work_of_a_batch(units, density, rc):
+    """Small bricks let a lone small domain use the whole device, but a batch in one launch costs what all
+    bricks stage together: that stays near the least of any shape (300: a workgroup's own cost in staged
+    molecules)."""
+    p, r, _ = config.config_fcc((units,) * 3, density, rc, seed=1, tplot=10)
+    nc = [int(p.domain[d] // (rc + 0.3)) for d in range(3)]
+    occ = max(1.0, r.shape[0] / np.prod(nc))
+
+    def work(b):
+        return np.prod([-(-n // x) for n, x in zip(nc, b)]) * (np.prod([x + 2 for x in b]) * occ + 300.0)
+
+    least = min(work(b) for b in itertools.product(*[range(1, min(n, 12) + 1) for n in nc])
+                if np.prod(b) == 1 or np.prod(b) * occ <= FB_BLOCK * 15 / 16)
+    assert work(layout(p, r.shape[0])[0]) <= max(1.4 * least, least + 80000.0) * (1 + 1e-12)
