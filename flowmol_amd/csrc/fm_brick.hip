@@ -643,7 +643,7 @@ __global__ __launch_bounds__(FB_BLOCK) void k_nlist_brick(NlbArgs a) {
 // 2,800 are the tests at 7 a candidate, 1,500 the entries at 11, 400 the windows.  Windows by two
 // binary searches and FP64 roots, tests by compare and select and store addresses by entry number took
 // 9,260.  Per build: 1,048,576 LJ molecules 266 -> 199 us, walls and slide (1,048,576)
-// 238 -> 183 us, cutoff 4 in bricks of one cell (55,296) 131 -> 98 us.
+// 238 -> 183 us, cutoff 4 in bricks of three cells and 228 molecules (55,296) 131 -> 98 us.
 typedef short s16x2 __attribute__((ext_vector_type(2)));
 
 struct NlqArgs {
@@ -3274,7 +3274,7 @@ int launch_region_max(fm_ctx* c) {
 }
 
 // Wavefronts per workgroup of the tile list build: the most with which two workgroups share a CU's
-// LDS, or else that fit one; 0 when four do not fit (the FP64 build then runs)
+// LDS, or else that fit one; 0 when four do not fit (the scan then runs)
 static int nlt_waves(const fm_ctx* c, const BG& g, bool poly, size_t* lds) {
     const size_t fixed = nlt_fixed_bytes(g, c->maxreg, poly), wave = nlt_wave_bytes(c->maxnb, poly);
     for (size_t room : {std::min(c->lds_cu / 2, c->lds_limit), c->lds_limit})
